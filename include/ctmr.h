@@ -78,7 +78,12 @@ enum ctmr_conv_flags {
 };
 
 enum ctmr_dtype {
-  CTMR_F32 = 0,   /* fp32 operands, FP32 MFMA (v_mfma_f32_16x16x4_f32) */
+  CTMR_F32 = 0,   /* fp32 operands, fp32 accumulate: the LDS-staged GEMM (CTMR_K_LDS) splits
+                     each operand into three bf16 parts that together hold its 24
+                     significant bits and sums the six part products at or above 2^-17 of
+                     the full one on bf16 MFMA (v_mfma_f32_32x32x16_bf16); results that
+                     are not finite are recomputed with plain fp32 products.  The other
+                     formulations run FP32 MFMA (v_mfma_f32_16x16x4_f32). */
   CTMR_BF16 = 1,  /* bf16 operands, fp32 accumulate (v_mfma_f32_16x16x32_bf16);
                      activations and outputs stay fp32 in memory */
   CTMR_F16X2 = 2  /* split fp16, the reference's "exact" mode for fp32 tensors
@@ -141,7 +146,7 @@ int ctmr_conv3d_split(const ctmr_conv_desc* desc);
 enum ctmr_conv_kernel {
   CTMR_K_STREAM = 0,        /* register-streaming GEMM over the packed copy */
   CTMR_K_STREAM_DIRECT = 1, /* register-streaming GEMM reading x itself */
-  CTMR_K_LDS = 2,           /* fp32 LDS-staged GEMM (halo bricks of x) */
+  CTMR_K_LDS = 2,           /* fp32 LDS-staged GEMM (halo bricks of x, three bf16 parts) */
   CTMR_K_LDS_BF16 = 3,      /* bf16 LDS-staged GEMM over the packed copy */
   CTMR_K_POINTWISE = 4,     /* persistent one-tap GEMM (1x1x1, im2col rows) */
   CTMR_K_SPLIT_WAVES = 5,   /* 64 x 64 tiles, each split range over the four waves */

@@ -9,6 +9,7 @@ from __future__ import annotations
 import os
 import shutil
 import subprocess
+from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
 PACKAGE_DIR = Path(__file__).resolve().parent
@@ -17,7 +18,7 @@ CSRC = PACKAGE_DIR / "csrc"
 INCLUDE = REPO_DIR / "include"
 LIB_NAME = "libctmr_hip.so"
 LIB_PATH = PACKAGE_DIR / LIB_NAME
-SOURCES = ("conv.hip", "norm.hip", "attention.hip", "noalloc.hip")
+SOURCES = ("conv.hip", "conv_lds.hip", "norm.hip", "attention.hip", "noalloc.hip")
 ARCH = "gfx950"
 
 # Packed FP32 VALU ops are disabled for every device pass; hipcc's host pass
@@ -55,13 +56,15 @@ def build(verbose: bool = False) -> Path:
     compiler = hipcc()
     build_dir = PACKAGE_DIR / "_build"
     build_dir.mkdir(exist_ok=True)
-    objects = []
-    for name in SOURCES:
+
+    def compile_source(name: str) -> str:
         obj = build_dir / (Path(name).stem + ".o")
-        cmd = [compiler, *HIP_FLAGS, *EXTRA_FLAGS.get(name, ()), f"-I{INCLUDE}", f"-I{CSRC}", "-c", str(CSRC / name),
-               "-o", str(obj)]
-        _run(cmd, verbose)
-        objects.append(str(obj))
+        _run([compiler, *HIP_FLAGS, *EXTRA_FLAGS.get(name, ()), f"-I{INCLUDE}", f"-I{CSRC}", "-c", str(CSRC / name),
+              "-o", str(obj)], verbose)
+        return str(obj)
+
+    with ThreadPoolExecutor(len(SOURCES)) as pool:  # one compiler process per source
+        objects = list(pool.map(compile_source, SOURCES))
     tmp = LIB_PATH.with_suffix(".so.tmp")
     _run([compiler, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objects, "-o", str(tmp)], verbose)
     os.replace(tmp, LIB_PATH)

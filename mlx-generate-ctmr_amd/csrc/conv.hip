@@ -1,5 +1,6 @@
 // Implicit-GEMM 3x3x3 / 1x1x1 convolution for MI355X (gfx950) on NDHWC fp32
-// activations, with FP32 MFMA (v_mfma_f32_16x16x4_f32) or bf16-in /
+// activations, with FP32 MFMA (v_mfma_f32_16x16x4_f32; the brick GEMM of
+// conv_lds.hip multiplies fp32 operands in bf16 parts) or bf16-in /
 // fp32-accumulate MFMA (v_mfma_f32_16x16x32_bf16).
 //
 // Dataflow (reference: src/mlx_generate_ctmr/_nax_conv.py:1-35, 475-684):
@@ -26,7 +27,7 @@
 // block, consumed by one 16x16x32 MFMA.  The packed weight stores each
 // (block, output channel) pair as 64 contiguous bytes in the same order, so A
 // and B lanes always pair the same input channel.
-#include "ctmr_common.hpp"
+#include "conv_gemm.hpp"
 
 #include <algorithm>
 #include <cstdarg>
@@ -42,8 +43,6 @@ void set_error(const char* fmt, ...) {
   vsnprintf(g_error, sizeof(g_error), fmt, ap);
   va_end(ap);
 }
-
-typedef unsigned int u4 __attribute__((ext_vector_type(4)));
 
 // ---------------------------------------------------------------------------
 // 1. Input packing
@@ -785,31 +784,6 @@ struct ConvArgs {
   int kb1;
 };
 
-// Final step of the group-norm partials of a stored tile: red[wave][c] holds
-// the fp64 (sum, sum of squares) of column c of each wave's 64 x (NSUB*16)
-// block over its rows (published by a barrier); each group's columns and
-// waves are added in ascending order -- a fixed order for a given shape.
-template <int NSUB, int WM, int WN>
-__device__ __forceinline__ void combine_gn_partials(const double (*red)[64][2], int col0, int cout, int cpg,
-                                                    int groups, double* __restrict__ stats_tile) {
-  constexpr int kWaveCols = NSUB * 16;
-  const int groups_here = (WN * kWaveCols) / cpg;
-  for (int gl = threadIdx.x; gl < groups_here; gl += 256) {
-    const int g = col0 / cpg + gl;
-    if (g >= groups || g * cpg >= cout) continue;
-    double a = 0.0, q = 0.0;
-    for (int wm = 0; wm < WM; ++wm)
-      for (int cc = 0; cc < cpg; ++cc) {
-        const int col = gl * cpg + cc;
-        const int wv = (col / kWaveCols) * WM + wm;
-        a += red[wv][col % kWaveCols][0];
-        q += red[wv][col % kWaveCols][1];
-      }
-    stats_tile[(int64_t)g * 2] = a;
-    stats_tile[(int64_t)g * 2 + 1] = q;
-  }
-}
-
 template <int DT>
 __device__ __forceinline__ void mfma_step(f4& acc, const u4& a, const u4& b);
 
@@ -860,29 +834,6 @@ __device__ __forceinline__ void mma_block(f4 (&acc)[4][NSUB], const u4 (&A)[4], 
           mfma_step<DT>(acc[ms][ns], A[ms], B[ns]);
       }
   }
-}
-
-// One DPP lane move of an fp64 value (two 32-bit halves; every source lane
-// lies inside the lane's row of 16).
-template <int CTRL>
-__device__ __forceinline__ double dpp_f64(double v) {
-  const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
-  const int lo = __builtin_amdgcn_mov_dpp((int)(unsigned)u, CTRL, 0xF, 0xF, false);
-  const int hi = __builtin_amdgcn_mov_dpp((int)(unsigned)(u >> 32), CTRL, 0xF, 0xF, false);
-  return __builtin_bit_cast(double, ((unsigned long long)(unsigned)hi << 32) | (unsigned)lo);
-}
-
-// Sum over the 16 lanes of a row, in the tree of an xor butterfly (partners
-// 1, 2, 4, 8): quad_perm [1,0,3,2] and [2,3,0,1] are xor 1 and xor 2; after
-// them lane 7 - i of a half row holds the value lane i ^ 4 holds (fp32/fp64
-// addition commutes), so the half-row mirror is the xor-4 step and the row
-// mirror the xor-8 step.  VALU moves instead of LDS permutes.
-__device__ __forceinline__ double row16_sum(double v) {
-  v += dpp_f64<0xB1>(v);   // quad_perm [1,0,3,2]
-  v += dpp_f64<0x4E>(v);   // quad_perm [2,3,0,1]
-  v += dpp_f64<0x141>(v);  // row_half_mirror
-  v += dpp_f64<0x140>(v);  // row_mirror
-  return v;
 }
 
 // Column sums over a wave's 64 rows of a transposed accumulator block set
@@ -946,26 +897,9 @@ __device__ __forceinline__ void load_bias(const ConvArgs& p, int b, int n0, int 
 // load would wait for the stores before it (the compiler cannot prove the
 // output and its inputs apart).  Rows past the grid are clamped for the loads
 // and masked for the stores.
-// Cache-policy operands of the GEMMs' output stores (gfx950 encoding: bit 1 =
-// NT, non-temporal; bit 4 = SC1, device scope).  Same values under every
-// policy; measured on MI355X, default / NT / SC1, A/B twice in one run: the
-// brick GEMMs (fp32 and bf16 LDS-staged) and the streaming GEMM take SC1
-// (config-0 fp32 + bf16 GEMMs 0.462 / 0.505 / 0.451 ms, UNet step 17.72 /
-// 17.80 / 17.69 ms, config-1 block 26.18 / 26.17 / 26.14 ms, config 2a and
-// the decoder window within 0.5 % either way); the persistent 1x1 GEMM takes
-// NT (config 2c 0.165 / 0.160 / 0.171 ms).
-constexpr int kStoreSC1 = 16;
-constexpr int kStoreNT = 2;
-
 // IDENT: GEMM row v of batch item b is output voxel b * s_out + v (every route
 // but the nearest-2x parity phases), so a wave's 64 rows are contiguous and
 // its stores go through one buffer descriptor with the SC1 cache policy.
-// No term after the bias (the epilogues' default `after_bias`).
-struct NoTerm {
-  template <typename Acc>
-  __device__ void operator()(Acc&) const {}
-};
-
 template <int NSUB, int WM, int WN, bool IDENT, typename OutVoxel, typename AfterBias = NoTerm>
 __device__ __forceinline__ void store_tile(const ConvArgs& p, f4 (&acc)[4][NSUB], const f4 (&bq)[NSUB], int b,
                                            int m0, int n0, int S, int split_id, int wave, int lane, int col0,
@@ -1321,28 +1255,8 @@ __global__ __launch_bounds__(256 * SETS, SETS == 1 ? 2 : 1) void conv_kernel(Con
 }
 
 // ---------------------------------------------------------------------------
-// 3b. LDS-staged implicit GEMM (large stride-1 fp32 volumes)
+// 3b. Brick GEMMs (the fp32 LDS-staged one is conv_lds_kernel, conv_lds.hip)
 // ---------------------------------------------------------------------------
-// A workgroup owns a 4x8x8 brick of output voxels (256 GEMM rows: wave m holds
-// depth m, MFMA row block ms holds brick rows ms and ms+4, lane%16 -> (row
-// half, column)) and 64 output channels.  For each 16-channel chunk it
-// stages the brick's 6x10x10 halo from the unpadded NDHWC input into LDS --
-// zero outside the volume, group-norm affine + SiLU applied on the way, so the
-// streaming path's separate pack pass disappears -- then runs all 27 taps with
-// A read from LDS at compile-time offsets and B (packed weight) fetched one tap
-// ahead through buffer loads.  The next chunk's halo is in flight in registers
-// while the current chunk multiplies.  A staged voxel row is 80 bytes (16
-// channels + 16 bytes of padding): the 16 rows a 16-lane group reads (8
-// columns of brick lines y and y+4, 40 voxels apart) then fall on 16 distinct
-// 16-byte bank groups of the 256-byte LDS line -- 5*x + 2*y (mod 16) takes
-// every value once over x < 8, y in {y0, y0+4}.
-constexpr int kBD = 4, kBH = 8, kBW = 8;
-constexpr int kHD = kBD + 2, kHH = kBH + 2, kHW = kBW + 2;
-constexpr int kHaloVox = kHD * kHH * kHW;                 // 600
-constexpr int kLdsRow = 80;
-constexpr int kStageIters = (kHaloVox * 4 + 255) / 256;  // 16-byte pieces per thread
-
-
 // Epilogue of the brick GEMMs (conv_lds_kernel, conv_lds_bf16_kernel) from
 // transposed accumulators: lane l of block (ms, ns) holds voxel (z0 + wave,
 // y0 + ms + 4*((l/8)%2), x0 + l%8) of the 4x8x8 brick and output columns
@@ -1416,275 +1330,6 @@ __device__ __forceinline__ void store_brick(const Args& p, f4 (&acc)[4][4], int 
     __syncthreads();
     combine_gn_partials<4, 4, 1>(red, n0, p.cout, p.gn_cpg, p.gn_groups,
                                  p.stats + ((int64_t)b * p.tz * p.ty * p.tx * S * S * S + tile_id) * p.gn_groups * 2);
-  }
-}
-
-struct LdsArgs {
-  const float* x;       // unpadded NDHWC input (channels [0, c1) of a two-source input)
-  const float* x2;      // channels [c1, cin) of a two-source input, or null
-  int c1;               // channels of x (cin for one source; a multiple of 16)
-  const float* affine;  // (n, cin, 2) or null
-  const char* wp;       // packed weight [tap][kblock][np][64 bytes]
-  const float* bias;
-  const float* res;
-  float* y;             // output, or split partial planes
-  int64_t x_bytes, w_bytes, plane;
-  int n, d, h, w, cin, cout, np, kb;
-  int tz, ty, tx;       // bricks per axis
-  int n_tiles, split;
-  int affine_on, silu_on, batch_bias, has_res, has_bias;
-  double* stats;        // group-norm partials of the output (ctmr_conv3d_gn) or null
-  int gn_groups, gn_cpg;
-};
-
-// TWO: the input is two tensors (ctmr_conv3d_cat); the one-tensor kernel keeps
-// precomputed byte offsets and a single descriptor.  XF: the staging
-// transform, bit 0 the GN affine and bit 1 SiLU (p.affine_on, p.silu_on), as
-// template flags so the transform is branch-free code.  WS = 2: a K split of
-// two ranges inside the workgroup -- wave set s (waves 4s .. 4s + 3, each set
-// with its own halo buffer) runs the chunks of range s of one brick, and set
-// 0 adds set 1's sums after the bias, the order of the split reduction
-// (bias, range 0, range 1, residual), with no partial planes in memory.
-template <bool TWO, int XF, int WS>
-__global__ __launch_bounds__(256 * WS, WS == 1 ? 2 : 1) void conv_lds_kernel(LdsArgs p) {
-  static_assert(WS == 1 || WS == 2, "one or two wave sets");
-  __shared__ __attribute__((aligned(16))) char lds_sets[WS * kHaloVox * kLdsRow];
-  const int set = WS == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 8));
-  char* const lds = lds_sets + set * (kHaloVox * kLdsRow);
-  const int tid = threadIdx.x & 255, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // XCD-aware order (as conv_kernel): neighbouring bricks share halo planes.
-  const int nb = gridDim.x, bid = blockIdx.x;
-  const int xcd = bid & 7, slot = bid >> 3, per = nb >> 3, rem = nb & 7;
-  const int tile = (xcd < rem) ? xcd * (per + 1) + slot : rem * (per + 1) + (xcd - rem) * per + slot;
-  const int n_tile = tile % p.n_tiles;
-  int rest = tile / p.n_tiles;
-  const int bx = rest % p.tx;
-  rest /= p.tx;
-  const int by = rest % p.ty;
-  rest /= p.ty;
-  const int bz = rest % p.tz;
-  rest /= p.tz;
-  const int b = rest % p.n;
-  const int split_id = rest / p.n;
-  const int z0 = bz * kBD, y0 = by * kBH, x0 = bx * kBW;
-  const int lrow = lane & 15, lgrp = lane >> 4;
-
-  // Staging: piece i of thread t is channels 4*(t&3)..+3 of the chunk at halo
-  // voxel (t>>2) + 64i.  Offsets are relative to the first staged plane, so
-  // they stay within 32 bits (the host checks 6 planes fit).  goff[i] is the
-  // piece's byte offset; with TWO it is the piece's voxel index instead: a
-  // chunk comes from x (chunks below c1 / 16) or from x2, whose rows hold the
-  // remaining channels, and the byte offset follows from the chunk's source.
-  const int part = tid & 3;
-  const int zb = max(z0 - 1, 0);
-  const int c2 = p.cin - p.c1;
-  const int kb1 = p.c1 >> 4;
-  const int64_t vbase = ((int64_t)b * p.d + zb) * p.h * p.w;     // first staged voxel
-  const int64_t vtotal = (int64_t)p.n * p.d * p.h * p.w;
-  const __amdgpu_buffer_rsrc_t xrsrc1 = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)(p.x + vbase * p.c1), (short)0, (int)min((vtotal - vbase) * p.c1 * 4, (int64_t)0x7fffffff),
-      0x00020000);
-  const __amdgpu_buffer_rsrc_t xrsrc2 = TWO ? __builtin_amdgcn_make_buffer_rsrc(
-      (void*)(p.x2 + vbase * c2), (short)0, (int)min((vtotal - vbase) * c2 * 4, (int64_t)0x7fffffff),
-      0x00020000) : xrsrc1;
-  int goff[kStageIters];
-  unsigned valid = 0;
-#pragma unroll
-  for (int i = 0; i < kStageIters; ++i) {
-    const int hv = (tid >> 2) + 64 * i;
-    goff[i] = 0;
-    if (hv < kHaloVox) {
-      const int hz = hv / (kHH * kHW), hr = hv - hz * (kHH * kHW);
-      const int hy = hr / kHW, hx = hr - hy * kHW;
-      const int gz = z0 - 1 + hz, gy = y0 - 1 + hy, gx = x0 - 1 + hx;
-      if (gz >= 0 && gz < p.d && gy >= 0 && gy < p.h && gx >= 0 && gx < p.w) {
-        valid |= 1u << i;
-        const int vox = ((gz - zb) * p.h + gy) * p.w + gx;
-        goff[i] = TWO ? vox : vox * p.cin * 4 + part * 16;
-      }
-    }
-  }
-  // Source of a chunk: descriptor, row bytes (TWO) and the chunk's byte offset in a row.
-  struct ChunkSrc {
-    __amdgpu_buffer_rsrc_t rs;
-    int row, so;
-  };
-  auto chunk_src = [&](int chunk) {
-    ChunkSrc c;
-    const bool second = TWO && chunk >= kb1;
-    c.rs = second ? xrsrc2 : xrsrc1;
-    c.row = (second ? c2 : p.c1) * 4;
-    c.so = __builtin_amdgcn_readfirstlane((second ? chunk - kb1 : chunk) * 64);
-    return c;
-  };
-  auto piece_off = [&](int i, const ChunkSrc& c) { return TWO ? goff[i] * c.row + part * 16 : goff[i]; };
-
-  // A: LDS byte address of this lane's voxel at tap (0,0,0) per row block.
-  int abase[4];
-#pragma unroll
-  for (int ms = 0; ms < 4; ++ms)
-    abase[ms] = ((wave * kHH + ms + 4 * (lrow >> 3)) * kHW + (lrow & 7)) * kLdsRow + lgrp * 16;
-  // B: one output column per lane per 16-column block.
-  const int n0 = n_tile * 64;
-  const __amdgpu_buffer_rsrc_t brsrc = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)p.wp, (short)0, (int)min(p.w_bytes, (int64_t)0x7fffffff), 0x00020000);
-  int boff[4];
-#pragma unroll
-  for (int ns = 0; ns < 4; ++ns) boff[ns] = min(n0 + ns * 16 + lrow, p.np - 1) * 64 + lgrp * 16;
-  const int bchunk = p.np * 64;
-
-  f4 acc[4][4];
-#pragma unroll
-  for (int ms = 0; ms < 4; ++ms)
-#pragma unroll
-    for (int ns = 0; ns < 4; ++ns) acc[ms][ns] = f4{0.f, 0.f, 0.f, 0.f};
-
-  const int kpart = split_id * WS + set, kparts = p.split * WS;
-  const int c_begin = __builtin_amdgcn_readfirstlane((int)((int64_t)kpart * p.kb / kparts));
-  const int c_end = __builtin_amdgcn_readfirstlane((int)((int64_t)(kpart + 1) * p.kb / kparts));
-
-  u4 stage[kStageIters];
-  auto fetch = [&](int chunk) {
-    const ChunkSrc c = chunk_src(chunk);
-#pragma unroll
-    for (int i = 0; i < kStageIters; ++i)
-      stage[i] = __builtin_amdgcn_raw_buffer_load_b128(c.rs, piece_off(i, c), c.so, 0);
-  };
-  // GN affine of this thread's four channels of a chunk: (scale, offset) pairs.
-  auto load_affine = [&](int chunk, f4& sc, f4& of) {
-    sc = f4{1.f, 1.f, 1.f, 1.f};
-    of = f4{0.f, 0.f, 0.f, 0.f};
-    if constexpr ((XF & 1) != 0) {
-      const f4* q = reinterpret_cast<const f4*>(p.affine + ((int64_t)b * p.cin + chunk * 16 + part * 4) * 2);
-      const f4 a0 = q[0], a1 = q[1];
-      sc = f4{a0[0], a0[2], a1[0], a1[2]};
-      of = f4{a0[1], a0[3], a1[1], a1[3]};
-    }
-  };
-  // Piece i as staged: GN affine, SiLU, zero outside the volume.
-  auto transform = [&](int i, const f4& sc, const f4& of) {
-    f4 v = __builtin_bit_cast(f4, stage[i]);
-    const bool in = (valid >> i) & 1u;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      float t = v[j];
-      if constexpr ((XF & 1) != 0) t = fmaf(t, sc[j], of[j]);
-      if constexpr ((XF & 2) != 0) t = silu_f(t);
-      v[j] = in ? t : 0.f;
-    }
-    stage[i] = __builtin_bit_cast(u4, v);
-  };
-  auto commit = [&]() {
-#pragma unroll
-    for (int i = 0; i < kStageIters; ++i) {
-      const int hv = (tid >> 2) + 64 * i;
-      if (hv >= kHaloVox) continue;
-      *reinterpret_cast<u4*>(lds + hv * kLdsRow + part * 16) = stage[i];
-    }
-  };
-  auto load_a = [&](f4 (&A)[4], int tap) {
-    const int off = (((tap / 9) * kHH + (tap / 3) % 3) * kHW + tap % 3) * kLdsRow;
-#pragma unroll
-    for (int ms = 0; ms < 4; ++ms) A[ms] = *reinterpret_cast<const f4*>(lds + abase[ms] + off);
-  };
-  auto load_b = [&](u4 (&B)[4], int tap, int chunk) {
-    const int so = __builtin_amdgcn_readfirstlane((tap * p.kb + chunk) * bchunk);
-#pragma unroll
-    for (int ns = 0; ns < 4; ++ns) B[ns] = __builtin_amdgcn_raw_buffer_load_b128(brsrc, boff[ns], so, 0);
-  };
-  auto mma = [&](const f4 (&A)[4], const u4 (&B)[4]) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int ms = 0; ms < 4; ++ms)
-#pragma unroll
-        for (int ns = 0; ns < 4; ++ns)
-          acc[ms][ns] = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(f4, B[ns])[j], A[ms][j],
-                                                             acc[ms][ns], 0, 0, 0);  // B^T A^T: see store_brick
-  };
-
-  // Without affine or SiLU the staging transform is the zero mask alone: it
-  // runs inside the previous chunk's tap loop, among the MFMAs, and the
-  // commit between the barriers only writes LDS (config 0: 409-412 -> 405-406
-  // us).  With affine + SiLU the same placement measured ~1 % slower than
-  // transforming at the commit, which those variants keep.
-  constexpr bool kInLoop = XF == 0;
-  fetch(c_begin);
-  if constexpr (kInLoop) {
-    f4 sc, of;
-    load_affine(c_begin, sc, of);
-#pragma unroll
-    for (int i = 0; i < kStageIters; ++i) transform(i, sc, of);
-  }
-  for (int chunk = c_begin; chunk < c_end; ++chunk) {
-    __syncthreads();  // every wave has finished reading the previous chunk
-    if constexpr (!kInLoop) {
-      f4 sc, of;
-      load_affine(chunk, sc, of);
-#pragma unroll
-      for (int i = 0; i < kStageIters; ++i) transform(i, sc, of);
-    }
-    commit();
-    __syncthreads();
-    f4 A[2][4];
-    u4 B[2][4];
-    load_b(B[0], 0, chunk);
-    load_a(A[0], 0);
-    // Unconditional (see conv_kernel): the last chunk re-reads itself.
-    const int next = min(chunk + 1, c_end - 1);
-    const ChunkSrc nx = chunk_src(next);
-    f4 nsc, nof;
-    load_affine(next, nsc, nof);
-#pragma unroll
-    for (int t = 0; t < 27; ++t) {
-      if (t + 1 < 27) {
-        load_b(B[(t + 1) & 1], t + 1, chunk);
-        load_a(A[(t + 1) & 1], t + 1);
-      }
-      // The next chunk's halo, one 16-byte piece every other tap: loads
-      // retire in order, so each piece has two taps of products to arrive
-      // before a later weight load has to wait for it.
-      if ((t & 1) && (t >> 1) < kStageIters)
-        stage[t >> 1] = __builtin_amdgcn_raw_buffer_load_b128(nx.rs, piece_off(t >> 1, nx), nx.so, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      // Raised priority while this wave's MFMAs issue, so a wave whose
-      // operands are ready wins issue slots over waves in their staging code.
-      __builtin_amdgcn_s_setprio(1);
-      mma(A[t & 1], B[t & 1]);
-      // Piece i, loaded at tap 2i + 1, is masked at tap 2i + 6.
-      if (kInLoop && t >= 6 && !(t & 1) && ((t - 6) >> 1) < kStageIters) {
-        transform((t - 6) >> 1, nsc, nof);
-      }
-      __builtin_amdgcn_s_setprio(0);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  }
-
-  __shared__ double red[4][64][2];
-  const int tile_id = (bz * p.ty + by) * p.tx + bx;
-  if constexpr (WS == 2) {
-    // Set 1 hands its sums to set 0 through the halo buffers (64 KiB of the
-    // 2 x 47 KiB) once every wave has finished reading them, then ends; the
-    // barriers after that wait only for set 0's waves.
-    f4* const xs = reinterpret_cast<f4*>(lds_sets);
-    __syncthreads();
-    if (set == 1) {
-#pragma unroll
-      for (int ms = 0; ms < 4; ++ms)
-#pragma unroll
-        for (int ns = 0; ns < 4; ++ns) xs[(wave * 16 + ms * 4 + ns) * 64 + lane] = acc[ms][ns];
-    }
-    __syncthreads();
-    if (set == 1) return;
-    store_brick(p, acc, b, split_id, z0, y0, x0, n0, wave, lane, tile_id, red, 0, [&](f4 (&a)[4][4]) {
-#pragma unroll
-      for (int ms = 0; ms < 4; ++ms)
-#pragma unroll
-        for (int ns = 0; ns < 4; ++ns) a[ms][ns] += xs[(wave * 16 + ms * 4 + ns) * 64 + lane];
-    });
-  } else {
-    store_brick(p, acc, b, split_id, z0, y0, x0, n0, wave, lane, tile_id, red);
   }
 }
 
@@ -3365,18 +3010,6 @@ static void launch_lds16(bool up, dim3 grid, hipStream_t st, const Lds16Args& a)
   else hipLaunchKernelGGL((conv_lds_bf16_kernel<DT, false, WS>), grid, dim3(256 * WS), 0, st, a);
 }
 
-// conv_lds_kernel for a staging transform xf (bit 0 affine, bit 1 SiLU).
-template <bool TWO, int WS>
-static void launch_lds(int xf, dim3 grid, hipStream_t st, const LdsArgs& a) {
-  const dim3 block(256 * WS);
-  switch (xf) {
-    case 0: hipLaunchKernelGGL((conv_lds_kernel<TWO, 0, WS>), grid, block, 0, st, a); break;
-    case 1: hipLaunchKernelGGL((conv_lds_kernel<TWO, 1, WS>), grid, block, 0, st, a); break;
-    case 2: hipLaunchKernelGGL((conv_lds_kernel<TWO, 2, WS>), grid, block, 0, st, a); break;
-    default: hipLaunchKernelGGL((conv_lds_kernel<TWO, 3, WS>), grid, block, 0, st, a); break;
-  }
-}
-
 // The 64-column register-streaming GEMM is tuned for two resident workgroups
 // per CU (two waves per SIMD; its split policy and round sizes assume 512 per
 // launch).  Its ~160 VGPRs would let a third in, which measured slower
@@ -3832,13 +3465,7 @@ static int conv3d_gemm_impl(const ctmr_conv_desc* desc, const float* x, const fl
     const int64_t blocks = (int64_t)g.m_tiles * g.n_tiles * desc->n * a.split;
     const dim3 grid((unsigned)blocks);
     const int xf = (a.affine_on ? 1 : 0) | (a.silu_on ? 2 : 0);
-    if (a.x2) {
-      if (g.wsets == 2) launch_lds<true, 2>(xf, grid, st, a);
-      else launch_lds<true, 1>(xf, grid, st, a);
-    } else {
-      if (g.wsets == 2) launch_lds<false, 2>(xf, grid, st, a);
-      else launch_lds<false, 1>(xf, grid, st, a);
-    }
+    launch_conv_lds(xf, g.wsets, grid, st, a);
     if ((rc = check_launch("conv_lds"))) return rc;
     if (partial) {
       launch_split_reduce(desc, g, part, a.plane, bias, a.batch_bias, residual, y, s_out, groups, stats, st);

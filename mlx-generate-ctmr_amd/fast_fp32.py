@@ -8,8 +8,8 @@ hand-written HIP kernels of ``libctmr_hip.so``:
 
 * padding-1 3x3x3 convolutions (stride 1/2, nearest-2x folded into parity
   weights, trilinear-2x computed while packing the input) and 1x1x1
-  convolutions are implicit GEMMs on FP32 MFMA (or bf16 MFMA with fp32
-  accumulation inside ``precision("bf16")``, or split fp16 -- the reference's
+  convolutions are implicit GEMMs on FP32 operands (three bf16 parts each on
+  bf16 MFMA, or FP32 MFMA; or bf16 MFMA with fp32 accumulation inside ``precision("bf16")``, or split fp16 -- the reference's
   "exact" mode for fp32 tensors, _nax_conv.py:27-35 -- on fp16 MFMA inside
   ``precision("f16x2")``);
 * a preceding group norm + SiLU is applied while packing the convolution
@@ -54,7 +54,7 @@ _precision: ContextVar[str] = ContextVar("ctmr_precision", default="fp32")
 
 @contextlib.contextmanager
 def precision(mode: str) -> Iterator[None]:
-    """Select ``"fp32"`` (FP32 MFMA), ``"bf16"`` (bf16 MFMA, fp32 accumulate) or ``"f16x2"`` convs.
+    """Select ``"fp32"`` (fp32 products), ``"bf16"`` (bf16 MFMA, fp32 accumulate) or ``"f16x2"`` convs.
 
     ``"f16x2"`` is the reference's exact mode for fp32 tensors (``_nax_conv.py:27-35``): each fp32
     value is split into an fp16 high half and an fp16 low half scaled by 2^11, weights are scaled per
@@ -62,7 +62,7 @@ def precision(mode: str) -> Iterator[None]:
     MFMA with fp32 accumulation (about 2^-22 relative per product).  It applies to the stride-1
     3x3x3 convs the LDS-staged 16-bit GEMM takes (cout a multiple of 64, at least 16 input
     channels) and to flash attention (the reference's split-fp16 kernel, ``_flash_attention.py:
-    140-290``); every other conv runs on FP32 MFMA.  Values must stay below 65504 in magnitude."""
+    140-290``); every other conv runs as under ``"fp32"``.  Values must stay below 65504 in magnitude."""
     if mode not in PRECISIONS:
         raise ValueError(f"precision must be one of {PRECISIONS}; got {mode!r}")
     token = _precision.set(mode)
