@@ -350,6 +350,16 @@ int ctmr_add_gn_partials(int32_t n, int64_t s, int32_t c, const float* a, const 
 int ctmr_gn_apply(int32_t n, int64_t s, int32_t c, const float* x, const float* affine,
                   int32_t silu, float* y, void* stream);
 
+/* Group norm (+ SiLU) of a planar (n, c, s) tensor -- the reference's NCDHW
+ * layout, s voxels -- in one call: the statistics and (scale, offset) of
+ * ctmr_gn_affine and the apply of ctmr_gn_apply without a transposed copy
+ * (fast_fp32.group_norm_ncdhw, fast_fp32.py:102-118).  At most 1024 channels
+ * a group, under 2^31 values a (batch item, group); any 4-byte alignment; y
+ * may equal x.  Workspace: ctmr_gn_planar_workspace_bytes (0 for small runs). */
+int64_t ctmr_gn_planar_workspace_bytes(int32_t n, int64_t s, int32_t c, int32_t groups);
+int ctmr_gn_planar(int32_t n, int64_t s, int32_t c, int32_t groups, float eps, const float* x, const float* gamma,
+                   const float* beta, int32_t silu, float* y, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Down-sampling residual-block input (fast_fp32.residual_block_ncdhw's down
  * branch, fast_fp32.py:250-255: avg_pool3d of group_norm_ncdhw(x, silu) and
  * avg_pool3d of x) from one read of x: y = 2x2x2 average pool of

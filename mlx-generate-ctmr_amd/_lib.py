@@ -78,6 +78,8 @@ _PROTOTYPES = {
                                             _c_i32, _c_i32, _vp, _vp, _vp, _vp]),
     "ctmr_add_gn_partials": (_c_int, [_c_i32, _c_i64, _c_i32, _vp, _vp, _vp, _vp, _sz, _vp]),
     "ctmr_gn_apply": (_c_int, [_c_i32, _c_i64, _c_i32, _vp, _vp, _c_i32, _vp, _vp]),
+    "ctmr_gn_planar_workspace_bytes": (_c_i64, [_c_i32, _c_i64, _c_i32, _c_i32]),
+    "ctmr_gn_planar": (_c_int, [_c_i32, _c_i64, _c_i32, _c_i32, _f, _vp, _vp, _vp, _c_i32, _vp, _vp, _sz, _vp]),
     "ctmr_silu": (_c_int, [_c_i64, _vp, _vp, _vp]),
     "ctmr_resample": (_c_int, [_c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _vp, _vp, _vp]),
     "ctmr_gn_avgpool": (_c_int, [_c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _vp, _vp, _c_i32, _vp, _vp, _vp]),

@@ -476,6 +476,200 @@ __global__ __launch_bounds__(256) void resample_kernel(int op, int n, int d, int
   }
 }
 
+// ---------------------------------------------------------------------------
+// Group norm of a planar (NCDHW) tensor
+// ---------------------------------------------------------------------------
+// In NCDHW a (batch item, group) is one contiguous run of cpg * s values, so
+// the norm needs no transposed copy: statistics (fp64, fixed order), scale and
+// offset, apply and SiLU run over the run itself.  Bound by launches for small
+// tensors and by HBM for large ones.
+//  * Runs of up to kPlanarRun values stay in one workgroup's registers between
+//    the statistics and the apply: one launch, one read, one write.  512
+//    channels of 8x8x4 x 2 with the SiLU: 14.0 us a call, against 42.1 us as
+//    two transposed copies, statistics, finalize and apply (same bits).
+//  * Longer runs are cut into chunks: one launch writes each chunk's (sum, sum
+//    of squares), the next sums its run's chunk partials -- every workgroup
+//    the same sums in the same order -- and applies its chunk.
+// VEC 4 reads 16 bytes: s % 4 == 0 and 16-byte pointers, so that four values
+// share a channel; otherwise one value at a time.
+constexpr int kPlanarThreads = 1024;
+constexpr int kPlanarVecs = 8;                                     // vectors a thread of the one-launch form holds
+constexpr int kPlanarRun = kPlanarThreads * kPlanarVecs;           // x VEC values: the one-launch form's longest run
+constexpr int kPlanarChunk = 256 * 16;                             // vectors per chunk of the two-launch form
+constexpr int kPlanarMaxCpg = 1024;
+
+struct PlanarArgs {
+  const float* x;
+  const float* gamma;
+  const float* beta;
+  float* y;
+  double* part;     // (n * groups, chunks, 2)
+  int s, c, groups, cpg, chunks, silu;
+  float eps;
+};
+
+template <int VEC>
+struct PlanarVec {
+  float v[VEC];
+};
+
+template <int VEC>
+__device__ __forceinline__ PlanarVec<VEC> planar_load(const float* p) {
+  PlanarVec<VEC> o;
+  if constexpr (VEC == 4) {
+    const f4 q = *reinterpret_cast<const f4*>(p);
+    o.v[0] = q[0]; o.v[1] = q[1]; o.v[2] = q[2]; o.v[3] = q[3];
+  } else {
+    o.v[0] = p[0];
+  }
+  return o;
+}
+
+// Workgroup sum of (a, q) over BLOCK threads: a butterfly across each wave,
+// then the waves in order; every thread gets both sums.
+template <int BLOCK>
+__device__ __forceinline__ void planar_block_sum(double& a, double& q) {
+  __shared__ double ws[BLOCK / 64][2];
+  a = wave_butterfly_sum<1>(a);
+  q = wave_butterfly_sum<1>(q);
+  if ((threadIdx.x & 63) == 0) {
+    ws[threadIdx.x >> 6][0] = a;
+    ws[threadIdx.x >> 6][1] = q;
+  }
+  __syncthreads();
+  a = q = 0.0;
+#pragma unroll
+  for (int w = 0; w < BLOCK / 64; ++w) {
+    a += ws[w][0];
+    q += ws[w][1];
+  }
+}
+
+// The run's (scale, offset) pairs in LDS from its sums (gn_group_affine's
+// formulas), published by a barrier.
+template <int BLOCK>
+__device__ __forceinline__ void planar_affine(const PlanarArgs& p, int g, double sum, double sq, float2* aff) {
+  const double count = (double)p.s * p.cpg, mean = sum / count;
+  double var = sq / count - mean * mean;
+  if (var < 0) var = 0;
+  const double rstd = 1.0 / sqrt(var + (double)p.eps);
+  for (int cc = threadIdx.x; cc < p.cpg; cc += BLOCK) {
+    const int ch = g * p.cpg + cc;
+    const double scale = (double)p.gamma[ch] * rstd;
+    aff[cc] = float2{(float)scale, (float)((double)p.beta[ch] - mean * scale)};
+  }
+  __syncthreads();
+}
+
+// silu?(x * scale + offset) of vector i of the run (channel i * VEC / s).
+template <int VEC>
+__device__ __forceinline__ void planar_store(const PlanarArgs& p, float* yr, unsigned i, PlanarVec<VEC> q,
+                                             const float2* aff) {
+  const float2 a = aff[(i * VEC) / (unsigned)p.s];
+#pragma unroll
+  for (int k = 0; k < VEC; ++k) {
+    const float t = fmaf(q.v[k], a.x, a.y);
+    q.v[k] = p.silu ? silu_f(t) : t;
+  }
+  if constexpr (VEC == 4) *reinterpret_cast<f4*>(yr + (int64_t)i * 4) = f4{q.v[0], q.v[1], q.v[2], q.v[3]};
+  else yr[i] = q.v[0];
+}
+
+// Grid (groups, n); the run has at most kPlanarRun vectors.
+template <int VEC>
+__global__ __launch_bounds__(kPlanarThreads) void gn_planar_kernel(PlanarArgs p) {
+  __shared__ float2 aff[kPlanarMaxCpg];
+  const int g = blockIdx.x;
+  const unsigned vecs = (unsigned)((int64_t)p.s * p.cpg / VEC);
+  const int64_t base = ((int64_t)blockIdx.y * p.groups + g) * p.s * p.cpg;
+  const float* xr = p.x + base;
+  PlanarVec<VEC> q[kPlanarVecs];
+  double a = 0.0, b = 0.0;
+#pragma unroll
+  for (int u = 0; u < kPlanarVecs; ++u) {
+    const unsigned i = threadIdx.x + u * kPlanarThreads;
+    if (i < vecs) q[u] = planar_load<VEC>(xr + (int64_t)i * VEC);
+  }
+#pragma unroll
+  for (int u = 0; u < kPlanarVecs; ++u) {
+    if (threadIdx.x + u * kPlanarThreads >= vecs) continue;
+#pragma unroll
+    for (int k = 0; k < VEC; ++k) {
+      const double d = (double)q[u].v[k];
+      a += d;
+      b = fma(d, d, b);
+    }
+  }
+  planar_block_sum<kPlanarThreads>(a, b);
+  planar_affine<kPlanarThreads>(p, g, a, b, aff);
+#pragma unroll
+  for (int u = 0; u < kPlanarVecs; ++u) {
+    const unsigned i = threadIdx.x + u * kPlanarThreads;
+    if (i < vecs) planar_store<VEC>(p, p.y + base, i, q[u], aff);
+  }
+}
+
+// Grid (chunks, groups, n): chunk partials of every run.
+template <int VEC>
+__global__ __launch_bounds__(256) void gn_planar_partial_kernel(PlanarArgs p) {
+  const int run = blockIdx.z * p.groups + blockIdx.y;
+  const unsigned vecs = (unsigned)((int64_t)p.s * p.cpg / VEC);
+  const float* xr = p.x + (int64_t)run * p.s * p.cpg;
+  const unsigned i0 = blockIdx.x * (unsigned)kPlanarChunk + threadIdx.x;
+  double a = 0.0, b = 0.0;
+#pragma unroll
+  for (int u0 = 0; u0 < kPlanarChunk / 256; u0 += 8) {
+    PlanarVec<VEC> q[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (i0 + (u0 + u) * 256 < vecs) q[u] = planar_load<VEC>(xr + (int64_t)(i0 + (u0 + u) * 256) * VEC);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      if (i0 + (u0 + u) * 256 >= vecs) continue;
+#pragma unroll
+      for (int k = 0; k < VEC; ++k) {
+        const double d = (double)q[u].v[k];
+        a += d;
+        b = fma(d, d, b);
+      }
+    }
+  }
+  planar_block_sum<256>(a, b);
+  if (threadIdx.x == 0) {
+    double* o = p.part + ((int64_t)run * p.chunks + blockIdx.x) * 2;
+    o[0] = a;
+    o[1] = b;
+  }
+}
+
+// Grid (chunks, groups, n): the run's sums, then its chunk normalised.
+template <int VEC>
+__global__ __launch_bounds__(256) void gn_planar_apply_kernel(PlanarArgs p) {
+  __shared__ float2 aff[kPlanarMaxCpg];
+  const int run = blockIdx.z * p.groups + blockIdx.y;
+  const unsigned vecs = (unsigned)((int64_t)p.s * p.cpg / VEC);
+  const int64_t base = (int64_t)run * p.s * p.cpg;
+  double a = 0.0, b = 0.0;
+  for (int k = threadIdx.x; k < p.chunks; k += 256) {
+    const double* o = p.part + ((int64_t)run * p.chunks + k) * 2;
+    a += o[0];
+    b += o[1];
+  }
+  planar_block_sum<256>(a, b);
+  planar_affine<256>(p, blockIdx.y, a, b, aff);
+  const unsigned i0 = blockIdx.x * (unsigned)kPlanarChunk + threadIdx.x;
+#pragma unroll
+  for (int u0 = 0; u0 < kPlanarChunk / 256; u0 += 8) {
+    PlanarVec<VEC> q[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (i0 + (u0 + u) * 256 < vecs) q[u] = planar_load<VEC>(p.x + base + (int64_t)(i0 + (u0 + u) * 256) * VEC);
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (i0 + (u0 + u) * 256 < vecs) planar_store<VEC>(p, p.y + base, i0 + (u0 + u) * 256, q[u], aff);
+  }
+}
+
 }  // namespace ctmr
 
 using namespace ctmr;
@@ -658,6 +852,70 @@ int ctmr_resample(int32_t op, int32_t n, int32_t d, int32_t h, int32_t w, int32_
   hipLaunchKernelGGL(resample_kernel, dim3(elementwise_blocks(total)), dim3(256), 0,
                      (hipStream_t)stream, op, n, d, h, w, c, vec, x, y);
   return check_launch("resample");
+}
+
+// Chunks a run is cut into, 1 when one workgroup holds it (workspace-free).
+// The size rule leaves out the alignment, so the workspace depends on the
+// shape only; a run read one value at a time may take more chunks than `vec`
+// ones would, never fewer.
+static int64_t planar_chunks(int64_t s, int32_t cpg, int vec) {
+  const int64_t vecs = s * cpg / vec;
+  return vecs <= kPlanarRun ? 1 : ceil_div(vecs, kPlanarChunk);
+}
+
+static int planar_check(int32_t n, int64_t s, int32_t c, int32_t groups) {
+  if (n <= 0 || s <= 0 || c <= 0 || groups <= 0) return fail(CTMR_E_INVALID, "non-positive dimension");
+  if (c % groups != 0) return fail(CTMR_E_INVALID, "channels must be divisible by groups");
+  if (c / groups > kPlanarMaxCpg) return fail(CTMR_E_UNSUPPORTED, "planar group norm needs at most 1024 channels a group");
+  if (n > 65535 || groups > 65535 || s * (c / groups) >= (1ll << 31))
+    return fail(CTMR_E_UNSUPPORTED, "volume too large for the planar group norm");
+  return CTMR_OK;
+}
+
+int64_t ctmr_gn_planar_workspace_bytes(int32_t n, int64_t s, int32_t c, int32_t groups) {
+  const int rc = planar_check(n, s, c, groups);
+  if (rc) return rc;
+  const int64_t chunks = planar_chunks(s, c / groups, 1);
+  return chunks == 1 ? 0 : (int64_t)n * groups * chunks * 2 * (int64_t)sizeof(double);
+}
+
+int ctmr_gn_planar(int32_t n, int64_t s, int32_t c, int32_t groups, float eps, const float* x, const float* gamma,
+                   const float* beta, int32_t silu, float* y, void* workspace, size_t workspace_bytes, void* stream) {
+  const int64_t need = ctmr_gn_planar_workspace_bytes(n, s, c, groups);
+  if (need < 0) return (int)need;
+  if (!x || !gamma || !beta || !y) return fail(CTMR_E_INVALID, "null pointer");
+  if ((int64_t)workspace_bytes < need || (need > 0 && !workspace)) {
+    set_error("planar group-norm workspace %zu bytes < required %lld", workspace_bytes, (long long)need);
+    return CTMR_E_WORKSPACE;
+  }
+  const bool vec = s % 4 == 0 && (((uintptr_t)x | (uintptr_t)y) & 15) == 0;
+  PlanarArgs p;
+  p.x = x;
+  p.gamma = gamma;
+  p.beta = beta;
+  p.y = y;
+  p.part = (double*)workspace;
+  p.s = (int)s;
+  p.c = c;
+  p.groups = groups;
+  p.cpg = c / groups;
+  p.chunks = (int)planar_chunks(s, p.cpg, vec ? 4 : 1);
+  p.silu = silu;
+  p.eps = eps;
+  hipStream_t st = (hipStream_t)stream;
+  if (p.chunks == 1) {
+    if (vec) hipLaunchKernelGGL(gn_planar_kernel<4>, dim3(groups, n), dim3(kPlanarThreads), 0, st, p);
+    else hipLaunchKernelGGL(gn_planar_kernel<1>, dim3(groups, n), dim3(kPlanarThreads), 0, st, p);
+    return check_launch("gn_planar");
+  }
+  const dim3 grid((unsigned)p.chunks, groups, n);
+  if (vec) hipLaunchKernelGGL(gn_planar_partial_kernel<4>, grid, dim3(256), 0, st, p);
+  else hipLaunchKernelGGL(gn_planar_partial_kernel<1>, grid, dim3(256), 0, st, p);
+  const int rc = check_launch("gn_planar_partial");
+  if (rc) return rc;
+  if (vec) hipLaunchKernelGGL(gn_planar_apply_kernel<4>, grid, dim3(256), 0, st, p);
+  else hipLaunchKernelGGL(gn_planar_apply_kernel<1>, grid, dim3(256), 0, st, p);
+  return check_launch("gn_planar_apply");
 }
 
 }  // extern "C"

@@ -891,8 +891,25 @@ def pointwise_conv_ncdhw(array: Tensor, weight: Tensor, bias: Optional[Tensor], 
     return to_ncdhw(pointwise_conv(to_ndhwc(array), weight, bias))
 
 
+def _planar(array, num_groups: int) -> bool:
+    """Whether a group norm takes its NCDHW input as it lies (``ctmr_gn_planar``): what the NDHWC path accepts,
+    contiguous as NCDHW.  A tensor that lies as NDHWC (a permuted view) needs no copy there and stays on it, as
+    does everything that path refuses; groups of more than 1024 channels and runs of 2^31 values too."""
+    if (not isinstance(array, Tensor) or array.dim() != 5 or array.dtype != torch.float32
+            or array.device.type != "cuda" or not array.is_contiguous() or array.numel() == 0
+            or not isinstance(num_groups, int) or num_groups <= 0):
+        return False
+    n, c = int(array.shape[0]), int(array.shape[1])
+    return (c % num_groups == 0 and c <= (1024 if c % 4 == 0 else 256) and n <= 65535
+            and array.numel() // n // num_groups < 1 << 31)
+
+
 def group_norm_ncdhw(array: Tensor, weight: Tensor, bias: Tensor, *, num_groups: int, eps: float, mx=None,
                      apply_silu: bool = False) -> Tensor:
+    if _planar(array, num_groups):
+        c = int(array.shape[1])
+        gamma, beta = _vec(weight, c, "norm weight", array.device), _vec(bias, c, "norm bias", array.device)
+        return ops.gn_planar(array, gamma, beta, int(num_groups), float(eps), bool(apply_silu))
     return to_ncdhw(group_norm(to_ndhwc(array), weight, bias, num_groups=num_groups, eps=eps,
                                apply_silu=apply_silu))
 

@@ -414,6 +414,27 @@ def _(x, affine, silu):
     return torch.empty_like(x)
 
 
+@_custom_op("ctmr::gn_planar")
+def gn_planar(x: Tensor, gamma: Tensor, beta: Tensor, groups: int, eps: float, silu: bool) -> Tensor:
+    """``ctmr_gn_planar``: group norm and optional SiLU of a contiguous NCDHW tensor, as it lies."""
+    _require_device(x, gamma, beta)
+    n, c = int(x.shape[0]), int(x.shape[1])
+    s = x.numel() // (n * c)
+    lib = _lib.lib()
+    nbytes = _lib.check(lib.ctmr_gn_planar_workspace_bytes(n, s, c, groups), "ctmr_gn_planar_workspace_bytes")
+    y = torch.empty_like(x)
+    ws = torch.empty(nbytes, device=x.device, dtype=torch.uint8) if nbytes else None
+    _lib.check(lib.ctmr_gn_planar(n, s, c, groups, float(eps), x.data_ptr(), gamma.data_ptr(), beta.data_ptr(),
+                                  int(silu), y.data_ptr(), _ptr(ws), nbytes, _stream(x.device)),
+               "ctmr_gn_planar")
+    return y
+
+
+@gn_planar.register_fake
+def _(x, gamma, beta, groups, eps, silu):
+    return torch.empty_like(x)
+
+
 @_custom_op("ctmr::silu")
 def silu(x: Tensor) -> Tensor:
     """Elementwise ``x / (1 + exp(-x))``."""
