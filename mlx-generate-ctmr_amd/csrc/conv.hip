@@ -1008,12 +1008,24 @@ __device__ __forceinline__ void store_tile(const ConvArgs& p, f4 (&acc)[4][NSUB]
 // K range s as above, and set 0 adds set 1's sum after the bias (the split
 // reduction's order: bias, range 0, range 1, residual), so the launch writes
 // the outputs and their group-norm partials with no partial planes.
+// X3: the fp32 products as three bf16 parts per operand (conv_lds.hip), for
+// K blocks in pairs: a step is 32 channels, lane group g holding channels 8g ..
+// 8g + 7 of A and B (two 16-byte loads each), split in registers by every wave
+// -- 352 VALU operations a wave and step beside 96 MFMAs of 16 cycles, where
+// FP32 MFMA takes 128 of 32.  Each raw operand register is refilled for the
+// next step as soon as it is split, so one set of raw registers suffices.
+// Bound by those VALU operations as much as by the MFMAs.  Measured, FP32 MFMA
+// / part products us: 16x16x8 x 2, 256 channels (split waves) 120 / 98, 8x8x4
+// x 2, 512 channels 70 / 62, 25^3, 256 channels 549 / 336, 49x49x33, 256
+// channels 2431 / 1627; UNet pass 12.29 -> 11.82 ms.
 template <int DT, int NSUB, int WM, int WN, int KT, int STRIDE, bool UP, bool DIRECT = false, int KWS = 1,
-          int SETS = 1>
+          int SETS = 1, bool X3 = false>
 __global__ __launch_bounds__(256 * SETS, SETS == 1 ? 2 : 1) void conv_kernel(ConvArgs p) {
   static_assert(WM * WN * KWS == 4, "four waves per wave set");
   static_assert(SETS == 1 || (SETS == 2 && KWS == 4), "two wave sets only with the four-wave K split");
   static_assert(!DIRECT || (KT == 3 && !UP && DT == CTMR_F32), "direct reads: plain fp32 3x3x3 convs");
+  static_assert(!X3 || (KT > 1 && DT == CTMR_F32), "part products: fp32 convs over taps");
+  constexpr int kStep = X3 ? 2 : 1;  // K blocks per step
   const int lane = threadIdx.x & 63;
   // Wave index made provably uniform so every address base below lives in SGPRs.
   const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1070,7 +1082,7 @@ __global__ __launch_bounds__(256 * SETS, SETS == 1 ? 2 : 1) void conv_kernel(Con
       const int d = v / ghw, r = v - d * ghw;
       const int h = r / p.gw, w = r - h * p.gw;
       const int zi = STRIDE * d - 1, yi = STRIDE * h - 1, xi = STRIDE * w - 1;
-      lane_off[ms] = ((zi * p.in_h + yi) * p.in_w + xi) * (int)p.row_bytes + lgrp * 16;
+      lane_off[ms] = ((zi * p.in_h + yi) * p.in_w + xi) * (int)p.row_bytes + lgrp * 16 * kStep;
       unsigned m = 0;
 #pragma unroll
       for (int t = 0; t < 3; ++t) {
@@ -1081,7 +1093,7 @@ __global__ __launch_bounds__(256 * SETS, SETS == 1 ? 2 : 1) void conv_kernel(Con
       vmask[ms] = m;
       aoff[ms] = 0;
     } else {
-      aoff[ms] = (int)((window_row(min(m0 + ms * 16 + lrow, S - 1)) - row0) * p.row_bytes) + lgrp * 16;
+      aoff[ms] = (int)((window_row(min(m0 + ms * 16 + lrow, S - 1)) - row0) * p.row_bytes) + lgrp * 16 * kStep;
     }
   }
   // B: one output column per lane per 16-column block.
@@ -1091,7 +1103,8 @@ __global__ __launch_bounds__(256 * SETS, SETS == 1 ? 2 : 1) void conv_kernel(Con
       (void*)(p.wp + bbase_off), (short)0, (int)min(p.w_bytes - bbase_off, (int64_t)0x7fffffff), 0x00020000);
   int boff[NSUB];
 #pragma unroll
-  for (int ns = 0; ns < NSUB; ++ns) boff[ns] = min(n0 + ns * 16 + lrow, p.np - 1) * 64 + lgrp * 16;
+  for (int ns = 0; ns < NSUB; ++ns)
+    boff[ns] = min(n0 + ns * 16 + lrow, p.np - 1) * 64 + (X3 ? (lgrp >> 1) * p.np * 64 + (lgrp & 1) * 32 : lgrp * 16);
 
   f4 acc[4][NSUB];
 #pragma unroll
@@ -1099,7 +1112,7 @@ __global__ __launch_bounds__(256 * SETS, SETS == 1 ? 2 : 1) void conv_kernel(Con
 #pragma unroll
     for (int ns = 0; ns < NSUB; ++ns) acc[ms][ns] = f4{0.f, 0.f, 0.f, 0.f};
 
-  const int steps = p.taps * p.kb;
+  const int steps = p.taps * p.kb / kStep;  // X3: kb is even
   // Wave-uniform (readfirstlane) so the loop counter and the load cursor
   // derived from them stay in SGPRs.
   const int kpart = split_id * SETS + set, kparts = p.split * SETS;
@@ -1107,15 +1120,15 @@ __global__ __launch_bounds__(256 * SETS, SETS == 1 ? 2 : 1) void conv_kernel(Con
   const int g_end = (int)((int64_t)(kpart + 1) * steps / kparts);
   const int s_begin = __builtin_amdgcn_readfirstlane(g_begin + (g_end - g_begin) * wave_k / KWS);
   const int s_end = __builtin_amdgcn_readfirstlane(g_begin + (g_end - g_begin) * (wave_k + 1) / KWS);
-  const int bstep = p.np * 64;
+  const int bstep = p.np * 64 * kStep;
 
-  // Load cursor over the step sequence (tap-major, 64-byte channel block
-  // minor), advanced incrementally so a step costs a few scalar adds.
+  // Load cursor over the step sequence (tap-major, channel block minor),
+  // advanced incrementally so a step costs a few scalar adds.
   const int rb = (int)p.row_bytes;
   int c_kb, c_tw, c_th, c_td, c_tapoff, c_bo;
   {
-    const int tap = s_begin / p.kb;
-    c_kb = s_begin - tap * p.kb;
+    const int tap = s_begin * kStep / p.kb;
+    c_kb = s_begin * kStep - tap * p.kb;
     c_tw = tap % KT;
     c_th = (tap / KT) % KT;
     c_td = tap / (KT * KT);
@@ -1138,17 +1151,13 @@ __global__ __launch_bounds__(256 * SETS, SETS == 1 ? 2 : 1) void conv_kernel(Con
     }
   };
   direct_offsets();
-  auto load = [&](u4 (&A)[4], u4 (&B)[NSUB]) {
-    // readfirstlane: the step offsets are wave-uniform; saying so keeps them in
-    // SGPRs (buffer soffset) instead of a per-lane waterfall.
-    const int ao = __builtin_amdgcn_readfirstlane(DIRECT ? c_kb * 64 : c_tapoff + c_kb * 64);
-    const int bo = __builtin_amdgcn_readfirstlane(c_bo);
-#pragma unroll
-    for (int ms = 0; ms < 4; ++ms) A[ms] = __builtin_amdgcn_raw_buffer_load_b128(arsrc, aoff[ms], ao, 0);
-#pragma unroll
-    for (int ns = 0; ns < NSUB; ++ns) B[ns] = __builtin_amdgcn_raw_buffer_load_b128(brsrc, boff[ns], bo, 0);
+  // readfirstlane: the step offsets are wave-uniform; saying so keeps them in
+  // SGPRs (buffer soffset) instead of a per-lane waterfall.
+  auto a_step = [&]() { return __builtin_amdgcn_readfirstlane(DIRECT ? c_kb * 64 : c_tapoff + c_kb * 64); };
+  auto b_step = [&]() { return __builtin_amdgcn_readfirstlane(c_bo); };
+  auto advance = [&]() {
     c_bo += bstep;
-    if (++c_kb == p.kb) {
+    if ((c_kb += kStep) == p.kb) {
       c_kb = 0;
       c_tapoff += rb;
       if (++c_tw == KT) {
@@ -1163,6 +1172,14 @@ __global__ __launch_bounds__(256 * SETS, SETS == 1 ? 2 : 1) void conv_kernel(Con
       direct_offsets();
     }
   };
+  auto load = [&](u4 (&A)[4], u4 (&B)[NSUB]) {
+    const int ao = a_step(), bo = b_step();
+#pragma unroll
+    for (int ms = 0; ms < 4; ++ms) A[ms] = __builtin_amdgcn_raw_buffer_load_b128(arsrc, aoff[ms], ao, 0);
+#pragma unroll
+    for (int ns = 0; ns < NSUB; ++ns) B[ns] = __builtin_amdgcn_raw_buffer_load_b128(brsrc, boff[ns], bo, 0);
+    advance();
+  };
   auto compute = [&](const u4 (&A)[4], const u4 (&B)[NSUB]) { mma_block<DT, NSUB, true>(acc, A, B); };
 
   // Register double buffer: the next K block is in flight while this one
@@ -1176,22 +1193,118 @@ __global__ __launch_bounds__(256 * SETS, SETS == 1 ? 2 : 1) void conv_kernel(Con
   // last step reads through the buffer descriptors -- in range it is data
   // that is never used, out of range the hardware returns zeros -- so it is
   // harmless.
-  u4 A0[4], B0[NSUB], A1[4], B1[NSUB];
-  load(A0, B0);  // step s_begin; each load() fetches the cursor's step, then advances it
-  for (int s = s_begin; s < s_end; s += 2) {
-    load(A1, B1);
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_setprio(1);  // MFMA bursts win issue slots over address/load code
-    compute(A0, B0);
-    __builtin_amdgcn_s_setprio(0);
-    __builtin_amdgcn_sched_barrier(0);
-    if (s + 1 >= s_end) break;
-    load(A0, B0);
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_setprio(1);
-    compute(A1, B1);
-    __builtin_amdgcn_s_setprio(0);
-    __builtin_amdgcn_sched_barrier(0);
+  if constexpr (X3) {
+    u4 A[4][2], B[NSUB][2];
+    auto load_a = [&]() {
+      const int ao = a_step();
+#pragma unroll
+      for (int ms = 0; ms < 4; ++ms)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) A[ms][q] = __builtin_amdgcn_raw_buffer_load_b128(arsrc, aoff[ms] + 16 * q, ao, 0);
+    };
+    auto load_b = [&](int ns, int bo) {
+#pragma unroll
+      for (int q = 0; q < 2; ++q) B[ns][q] = __builtin_amdgcn_raw_buffer_load_b128(brsrc, boff[ns] + 16 * q, bo, 0);
+    };
+    auto split = [](const u4 (&v)[2], bf8 (&o)[3]) {
+      uint2 h[2], m[2], l[2];
+#pragma unroll
+      for (int q = 0; q < 2; ++q) split_bf16x3(__builtin_bit_cast(f4, v[q]), h[q], m[q], l[q]);
+      o[0] = __builtin_bit_cast(bf8, u4{h[0].x, h[0].y, h[1].x, h[1].y});
+      o[1] = __builtin_bit_cast(bf8, u4{m[0].x, m[0].y, m[1].x, m[1].y});
+      o[2] = __builtin_bit_cast(bf8, u4{l[0].x, l[0].y, l[1].x, l[1].y});
+    };
+    load_a();
+    {
+      const int bo = b_step();
+#pragma unroll
+      for (int ns = 0; ns < NSUB; ++ns) load_b(ns, bo);
+    }
+    advance();
+    for (int s = s_begin; s < s_end; ++s) {
+      bf8 pa[4][3];
+#pragma unroll
+      for (int ms = 0; ms < 4; ++ms) split(A[ms], pa[ms]);
+      __builtin_amdgcn_sched_barrier(0);
+      load_a();  // unconditional, as load() above
+      const int bo = b_step();
+      advance();
+#pragma unroll
+      for (int ns = 0; ns < NSUB; ++ns) {
+        bf8 pb[3];
+        split(B[ns], pb);
+        __builtin_amdgcn_sched_barrier(0);
+        load_b(ns, bo);
+        __builtin_amdgcn_s_setprio(1);
+        constexpr int ia[6] = {2, 1, 0, 1, 0, 0}, ib[6] = {0, 0, 0, 1, 1, 2};  // lh mh hh mm hm hl (A, B)
+#pragma unroll
+        for (int k = 0; k < 6; ++k)
+#pragma unroll
+          for (int ms = 0; ms < 4; ++ms)
+            acc[ms][ns] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pb[ib[k]], pa[ms][ia[k]], acc[ms][ns], 0, 0, 0);
+        __builtin_amdgcn_s_setprio(0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    // Results that are not finite, again in plain fp32 (x3_recompute's reason),
+    // one per lane and pass; bit e of `bad` is row block e / (4 NSUB), column
+    // block (e / 4) % NSUB, column e % 4 of the lane's four.
+    static_assert(16 * NSUB <= 64, "one bit per result");
+    unsigned long long bad = 0;
+#pragma unroll
+    for (int e = 0; e < 16 * NSUB; ++e)
+      if (!(fabsf(acc[e / (4 * NSUB)][(e / 4) % NSUB][e & 3]) < INFINITY)) bad |= 1ull << e;
+    while (__any(bad != 0)) {
+      if (bad == 0) continue;
+      const int e = __builtin_ctzll(bad);
+      bad &= bad - 1;
+      const int ms = e / (4 * NSUB), ns = (e / 4) % NSUB;
+      const int col = min(n0 + ns * 16 + 4 * lgrp + (e & 3), p.np - 1);
+      const int v = min(m0 + ms * 16 + lrow, S - 1);
+      const int d = v / ghw, r = v - d * ghw, h = r / p.gw, w = r - h * p.gw;
+      const int64_t row = window_row(v);
+      float sum = 0.f;
+#pragma clang loop unroll(disable)
+      for (int s = s_begin * kStep; s < s_end * kStep; ++s) {
+        const int tap = s / p.kb, kb = s - tap * p.kb;
+        const int td = tap / (KT * KT), th = (tap / KT) % KT, tw = tap % KT;
+        bool in = true;
+        int64_t off;
+        if constexpr (DIRECT) {
+          const int z = STRIDE * d - 1 + td, y = STRIDE * h - 1 + th, x = STRIDE * w - 1 + tw;
+          in = z >= 0 && z < p.in_d && y >= 0 && y < p.in_h && x >= 0 && x < p.in_w;
+          off = ((int64_t)z * p.in_h + y) * p.in_w + x;
+        } else {
+          off = row + (int64_t)td * p.P + (int64_t)th * p.Q + tw;
+        }
+        const float* xa = reinterpret_cast<const float*>(
+            p.xp + ((int64_t)b * p.rows_per_batch + (in ? off : 0)) * p.row_bytes + kb * 64);
+        const float* wb = reinterpret_cast<const float*>(p.wp + bbase_off + ((int64_t)s * p.np + col) * 64);
+#pragma clang loop unroll(disable)
+        for (int c = 0; c < 16; ++c) sum = fmaf(in ? xa[c] : 0.f, wb[c], sum);
+      }
+#pragma unroll
+      for (int k = 0; k < 16 * NSUB; ++k)
+        if (k == e) acc[k / (4 * NSUB)][(k / 4) % NSUB][k & 3] = sum;
+    }
+  } else {
+    u4 A0[4], B0[NSUB], A1[4], B1[NSUB];
+    load(A0, B0);  // step s_begin; each load() fetches the cursor's step, then advances it
+    for (int s = s_begin; s < s_end; s += 2) {
+      load(A1, B1);
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_setprio(1);  // MFMA bursts win issue slots over address/load code
+      compute(A0, B0);
+      __builtin_amdgcn_s_setprio(0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (s + 1 >= s_end) break;
+      load(A0, B0);
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_setprio(1);
+      compute(A1, B1);
+      __builtin_amdgcn_s_setprio(0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
   }
 
   const int tile_id = UP ? phase * p.m_tiles + m_tile : m_tile;
@@ -2775,12 +2888,14 @@ static int geometry(const ctmr_conv_desc* d, Geometry& g) {
       return CTMR_OK;
     }
   }
-  // LDS-staged GEMM: stride-1 fp32 volumes whose 4x8x8 bricks are at least
-  // 3/4 full, with at least 64 input channels (4 staged chunks; measured on
-  // MI355X: 64-channel UNet-level convs 3-6 % faster than the streaming GEMM
-  // with or without its pack pass; below that the per-chunk staging and
-  // barriers dominate), 64-wide column tiles, at least 4 chunks per split, and
-  // 6 staged planes within 32-bit buffer offsets.
+  // LDS-staged GEMM: stride-1 fp32 volumes with at least 64 input channels,
+  // 64-wide column tiles and 6 staged planes within 32-bit buffer offsets,
+  // whose 4x8x8 bricks are at least 3/4 full, or 0.6 full with the grid's
+  // last round of 512 workgroups not too empty (0.8 of the rounds' slots
+  // taken).  Measured, streaming / LDS us: 49x49x33 (0.68 full) 64 channels
+  // 146 / 140, 128 488 / 434, 256 1627 / 1660; 33x41x25 (0.61) 128 255 / 231,
+  // 256 913 / 812; 20^3 x 2 (0.69) 256 355 / 425 (0.70 of the slots), 512 1298
+  // / 1331; 25^3 (0.54) 256 336 / 428, 512 1290 / 1594.
   g.lds = false;
   g.wsets = 1;
   g.lds16 = false;
@@ -2793,13 +2908,19 @@ static int geometry(const ctmr_conv_desc* d, Geometry& g) {
     g.tx = (int)ceil_div(d->w, kBW);
     const int64_t slots = (int64_t)g.tz * g.ty * g.tx * kBD * kBH * kBW;
     const int64_t planes = (int64_t)kHD * d->h * d->w * d->cin * 4;
-    // The policy split (below) must leave each workgroup at least 4 chunks:
-    // with fewer, the exposed first-chunk staging outweighs the saved pack
-    // (measured on the UNet's 16x16x8 level: streaming 68 % vs LDS 63 %).
+    // A split must leave each range at least 4 chunks (with fewer, the exposed
+    // first-chunk staging and the partial planes outweigh the faster products:
+    // 20^3 x 2, 128 channels, split waves 112 us, LDS in 3 ranges 140), or 2
+    // chunks where it is two wave sets of one workgroup: 60x44x28, 64 channels
+    // 146 / 134 us.
     const int64_t base = (int64_t)g.tz * g.ty * g.tx * (d->cout / 64) * d->n;
     const int64_t policy_split = lds_policy_split(base, d->cin / 16);
     const int64_t split = d->split > 0 ? d->split : policy_split;
-    if (4 * S >= 3 * slots && planes < (1ll << 31) && brick_out_fits && (d->cin / 16) / split >= 4) g.lds = true;
+    const int64_t chunks = d->cin / 16, range = chunks / split;
+    const bool full = 4 * S >= 3 * slots || (5 * S >= 3 * slots &&
+                                             5 * base * split >= 4 * 512 * ceil_div(base * split, 512));
+    if (full && planes < (1ll << 31) && brick_out_fits &&
+        (range >= 4 || (split == 2 && chunks % 2 == 0 && range >= 2))) g.lds = true;
   }
   if (g.lds) {
     g.pack = false;
@@ -3022,8 +3143,16 @@ template <int DT, int NSUB, int WM, int WN, int KT, int STRIDE, bool UP, bool DI
 static void launch_conv(dim3 grid, dim3, hipStream_t st, const ConvArgs& a) {
   // KWS = 4 holds 48 KiB of quarter sums in LDS: 8 KiB more keeps it at two per CU.  Two wave sets (512
   // threads, 96 KiB of quarter sums) run one per CU.
-  hipLaunchKernelGGL((conv_kernel<DT, NSUB, WM, WN, KT, STRIDE, UP, DIRECT, KWS, SETS>), grid, dim3(256 * SETS),
-                     SETS == 2 ? 0 : KWS > 1 ? 8 * 1024 : NSUB == 4 ? kConvTwoPerCuLds : 0, st, a);
+  const size_t lds = SETS == 2 ? 0 : KWS > 1 ? 8 * 1024 : NSUB == 4 ? kConvTwoPerCuLds : 0;
+  if constexpr (DT == CTMR_F32 && KT > 1 && NSUB >= 2) {
+    if (a.kb % 2 == 0) {  // channel blocks in pairs
+      hipLaunchKernelGGL((conv_kernel<DT, NSUB, WM, WN, KT, STRIDE, UP, DIRECT, KWS, SETS, true>), grid,
+                         dim3(256 * SETS), lds, st, a);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((conv_kernel<DT, NSUB, WM, WN, KT, STRIDE, UP, DIRECT, KWS, SETS>), grid, dim3(256 * SETS), lds,
+                     st, a);
 }
 
 // Compute units of the current device (cached per device).

@@ -1,6 +1,6 @@
-"""The fp32 LDS-staged GEMM's part products (three bf16 parts per operand, six products): each product must
-hold fp32's precision at the operands' own exponents, and a result that is not finite must be the fp32
-convolution's.
+"""The part products (three bf16 parts per operand, six products) of the fp32 LDS-staged and register-streaming
+GEMMs: each product must hold fp32's precision at the operands' own exponents, and a result that is not finite
+must be the fp32 convolution's.
 
 The float64 bar is elementwise, derived from the method: per product the dropped parts and the roundings of
 the parts are below 2^-23 of |a w|, and the sum rounds once per 16 channels and part product, each rounding at
@@ -104,3 +104,83 @@ def test_not_finite_through_the_norm_and_silu(ctmr, dev):
     taint = torch.zeros(1, 4, 8, 8, dtype=torch.bool)
     taint[0, 0:3, 2:5, 2:5] = True
     assert torch.equal(y.isnan().all(-1), taint) and torch.equal(y.isnan().any(-1), taint)
+
+
+# The register-streaming GEMM (whole pairs of 16-channel blocks; an odd block count stays on FP32 MFMA):
+# (name, shape, cout, options, kernel)
+STREAM_CASES = [
+    ("direct reads, one tile", (1, 3, 4, 5, 64), 64, {"stream_gemm": True, "split": 1}, "stream_direct"),
+    ("direct, remainder rows and columns", (2, 5, 7, 9, 32), 48, {"stream_gemm": True, "split": 1}, "stream_direct"),
+    ("two 16-column blocks", (1, 6, 9, 11, 32), 32, {"split": 1}, "stream_direct"),
+    ("128-wide tiles, odd split of the steps", (1, 5, 6, 7, 96), 128, {"split": 7}, "stream_direct"),
+    ("an odd block count", (1, 5, 6, 7, 48), 64, {"split": 1}, "stream_direct"),
+    ("stride 2, ragged", (1, 7, 9, 10, 64), 96, {"stride": 2, "split": 1}, "stream_direct"),
+    ("packed copy", (1, 4, 5, 6, 64), 64, {"stream_gemm": True, "split": 2, "silu": True}, "stream"),
+    ("nearest-2x", (1, 3, 4, 5, 64), 64, {"upsample": True, "split": 1}, "stream"),
+    ("nearest-2x, 128-wide", (2, 3, 5, 4, 128), 128, {"upsample": True}, "split_waves"),
+    ("trilinear-2x", (1, 3, 4, 5, 64), 64, {"trilinear": True, "split": 1}, "stream"),
+    ("split over four waves", (2, 8, 8, 4, 128), 128, {}, "split_waves"),
+    ("split over four waves, two sets", (1, 18, 21, 11, 256), 256, {}, "split_waves"),
+]
+
+
+def _stream_conv(ctmr, dev, x, w, cout, options, kernel):
+    """The op on the named route, and the float64 result with its bar (of |x|, |w|)."""
+    f, L, ops = ctmr.fast_fp32, ctmr._lib, ctmr.ops
+    opts = dict(options)
+    mode = (L.MODE_NEAREST2X if opts.get("upsample") else L.MODE_TRILINEAR2X if opts.get("trilinear")
+            else L.MODE_PLAIN)
+    flags = (L.F_STREAM if opts.get("stream_gemm") else 0) | (L.F_SILU if opts.get("silu") else 0)
+    desc = ops.make_desc(tuple(x.shape), cout, 3, opts.get("stride", 1), mode, flags, L.DT_F32, opts.get("split", 0))
+    assert L.conv_kernel(desc) == kernel
+    packed = (f.pack_upsample_weight if opts.get("upsample") else f.pack_weight)(w.to(dev), dtype="fp32")
+    y = f.implicit_gemm_conv3d(x.to(dev), packed, None, cout=cout, **opts).cpu()
+    xd = x.double()
+    if opts.get("silu"):
+        xd = xd * torch.sigmoid(xd)
+    if opts.get("upsample"):
+        for axis in (1, 2, 3):
+            xd = xd.repeat_interleave(2, axis)
+    if opts.get("trilinear"):
+        xd = torch.nn.functional.interpolate(xd.permute(0, 4, 1, 2, 3), scale_factor=2, mode="trilinear",
+                                             align_corners=False).permute(0, 2, 3, 4, 1)
+    st = opts.get("stride", 1)
+    sub = (slice(None), *(slice(None, None, st),) * 3)
+    # the staging transform and the parity fold round once more each: 2e-6 of the operands together
+    return y, _conv64(xd, w)[sub], lambda a, b: (_bar(a, b) + 2e-6 * _conv64(a.abs(), b.abs()))[sub], xd
+
+
+@pytest.mark.parametrize(("name", "shape", "cout", "options", "kernel"), STREAM_CASES, ids=[c[0] for c in STREAM_CASES])
+def test_streaming_products_hold_fp32(ctmr, dev, name, shape, cout, options, kernel):
+    g = torch.Generator().manual_seed(23)
+    wide = 0 if options.get("silu") else 30
+    scale = torch.exp2(torch.randint(-wide, wide + 1, (shape[-1],), generator=g).float())
+    x = torch.randn(*shape, generator=g) * scale
+    w = torch.randn(cout, shape[-1], 3, 3, 3, generator=g) / scale.reshape(1, -1, 1, 1, 1)
+    y, ref, bar, xd = _stream_conv(ctmr, dev, x, w, cout, options, kernel)
+    err, limit = (y.double() - ref).abs(), bar(xd, w)
+    assert bool((err <= limit).all()), f"{name}: {(err / limit).max():.2f} of the bar"
+
+
+@pytest.mark.parametrize(("name", "shape", "cout", "options", "kernel"),
+                         [c for c in STREAM_CASES if not c[3].get("trilinear")],
+                         ids=[c[0] for c in STREAM_CASES if not c[3].get("trilinear")])
+def test_streaming_results_that_are_not_finite(ctmr, dev, name, shape, cout, options, kernel):
+    g = torch.Generator().manual_seed(29)
+    x, w = torch.randn(*shape, generator=g), torch.randn(cout, shape[-1], 3, 3, 3, generator=g) * 0.02
+    n, d, h, wd, c = shape
+    x[n - 1, d - 1, h - 1, wd - 1, c - 1] = float("nan")
+    if not options.get("silu"):  # the staged SiLU itself turns these into NaN
+        x[0, 0, 0, 0, 3] = float("inf")
+        x[0, d - 1, 0, wd - 1, 9] = 3.402e38  # rounds to infinity in bf16; finite here
+    y, ref, bar, xd = _stream_conv(ctmr, dev, x, w, cout, options, kernel)
+    ref = torch.where(ref.abs() > 3.4028235e38, torch.sign(ref) * float("inf"), ref)
+    if options.get("upsample"):  # the parity fold adds weights before they meet an infinity
+        assert torch.equal(y.isfinite(), ref.isfinite())
+    else:
+        assert torch.equal(y.isnan(), ref.isnan()) and torch.equal(y.isposinf(), ref.isposinf())
+        assert torch.equal(y.isneginf(), ref.isneginf())
+    ok = ref.isfinite()
+    xa = torch.nan_to_num(xd.abs(), 0.0, 0.0, 0.0)
+    limit = bar(xa, w) + np.sqrt(27 * c) * 4 * 2.0 ** -24 * ref.abs().nan_to_num(0.0, 0.0, 0.0).clamp(min=1e-3)
+    assert bool(((y.double() - ref).abs() <= limit)[ok].all()) and bool((~ok).any())
