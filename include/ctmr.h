@@ -387,11 +387,13 @@ int ctmr_resample(int32_t op, int32_t n, int32_t d, int32_t h, int32_t w, int32_
  * ldk / ldv; out is (n, lq, heads * head_dim) with row stride ldo.  q, k and v
  * may be column slices of one fused (n, l, 3C) projection.  head_dim must be
  * 32 (the MAISI UNet's num_head_channels).  Any lq, lk >= 1.  query_tiles
- * picks 16 (1) or 32 (2) queries per wave, 0 = the library's policy; results
- * are bit-identical either way (keys are visited in the same fixed order:
- * ascending 32-key blocks, or -- for grids of under two waves per SIMD, decided
- * from n, lq, lk and heads only -- two such runs over the key halves, combined
- * first half first). */
+ * (0, 1 or 2) is a hint: every wave takes 16 queries, the fastest form
+ * throughout, and results do not depend on it.  Keys are visited in a fixed
+ * order: ascending 32-key blocks, or -- for small grids, decided from n, lq, lk
+ * and heads only -- two such runs over the key halves, combined first half
+ * first.  The fp32 operands are multiplied as three bf16 parts that together
+ * hold their 24 significant bits (as CTMR_K_LDS convolutions); output rows that
+ * are not finite are recomputed with plain fp32 products. */
 typedef struct ctmr_attn_desc {
   int32_t n, lq, lk, heads, head_dim, query_tiles;
   int64_t ldq, ldk, ldv, ldo;
@@ -404,16 +406,15 @@ int ctmr_flash_attention(const ctmr_attn_desc* desc, const float* q, const float
 /* The same attention in the reference's split-fp16 arithmetic, its matrix-unit
  * kernel (_flash_attention.py:140-290, chosen at :336-350 when the device has
  * one): q * scale * log2(e), k and v are split into fp16 halves hi = fp16(x),
- * lo = fp16((x - hi) * 2^11) (_flash_attention.py:314-317) in the caller's
- * workspace, and each product runs as hi*hi + (hi*lo + lo*hi) * 2^-11 on fp16
- * MFMA with fp32 accumulation; P = 2^(S - m) is split the same way and the
- * cross terms of P V are summed apart and added at the end.  About 2^-22
- * relative per product; |q * scale * log2(e)|, |k| and |v| must stay below
- * 65504.  Same descriptor, checks, tilings and bit-identity across
- * query_tiles as ctmr_flash_attention.  workspace: at least
+ * lo = fp16((x - hi) * 2^11) (_flash_attention.py:314-317), and each product
+ * runs as hi*hi + (hi*lo + lo*hi) * 2^-11 on fp16 MFMA with fp32 accumulation;
+ * P = 2^(S - m) is split the same way and the cross terms of P V are summed
+ * apart and added at the end.  About 2^-22 relative per product;
+ * |q * scale * log2(e)|, |k| and |v| must stay below 65504.  Same descriptor,
+ * checks and key order as ctmr_flash_attention.  workspace: at least
  * ctmr_flash_attention_f16x2_workspace_bytes(desc) bytes, 256-byte aligned
- * (-1 from that call for an invalid shape); calls sharing a workspace must not
- * overlap. */
+ * (-1 from that call for an invalid shape); checked, but not written: the
+ * kernel splits each key block into LDS. */
 int64_t ctmr_flash_attention_f16x2_workspace_bytes(const ctmr_attn_desc* desc);
 int ctmr_flash_attention_f16x2(const ctmr_attn_desc* desc, const float* q, const float* k, const float* v,
                                float* out, void* workspace, int64_t workspace_bytes, void* stream);

@@ -7,8 +7,6 @@
 
 namespace ctmr {
 
-typedef unsigned int u4 __attribute__((ext_vector_type(4)));
-
 // Cache-policy operands of the GEMMs' output stores (gfx950 encoding: bit 1 =
 // NT, non-temporal; bit 4 = SC1, device scope).  Same values under every
 // policy; measured on MI355X, default / NT / SC1, A/B twice in one run: the
@@ -79,29 +77,6 @@ constexpr int kBD = 4, kBH = 8, kBW = 8;
 constexpr int kHD = kBD + 2, kHH = kBH + 2, kHW = kBW + 2;
 constexpr int kHaloVox = kHD * kHH * kHW;                 // 600
 constexpr int kStageIters = (kHaloVox * 4 + 255) / 256;  // 16-byte pieces per thread
-
-typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
-typedef float f2v __attribute__((ext_vector_type(2)));
-
-// The three bf16 parts of four fp32 values, each part as 8 bytes.
-__device__ __forceinline__ void split_bf16x3(f4 v, uint2& h, uint2& m, uint2& l) {
-  unsigned ph[2], pm[2], pl[2];
-#pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    const f2v a = f2v{v[2 * k], v[2 * k + 1]};
-    const bf2 hb = __builtin_convertvector(a, bf2);
-    const f2v r = f2v{a[0] - (float)hb[0], a[1] - (float)hb[1]};
-    const bf2 mb = __builtin_convertvector(r, bf2);
-    const f2v q = f2v{r[0] - (float)mb[0], r[1] - (float)mb[1]};
-    const bf2 lb = __builtin_convertvector(q, bf2);
-    ph[k] = __builtin_bit_cast(unsigned, hb);
-    pm[k] = __builtin_bit_cast(unsigned, mb);
-    pl[k] = __builtin_bit_cast(unsigned, lb);
-  }
-  h = uint2{ph[0], ph[1]};
-  m = uint2{pm[0], pm[1]};
-  l = uint2{pl[0], pl[1]};
-}
 
 struct LdsArgs {
   const float* x;       // unpadded NDHWC input (channels [0, c1) of a two-source input)

@@ -46,13 +46,6 @@ constexpr int kX3Tap = 64 * kX3Row;                       // one tap's 64 column
 constexpr int kX3Set = kX3Halo + 2 * kX3Tap;              // 69888
 
 typedef float f16v __attribute__((ext_vector_type(16)));
-// Workgroup barrier that orders LDS only: global loads stay in flight across it.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // Brick line of row r = lane % 32 of MFMA row block mb: mb + brick32_line(r)
 // (column r % 8).
 __device__ __forceinline__ int brick32_line(int r) { return ((r >> 3) & 1) * 4 + (r >> 4) * 2; }

@@ -17,6 +17,9 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+typedef float f2v __attribute__((ext_vector_type(2)));
+typedef unsigned int u4 __attribute__((ext_vector_type(4)));
 
 // Message for the last failing call on this thread (ctmr_last_error).
 void set_error(const char* fmt, ...);
@@ -66,6 +69,33 @@ __device__ __forceinline__ void split_f16x4(f4 v, h4& hi, h4& lo) {
     hi[k] = (_Float16)v[k];
     lo[k] = (_Float16)((v[k] - (float)hi[k]) * 2048.0f);
   }
+}
+
+// The three bf16 parts of four fp32 values, each part as 8 bytes.
+__device__ __forceinline__ void split_bf16x3(f4 v, uint2& h, uint2& m, uint2& l) {
+  unsigned ph[2], pm[2], pl[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const f2v a = f2v{v[2 * k], v[2 * k + 1]};
+    const bf2 hb = __builtin_convertvector(a, bf2);
+    const f2v r = f2v{a[0] - (float)hb[0], a[1] - (float)hb[1]};
+    const bf2 mb = __builtin_convertvector(r, bf2);
+    const f2v q = f2v{r[0] - (float)mb[0], r[1] - (float)mb[1]};
+    const bf2 lb = __builtin_convertvector(q, bf2);
+    ph[k] = __builtin_bit_cast(unsigned, hb);
+    pm[k] = __builtin_bit_cast(unsigned, mb);
+    pl[k] = __builtin_bit_cast(unsigned, lb);
+  }
+  h = uint2{ph[0], ph[1]};
+  m = uint2{pm[0], pm[1]};
+  l = uint2{pl[0], pl[1]};
+}
+
+// Workgroup barrier that orders LDS only: global loads stay in flight across it.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
 // SiLU y * sigmoid(y) = y / (1 + e^-y), with e^-y = 2^(-y log2 e) on the

@@ -9,9 +9,9 @@ hand-written HIP kernels of ``libctmr_hip.so``:
 * padding-1 3x3x3 convolutions (stride 1/2, nearest-2x folded into parity
   weights, trilinear-2x computed while packing the input) and 1x1x1
   convolutions are implicit GEMMs on FP32 operands (three bf16 parts each on
-  bf16 MFMA, or FP32 MFMA; or bf16 MFMA with fp32 accumulation inside ``precision("bf16")``, or split fp16 -- the reference's
-  "exact" mode for fp32 tensors, _nax_conv.py:27-35 -- on fp16 MFMA inside
-  ``precision("f16x2")``);
+  bf16 MFMA, or FP32 MFMA; or bf16 MFMA with fp32 accumulation inside
+  ``precision("bf16")``, or split fp16 -- the reference's "exact" mode for fp32
+  tensors, _nax_conv.py:27-35 -- on fp16 MFMA inside ``precision("f16x2")``);
 * a preceding group norm + SiLU is applied while packing the convolution
   input; bias, the residual block's per-batch time-embedding bias and the
   residual join the fp32 sum before the single store;
@@ -700,8 +700,9 @@ def _rows(t: Tensor, name: str) -> Tensor:
 def flash_attention(q: Tensor, k: Tensor, v: Tensor, *, heads: int, scale: float, mx=None,
                     query_tiles: int = 0) -> Tensor:
     """``softmax(q k^T * scale) v`` on head-interleaved ``(B, L, heads * 32)`` projections
-    (``_flash_attention.flash_attention``, :320-360); FP32 MFMA, or under ``precision("f16x2")``
-    the reference's split-fp16 kernel; output in the same layout."""
+    (``_flash_attention.flash_attention``, :320-360); fp32 products (on bf16 MFMA, each operand in
+    three parts), or under ``precision("f16x2")`` the reference's split-fp16 kernel; output in the
+    same layout."""
     q, k, v = _rows(q, "q"), _rows(k, "k"), _rows(v, "v")
     if not flash_eligible(q, k, heads) or v.shape != k.shape or q.shape[0] != k.shape[0]:
         raise ValueError(f"flash attention needs (B, L, heads*32) q/k/v with heads={heads}; got "
@@ -712,7 +713,7 @@ def flash_attention(q: Tensor, k: Tensor, v: Tensor, *, heads: int, scale: float
 def _flash(q: Tensor, k: Tensor, v: Tensor, heads: int, scale: float, query_tiles: int) -> Tensor:
     """The HIP flash kernel for the active precision: under ``precision("f16x2")`` the
     reference's split-fp16 attention (its matrix-unit path, ``_flash_attention.py:336-350``),
-    else FP32 MFMA (``bf16`` keeps attention in FP32, as its norms and projections)."""
+    else fp32 products (``bf16`` keeps attention in FP32, as its norms and projections)."""
     if _precision.get() == "f16x2":
         return ops.flash_attention_f16x2(q, k, v, heads, scale, query_tiles)
     return ops.flash_attention(q, k, v, heads, scale, query_tiles)

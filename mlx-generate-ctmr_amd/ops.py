@@ -535,7 +535,7 @@ def flash_attention_f16x2(q: Tensor, k: Tensor, v: Tensor, heads: int, scale: fl
                           query_tiles: int = 0) -> Tensor:
     """``flash_attention`` in the reference's split-fp16 arithmetic (its matrix-unit kernel,
     ``_flash_attention.py:140-290``): q (scaled by ``scale * log2(e)``), k and v split into fp16
-    halves in a workspace, products hi*hi + (hi*lo + lo*hi) * 2^-11 on fp16 MFMA with fp32
+    halves inside the kernel, products hi*hi + (hi*lo + lo*hi) * 2^-11 on fp16 MFMA with fp32
     accumulation.  ``|q * scale * log2(e)|``, ``|k|`` and ``|v|`` must stay below 65504."""
     _require_device(q, k, v)
     n, lq, c = (int(s) for s in q.shape)
