@@ -144,14 +144,16 @@ int ctmr_conv3d_split(const ctmr_conv_desc* desc);
  * (fast_fp32.py:93-99, _nax_conv.py:578-581); tests and tools use it to
  * assert which kernel a shape takes (the choice depends on the desc only). */
 enum ctmr_conv_kernel {
-  CTMR_K_STREAM = 0,        /* register-streaming GEMM over the packed copy */
+  CTMR_K_STREAM = 0,        /* register-streaming GEMM over the packed copy (cin 8 at stride 2,
+                               large: x streamed plane by plane) */
   CTMR_K_STREAM_DIRECT = 1, /* register-streaming GEMM reading x itself */
   CTMR_K_LDS = 2,           /* fp32 LDS-staged GEMM (halo bricks of x, three bf16 parts) */
   CTMR_K_LDS_BF16 = 3,      /* bf16 LDS-staged GEMM over the packed copy */
   CTMR_K_POINTWISE = 4,     /* persistent one-tap GEMM (1x1x1, im2col rows) */
   CTMR_K_SPLIT_WAVES = 5,   /* 64 x 64 tiles, each split range over the four waves */
   CTMR_K_TAP_EXPAND = 6,    /* cout <= 4: 27*cout-column GEMM + tap sum */
-  CTMR_K_LDS_SMALL = 7,     /* cin 4 / 8: im2col rows read from an LDS halo brick */
+  CTMR_K_LDS_SMALL = 7,     /* cin 4 / 8: im2col rows read from an LDS halo brick (8 -> 8, large:
+                               LDS halo planes) */
   CTMR_K_SMALL_COUT = 8,    /* cout <= 4: direct FMA conv from an LDS halo brick */
   CTMR_K_LDS_F16X2 = 9      /* split-fp16 LDS-staged GEMM over the packed hi/lo copy */
 };
@@ -203,10 +205,12 @@ int ctmr_pack_upsample_weight(const ctmr_conv_desc* desc, const float* weight, v
  * One-tap GEMMs (1x1x1, im2col rows) with cout % 4 == 0 and
  * no per-batch bias or residual run on a persistent grid with the streaming
  * GEMM's per-output order, so their outputs equal the CTMR_F_STREAM ones bit
- * for bit.  With a split, each
- * contiguous range of the sequence is summed separately and the partial planes
- * are added in ascending order after the bias.  Kernel, split and tiling depend
- * on the desc only, so results are bit-identical run to run.
+ * for bit.  Large volumes of 8 input channels (stride 1 to 8 outputs, stride 2
+ * to 17 .. 32; CTMR_F_STREAM not set) are walked plane by plane, depth taps
+ * outermost, each fp32 operand in three bf16 parts; nothing is packed.  With
+ * a split, each contiguous range of the sequence is summed separately and the
+ * partial planes are added in ascending order after the bias.  Kernel, split
+ * and tiling depend on the desc only, so results are bit-identical run to run.
  */
 int ctmr_conv3d(const ctmr_conv_desc* desc, const float* x, const void* packed,
                 const float* bias, const float* affine, const float* residual, float* y,
@@ -263,8 +267,9 @@ int ctmr_conv3d_noalloc(const ctmr_conv_desc* desc, const float* x, const void* 
  * implicit GEMM (and split reduce) reading it (_nax_conv.py:200-332).  A
  * packed input may be reused by several _gemm calls with the same desc.
  * For a 1x1x1 fp32 conv with cin % 16 == 0 and no affine/SiLU nothing is
- * packed and _gemm reads x directly; for the LDS-staged GEMM _pack only keeps
- * the affine table in `workspace` and _gemm reads x directly.
+ * packed and _gemm reads x directly; for the LDS-staged GEMM and the
+ * plane-by-plane form of 8 input channels _pack only keeps the affine table in
+ * `workspace` and _gemm reads x directly.
  */
 int ctmr_conv3d_pack(const ctmr_conv_desc* desc, const float* x, const float* affine,
                      void* workspace, size_t workspace_bytes, void* stream);

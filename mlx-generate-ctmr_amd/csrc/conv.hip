@@ -1629,7 +1629,8 @@ __global__ __launch_bounds__(256, 2) void conv_small_cout_kernel(SmallOutArgs p)
 
 // ---------------------------------------------------------------------------
 // 3b'. LDS-staged im2col GEMM for small channel counts (fp32, stride 1, cin 4
-// or 8: the 4-channel latent input convs, the 8-channel label-condition convs)
+// or 8: the 4-channel latent input convs; 8 -> 8 up to about 2^18 outputs, the
+// larger ones run on conv_march_kernel)
 // ---------------------------------------------------------------------------
 // The im2col formulation (K = tap * cin + c, blocks of 16, the packed weight of
 // WL_IM2COL) without its HBM rows: a workgroup stages the brick's 6x10x10 halo
@@ -2685,6 +2686,8 @@ struct Geometry {
   int wsets;             // its K ranges as wave sets of one workgroup (2: a split of 2 without partial planes)
   bool lds16;            // LDS-staged bf16 GEMM over the packed copy (conv_lds_bf16_kernel)
   bool small_out;        // direct cout <= 4 conv from an LDS halo (conv_small_cout_kernel)
+  bool march;            // plane-marching conv of 8 input channels (conv_march_kernel)
+  int run;               // its output depths per tile
   bool lds_small;        // LDS-staged im2col GEMM for cin 4 / 8 (conv_lds_small_kernel)
   bool cat;              // input given as two tensors, channels [0, c1) and [c1, cin)
   int c1;
@@ -2713,6 +2716,21 @@ static int64_t lds_policy_split(int64_t base, int64_t chunks) {
     if (e2 >= e1 + 0.1) return 2;
   }
   return 1;
+}
+
+// Output depths per tile of the plane-marching conv: the run that leaves the
+// fewest planes in series over the rounds of 512 resident workgroups (two per
+// CU), each run staging its planes (one or two beyond its outputs' own) and
+// about one plane's time more for its weights; at least 4 depths.
+static int march_run(int64_t tiles, int od, int stride) {
+  int64_t best = 0;
+  int run = od;
+  for (int chunks = 1; chunks == 1 || ceil_div(od, chunks) >= 4; ++chunks) {
+    const int64_t r = ceil_div(od, chunks);
+    const int64_t cost = ceil_div(tiles * ceil_div(od, r), 512) * (r * stride + 3);
+    if (chunks == 1 || cost < best) best = cost, run = (int)r;
+  }
+  return run;
 }
 
 static int geometry(const ctmr_conv_desc* d, Geometry& g) {
@@ -2826,6 +2844,36 @@ static int geometry(const ctmr_conv_desc* d, Geometry& g) {
   // taken (outputs past that span would be dropped by the buffer range).
   const bool brick_out_fits =
       (int64_t)kBD * (g.phases == 8 ? 2 : 1) * g.oh * g.ow * d->cout * 4 < (1ll << 31);
+  // Plane-marching conv: 8 input channels, fp32, stride 1 to 8 outputs or
+  // stride 2 to 17 .. 32.  Reads x itself.  From about 2^18 outputs at
+  // stride 1 and 2^15 at stride 2, tiles at least half full; a plane of x within
+  // 32-bit offsets.  Measured, brick GEMM (stride 1) or im2col rows and GEMM
+  // (stride 2) against this, us: 8 -> 8 at 32^3 10 / 22, 64^3 24 / 24, 64x72x80
+  // 33 / 25, 96^3 70 / 36, 128^3 151 / 56; 8 -> 32 from 64^3 34 / 24, 96^3 83 /
+  // 25, 128^3 203 / 35.
+  g.march = false;
+  if (g.layout == WL_IM2COL && !g.cat && d->dtype == CTMR_F32 && d->mode == CTMR_MODE_PLAIN && d->cin == 8 &&
+      (d->stride == 1 ? d->cout == 8 : d->cout > 16 && d->cout <= 32 && d->cout % 4 == 0) && d->split <= 1 &&
+      !(d->flags & (CTMR_F_STREAM | CTMR_F_SPLIT_WAVES)) && s_out >= (d->stride == 1 ? 5 << 16 : 1 << 15) &&
+      (int64_t)d->h * d->w * 32 < (1ll << 31)) {
+    const int64_t ty = ceil_div(g.oh, march_rows(d->stride)), tx = ceil_div(g.ow, march_cols(d->stride));
+    const int64_t slots = ty * march_rows(d->stride) * tx * march_cols(d->stride);
+    if (2 * (int64_t)g.oh * g.ow >= slots) {
+      g.march = true;
+      g.pack = false;
+      g.ty = (int)ty; g.tx = (int)tx;
+      g.run = march_run(ty * tx * d->n, g.od, d->stride);
+      g.tz = (int)ceil_div(g.od, g.run);
+      g.m_tiles = g.tz * g.ty * g.tx;
+      g.n_tiles = 1;
+      g.split = 1;
+      g.wsets = 1;
+      g.lds_small = g.lds = g.lds16 = g.small_out = g.direct = g.kws = g.pointwise = false;
+      g.pack_bytes = (d->flags & CTMR_F_AFFINE) ? round_up((int64_t)d->n * d->cin * 2 * 4, 256) : 0;
+      g.part_bytes = 0;
+      return CTMR_OK;
+    }
+  }
   // LDS-staged im2col GEMM: the im2col formulation of stride-1 fp32 convs with
   // 4 or 8 input channels, its rows read from a halo brick in LDS instead of
   // HBM (same K blocks and products: bit-identical outputs); 64-column tiles
@@ -3090,6 +3138,10 @@ static int split_gn_rows(const ctmr_conv_desc* d, const Geometry& g) {
 static int gn_stats_tiles(const ctmr_conv_desc* d, const Geometry& g, int groups) {
   if (groups <= 0 || d->cout % groups != 0) return 0;
   if (g.layout == WL_EXPAND) return 0;
+  if (g.march) {  // the stride-2 form's 32-column tiles
+    const int cpg = d->cout / groups;
+    return d->stride == 2 && 32 % cpg == 0 ? g.m_tiles : 0;
+  }
   if (g.lds_small) {  // 64-column bricks only (the narrow epilogue writes no statistics)
     const int cpg = d->cout / groups;
     return (g.nsub == 4 && cpg <= 64 && 64 % cpg == 0) ? g.tz * g.ty * g.tx : 0;
@@ -3315,7 +3367,7 @@ int ctmr_conv3d_kernel(const ctmr_conv_desc* desc) {
   int rc = geometry(desc, g);
   if (rc) return rc;
   if (g.lds) return CTMR_K_LDS;
-  if (g.lds_small) return CTMR_K_LDS_SMALL;
+  if (g.lds_small || (g.march && desc->stride == 1)) return CTMR_K_LDS_SMALL;
   if (g.lds16) return desc->dtype == CTMR_F16X2 ? CTMR_K_LDS_F16X2 : CTMR_K_LDS_BF16;
   if (g.small_out) return CTMR_K_SMALL_COUT;
   if (g.layout == WL_EXPAND) return CTMR_K_TAP_EXPAND;
@@ -3417,7 +3469,7 @@ static int pack_impl(const ctmr_conv_desc* desc, const float* x, const float* x2
   if (!x || (g.cat && !x2)) return fail(CTMR_E_INVALID, "null input");
   if ((desc->flags & CTMR_F_AFFINE) && !affine) return fail(CTMR_E_INVALID, "affine flag without affine");
   if ((rc = check_workspace(g, workspace, workspace_bytes))) return rc;
-  if (g.lds || g.lds_small || g.small_out) {
+  if (g.lds || g.lds_small || g.small_out || g.march) {
     if (!(desc->flags & CTMR_F_AFFINE)) return CTMR_OK;
     if (hipMemcpyAsync(workspace, affine, (size_t)desc->n * desc->cin * 2 * 4, hipMemcpyDeviceToDevice,
                        (hipStream_t)stream) != hipSuccess)
@@ -3551,7 +3603,7 @@ static int conv3d_gemm_impl(const ctmr_conv_desc* desc, const float* x, const fl
   if ((desc->flags & CTMR_F_BATCH_BIAS) && !bias) return fail(CTMR_E_INVALID, "batch bias flag without bias");
   if ((rc = check_workspace(g, workspace, workspace_bytes))) return rc;
   const char* xp = g.pack ? (const char*)workspace : (const char*)x;
-  if (!g.pack && ((uintptr_t)x & 15) != 0) return fail(CTMR_E_INVALID, "x must be 16-byte aligned");
+  if (!g.pack && !(g.march && desc->stride == 2) && ((uintptr_t)x & 15) != 0) return fail(CTMR_E_INVALID, "x must be 16-byte aligned");
   // The bf16 LDS GEMM and the pointwise GEMM store (and read the residual) 16 bytes at a time.
   const uintptr_t wide = (uintptr_t)y | ((desc->flags & CTMR_F_RESIDUAL) ? (uintptr_t)residual : 0) |
                          (g.split > 1 ? (uintptr_t)workspace : 0);
@@ -3601,6 +3653,26 @@ static int conv3d_gemm_impl(const ctmr_conv_desc* desc, const float* x, const fl
       if ((rc = check_launch("split_reduce"))) return rc;
     }
     return CTMR_OK;
+  }
+  if (g.march) {
+    MarchArgs a;
+    a.x = x;
+    a.affine = (desc->flags & CTMR_F_AFFINE) ? (affine_direct ? affine_direct : (const float*)workspace) : nullptr;
+    a.wp = (const float*)packed;
+    a.bias = bias;
+    a.res = (desc->flags & CTMR_F_RESIDUAL) ? residual : nullptr;
+    a.y = y;
+    a.n = desc->n; a.d = desc->d; a.h = desc->h; a.w = desc->w;
+    a.od = g.od; a.oh = g.oh; a.ow = g.ow;
+    a.cout = desc->cout; a.np = g.np;
+    a.tz = g.tz; a.ty = g.ty; a.tx = g.tx; a.run = g.run;
+    a.affine_on = (desc->flags & CTMR_F_AFFINE) != 0;
+    a.silu_on = (desc->flags & CTMR_F_SILU) != 0;
+    a.batch_bias = (desc->flags & CTMR_F_BATCH_BIAS) != 0;
+    a.stats = stats;
+    a.gn_groups = stats ? groups : 0;
+    launch_conv_march(desc->stride, dim3((unsigned)(g.m_tiles * desc->n)), st, a);
+    return check_launch("conv_march");
   }
   if (g.lds_small) {
     LdsSmallArgs a;
@@ -3798,7 +3870,7 @@ static int conv3d_run(const ctmr_conv_desc* desc, const float* x, const float* x
   int rc = geometry(desc, g);
   if (rc) return rc;
   if (!x || !packed || !y || (g.cat && !x2)) return fail(CTMR_E_INVALID, "null input, weight or output");
-  if (g.lds || g.lds_small || g.small_out) {  // no pack stage: these read x and the caller's affine table directly
+  if (g.lds || g.lds_small || g.small_out || g.march) {  // no pack stage: these read x and the caller's affine table directly
     if ((desc->flags & CTMR_F_AFFINE) && !affine) return fail(CTMR_E_INVALID, "affine flag without affine");
     return conv3d_gemm_impl(desc, x, x2, packed, bias, affine, residual, y, workspace, workspace_bytes, 0,
                             nullptr, stream);
@@ -3839,7 +3911,7 @@ static int conv3d_gn_run(const ctmr_conv_desc* desc, const float* x, const float
     return fail(CTMR_E_INVALID, "null input, weight, output or stats");
   if (gn_stats_tiles(desc, g, groups) == 0)
     return fail(CTMR_E_UNSUPPORTED, "this convolution cannot produce group-norm partials");
-  const bool direct_affine = g.lds || g.lds_small || g.small_out;
+  const bool direct_affine = g.lds || g.lds_small || g.small_out || g.march;
   if (direct_affine) {
     if ((desc->flags & CTMR_F_AFFINE) && !affine) return fail(CTMR_E_INVALID, "affine flag without affine");
   } else if ((rc = pack_impl(desc, x, x2, affine, workspace, workspace_bytes, stream))) {

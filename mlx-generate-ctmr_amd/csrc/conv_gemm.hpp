@@ -100,4 +100,24 @@ struct LdsArgs {
 // transform xf (bit 0 affine, bit 1 SiLU) and `wsets` wave sets a workgroup.
 void launch_conv_lds(int xf, int wsets, dim3 grid, hipStream_t st, const LdsArgs& a);
 
+// The plane-marching conv of 8 input channels (conv_march.hip).
+struct MarchArgs {
+  const float* x;       // unpadded NDHWC input, 8 channels
+  const float* affine;  // (n, 8, 2) or null
+  const float* wp;      // packed im2col weight [kblock][np][16]
+  const float* bias;    // null: none
+  const float* res;     // null: none
+  float* y;
+  int n, d, h, w, od, oh, ow, cout, np;
+  int tz, ty, tx, run;  // output tiles per axis; depths per tile
+  int affine_on, silu_on, batch_bias;
+  double* stats;        // group-norm partials per tile (stride 2) or null
+  int gn_groups;
+};
+
+// Output rows and columns of its workgroup's tile.
+constexpr int march_rows(int stride) { return stride == 1 ? 16 : 8; }
+constexpr int march_cols(int stride) { return stride == 1 ? 32 : 16; }
+void launch_conv_march(int stride, dim3 grid, hipStream_t st, const MarchArgs& a);
+
 }  // namespace ctmr
