@@ -530,6 +530,12 @@ def conv3d(x: Tensor, weight: Tensor, bias: Optional[Tensor], *, padding: int, s
            gn_groups: int = 0) -> Tensor:
     """NDHWC convolution with a Torch ``(O, C, k, k, k)`` weight (``fast_fp32.conv3d_ncdhw``, :133-154);
     ``gn_groups`` as in ``implicit_gemm_conv3d``."""
+    _check_conv_weight(x, weight, padding, stride)
+    return implicit_gemm_conv3d(x, _pack(weight, _lib.MODE_PLAIN, x, stride), bias, cout=int(weight.shape[0]),
+                                ksize=int(weight.shape[2]), stride=stride, gn_groups=gn_groups)
+
+
+def _check_conv_weight(x: Tensor, weight: Tensor, padding: int, stride: int) -> None:
     k = int(weight.shape[2])
     if tuple(weight.shape[2:]) != (k, k, k) or (k, padding) not in ((3, 1), (1, 0)):
         raise ValueError(f"supported kernels: 3x3x3 padding 1 and 1x1x1 padding 0; got k={k}, padding={padding}")
@@ -537,8 +543,20 @@ def conv3d(x: Tensor, weight: Tensor, bias: Optional[Tensor], *, padding: int, s
         raise ValueError("1x1x1 convolution supports only stride 1")
     if int(weight.shape[1]) != int(x.shape[-1]):
         raise ValueError(f"weight expects {int(weight.shape[1])} input channels; x has {int(x.shape[-1])}")
-    return implicit_gemm_conv3d(x, _pack(weight, _lib.MODE_PLAIN, x, stride), bias, cout=int(weight.shape[0]),
-                                ksize=k, stride=stride, gn_groups=gn_groups)
+
+
+def _silu_conv3d(x: Tensor, weight: Tensor, bias: Optional[Tensor], *, stride: int = 1) -> Tensor:
+    """``conv3d(silu(x), weight, bias, padding=1, stride=stride)`` of a 3x3x3 weight, same bits.  The SiLU
+    joins the pass that packs or stages the input; only where the plain conv streams ``x`` itself, and a
+    SiLU would make it pack a copy first, does it stay a pass of its own (a pass either way)."""
+    _check_conv_weight(x, weight, 1, stride)
+    packed = _pack(weight, _lib.MODE_PLAIN, x, stride)
+    cout, code = int(weight.shape[0]), _PACKED_DTYPES[packed.dtype]
+    plain, fused = (_lib.workspace_bytes(ops.make_desc(tuple(x.shape), cout, 3, stride, _lib.MODE_PLAIN, flags, code, 0))
+                    for flags in (0, _lib.F_SILU))
+    if fused > plain:
+        return conv3d(silu(x), weight, bias, padding=1, stride=stride)
+    return implicit_gemm_conv3d(x, packed, bias, cout=cout, stride=stride, silu=True)
 
 
 def pointwise_conv(x: Tensor, weight: Tensor, bias: Optional[Tensor]) -> Tensor:

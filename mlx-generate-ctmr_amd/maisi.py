@@ -413,15 +413,15 @@ def encode_controlnet_condition(cond: Tensor, weights: Mapping[str, Tensor], *, 
     if any(int(s) % scale for s in cond.shape[1:4]):
         raise ValueError(f"controlnet cond spatial sizes must be multiples of {scale}")
     p = "controlnet_cond_embedding"
-    hidden = ff.silu(ff.conv3d(cond, weights[f"{p}.conv_in.conv.weight"], weights[f"{p}.conv_in.conv.bias"], padding=1))
+    hidden = ff.conv3d(cond, weights[f"{p}.conv_in.conv.weight"], weights[f"{p}.conv_in.conv.bias"], padding=1)
     block = 0
     for _ in range(len(channels) - 1):
-        for stride in (1, 2):
-            hidden = ff.silu(ff.conv3d(hidden, _need(weights, f"{p}.blocks.{block}.conv.weight"),
-                                       _need(weights, f"{p}.blocks.{block}.conv.bias"), padding=1, stride=stride))
+        for stride in (1, 2):  # each conv applies the SiLU of the one before it
+            hidden = ff._silu_conv3d(hidden, _need(weights, f"{p}.blocks.{block}.conv.weight"),
+                                     _need(weights, f"{p}.blocks.{block}.conv.bias"), stride=stride)
             block += 1
-    return ff.conv3d(hidden, _need(weights, f"{p}.conv_out.conv.weight"), _need(weights, f"{p}.conv_out.conv.bias"),
-                     padding=1)
+    return ff._silu_conv3d(hidden, _need(weights, f"{p}.conv_out.conv.weight"),
+                           _need(weights, f"{p}.conv_out.conv.bias"))
 
 
 def _zero_conv(x: Tensor, weights: Mapping[str, Tensor], prefix: str) -> Tensor:
