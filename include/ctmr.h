@@ -187,8 +187,8 @@ int ctmr_pack_upsample_weight(const ctmr_conv_desc* desc, const float* weight, v
  * visits taps kd*9+kh*3+kw ascending (outer) and input channels in ascending
  * 16-wide (fp32) / 32-wide (bf16) blocks (inner).  The LDS-staged GEMM, chosen
  * by shape for large stride-1 fp32 volumes (cin >= 64 and a multiple of 16,
- * cout % 64 == 0, no resampling, CTMR_F_STREAM not set), stages 16-channel chunks of the input
- * with their halo (affine + SiLU and zero padding applied while staging) and
+ * cout % 64 == 0, or cin >= 32 with 32 outputs; no resampling, CTMR_F_STREAM
+ * not set), stages 16-channel chunks of the input with their halo (affine + SiLU and zero padding applied while staging) and
  * visits chunks ascending (outer), taps ascending (inner).  The LDS-staged
  * bf16 GEMM, chosen for stride-1 bf16 convs (plain, trilinear-2x, or
  * nearest-2x as the eight parity GEMMs of the fold) with cout % 64 == 0 and

@@ -2937,7 +2937,9 @@ static int geometry(const ctmr_conv_desc* d, Geometry& g) {
     }
   }
   // LDS-staged GEMM: stride-1 fp32 volumes with at least 64 input channels,
-  // 64-wide column tiles and 6 staged planes within 32-bit buffer offsets,
+  // 64-wide column tiles (or 32 outputs of at least 32 channels, unsplit:
+  // streaming / LDS us at 32 -> 32 channels 128x128x64 521 / 302, 96^3 437 / 253,
+  // 64x64x32 74 / 45, 50x70x61 128 / 76) and 6 staged planes within 32-bit buffer offsets,
   // whose 4x8x8 bricks are at least 3/4 full, or 0.6 full with the grid's
   // last round of 512 workgroups not too empty (0.8 of the rounds' slots
   // taken).  Measured, streaming / LDS us: 49x49x33 (0.68 full) 64 channels
@@ -2949,8 +2951,10 @@ static int geometry(const ctmr_conv_desc* d, Geometry& g) {
   g.lds16 = false;
   g.small_out = false;
   if (g.layout == WL_TAPS && d->dtype == CTMR_F32 && d->ksize == 3 && d->stride == 1 &&
-      d->mode == CTMR_MODE_PLAIN && d->cin % 16 == 0 && d->cin >= 64 && d->cout % 64 == 0 &&
+      d->mode == CTMR_MODE_PLAIN && d->cin % 16 == 0 &&
+      ((d->cin >= 64 && d->cout % 64 == 0) || (d->cin >= 32 && d->cout == 32 && !g.cat && d->split <= 1)) &&
       !(d->flags & (CTMR_F_STREAM | CTMR_F_SPLIT_WAVES))) {
+    const bool narrow = d->cout == 32;
     g.tz = (int)ceil_div(d->d, kBD);
     g.ty = (int)ceil_div(d->h, kBH);
     g.tx = (int)ceil_div(d->w, kBW);
@@ -2961,14 +2965,14 @@ static int geometry(const ctmr_conv_desc* d, Geometry& g) {
     // 20^3 x 2, 128 channels, split waves 112 us, LDS in 3 ranges 140), or 2
     // chunks where it is two wave sets of one workgroup: 60x44x28, 64 channels
     // 146 / 134 us.
-    const int64_t base = (int64_t)g.tz * g.ty * g.tx * (d->cout / 64) * d->n;
+    const int64_t base = (int64_t)g.tz * g.ty * g.tx * ceil_div(d->cout, 64) * d->n;
     const int64_t policy_split = lds_policy_split(base, d->cin / 16);
     const int64_t split = d->split > 0 ? d->split : policy_split;
     const int64_t chunks = d->cin / 16, range = chunks / split;
     const bool full = 4 * S >= 3 * slots || (5 * S >= 3 * slots &&
                                              5 * base * split >= 4 * 512 * ceil_div(base * split, 512));
     if (full && planes < (1ll << 31) && brick_out_fits &&
-        (range >= 4 || (split == 2 && chunks % 2 == 0 && range >= 2))) g.lds = true;
+        (narrow ? split == 1 : range >= 4 || (split == 2 && chunks % 2 == 0 && range >= 2))) g.lds = true;
   }
   if (g.lds) {
     g.pack = false;
@@ -2976,7 +2980,7 @@ static int geometry(const ctmr_conv_desc* d, Geometry& g) {
     g.kblocks = d->cin / 16;
     g.nsub = 4; g.wm = 4; g.wn = 1;
     g.m_tiles = g.tz * g.ty * g.tx;
-    g.n_tiles = d->cout / 64;
+    g.n_tiles = (int)ceil_div(d->cout, 64);
     const int chunks = g.kblocks;
     if (d->split > 0) {
       if (d->split > chunks) return fail(CTMR_E_INVALID, "split must not exceed the 16-channel chunk count");
@@ -3153,7 +3157,7 @@ static int gn_stats_tiles(const ctmr_conv_desc* d, const Geometry& g, int groups
     const int64_t chunks = (s_out + per - 1) / per;
     return chunks > 65535 ? 0 : (int)chunks;
   }
-  const int width = g.lds ? 64 : g.wn * g.nsub * 16;
+  const int width = g.lds ? std::min(64, d->cout) : g.wn * g.nsub * 16;
   if (cpg > width || width % cpg != 0) return 0;
   return (g.lds || g.lds16) ? g.tz * g.ty * g.tx * g.phases : g.m_tiles * g.phases;
 }

@@ -38,7 +38,9 @@ namespace ctmr {
 // Measured against the same tiling on FP32 MFMA: 128 -> 128 channels at 128^3
 // with the norm and SiLU 13.0 -> 7.73 ms (240 TFLOP/s: 1440 in bf16 products,
 // MFMA busy 81 % at the 1.65 GHz the power limit leaves), 64 -> 64 at 64^3 404
-// -> 268 us (MFMA busy 70 %), no bank conflicts; distance from 64 bits over
+// -> 268 us (MFMA busy 70 %), no bank conflicts; one 32-column block, 32 -> 32 at
+// 128 x 128 x 64, 302 us (192 TFLOP/s; a tap reads nine operands for six products,
+// twelve for twelve with two blocks); distance from 64 bits over
 // residual blocks 4.5e-7 .. 7.0e-7 -> 3.9e-7 .. 6.0e-7.
 constexpr int kX3Row = 96;                                // a staged voxel or weight column
 constexpr int kX3Halo = kHaloVox * kX3Row;                // 57600
@@ -55,8 +57,8 @@ __device__ __forceinline__ int brick32_line(int r) { return ((r >> 3) & 1) * 4 +
 // columns n0 + nb*32 + 8*q + 4*(l/32) + r in element 4*q + r.  Group-norm
 // column sums: per lane over mb, then the 16-lane rows (row16_sum), whose
 // eight partials per column (two per wave) combine in ascending order.
-template <typename Args, typename AfterBias = NoTerm>
-__device__ __forceinline__ void store_brick32(const Args& p, f16v (&acc)[2][2], int b, int split_id, int z0, int y0,
+template <int NB, typename Args, typename AfterBias = NoTerm>
+__device__ __forceinline__ void store_brick32(const Args& p, f16v (&acc)[2][NB], int b, int split_id, int z0, int y0,
                                               int x0, int n0, int wave, int lane, int tile_id,
                                               double (*red)[64][2], AfterBias after_bias = {}) {
   const int r32 = lane & 31, half = lane >> 5;
@@ -75,7 +77,7 @@ __device__ __forceinline__ void store_brick32(const Args& p, f16v (&acc)[2][2], 
   if (!partial && p.has_bias) {
     const float* bias_b = p.bias + (p.batch_bias ? (int64_t)b * p.cout : 0) + n0 + 4 * half;
 #pragma unroll
-    for (int nb = 0; nb < 2; ++nb)
+    for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const float bq = bias_b[nb * 32 + 8 * (i >> 2) + (i & 3)];
@@ -85,18 +87,18 @@ __device__ __forceinline__ void store_brick32(const Args& p, f16v (&acc)[2][2], 
   }
   after_bias(acc);
   if (!partial && p.has_res) {  // every residual load before the first store
-    f4 rq[2][2][4];
+    f4 rq[2][NB][4];
 #pragma unroll
     for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
-      for (int nb = 0; nb < 2; ++nb)
+      for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
         for (int q = 0; q < 4; ++q)
           rq[mb][nb][q] = *reinterpret_cast<const f4*>(p.res + base[mb] + nb * 32 + 8 * q);
 #pragma unroll
     for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
-      for (int nb = 0; nb < 2; ++nb)
+      for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[mb][nb][i] += rq[mb][nb][i >> 2][i & 3];
   }
@@ -109,7 +111,7 @@ __device__ __forceinline__ void store_brick32(const Args& p, f16v (&acc)[2][2], 
 #pragma unroll
     for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
-      for (int nb = 0; nb < 2; ++nb)
+      for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
         for (int q = 0; q < 4; ++q)
           if (row_ok[mb]) {
@@ -122,7 +124,7 @@ __device__ __forceinline__ void store_brick32(const Args& p, f16v (&acc)[2][2], 
   if (p.stats) {  // a kernel argument: every thread reaches the barriers
     __syncthreads();
 #pragma unroll
-    for (int nb = 0; nb < 2; ++nb)
+    for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const double d0 = row_ok[0] ? (double)acc[0][nb][i] : 0.0, d1 = row_ok[1] ? (double)acc[1][nb][i] : 0.0;
@@ -134,7 +136,7 @@ __device__ __forceinline__ void store_brick32(const Args& p, f16v (&acc)[2][2], 
         }
       }
     __syncthreads();
-    combine_gn_partials<4, 8, 1>(red, n0, p.cout, p.gn_cpg, p.gn_groups,
+    combine_gn_partials<2 * NB, 8, 1>(red, n0, p.cout, p.gn_cpg, p.gn_groups,
                                  p.stats + ((int64_t)b * p.tz * p.ty * p.tx + tile_id) * p.gn_groups * 2);
   }
 }
@@ -145,18 +147,18 @@ __device__ __forceinline__ void store_brick32(const Args& p, f16v (&acc)[2][2], 
 // convolution's.  Reached by volumes that hold an infinity, a NaN or values
 // near the fp32 limit.  `buf`: the wave's 16 KiB of LDS (no wave reads the
 // staged operands any more), so the results can be walked in a loop.
-template <int XF>
-__device__ __forceinline__ void x3_recompute(const LdsArgs& p, f16v (&acc)[2][2], f16v* buf, int b, int z, int y0,
+template <int XF, int NB>
+__device__ __forceinline__ void x3_recompute(const LdsArgs& p, f16v (&acc)[2][NB], f16v* buf, int b, int z, int y0,
                                              int x0, int n0, int lane, int c_begin, int c_end) {
   const int r32 = lane & 31, half = lane >> 5, x = x0 + (r32 & 7);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) buf[i * 64 + lane] = acc[i >> 1][i & 1];
+  for (int i = 0; i < 2 * NB; ++i) buf[i * 64 + lane] = acc[i / NB][i % NB];
 #pragma clang loop unroll(disable)
-  for (int e = 0; e < 64; ++e) {
+  for (int e = 0; e < 32 * NB; ++e) {
     float* const slot = reinterpret_cast<float*>(buf + (e >> 4) * 64 + lane) + (e & 15);
-    const int y = y0 + (e >> 5) + brick32_line(r32);
+    const int y = y0 + e / (16 * NB) + brick32_line(r32);
     if (fabsf(*slot) < INFINITY || z >= p.d || y >= p.h || x >= p.w) continue;
-    const int col = n0 + ((e >> 4) & 1) * 32 + 8 * ((e >> 2) & 3) + 4 * half + (e & 3);
+    const int col = n0 + (e >> 4) % NB * 32 + 8 * ((e >> 2) & 3) + 4 * half + (e & 3);
     float s = 0.f;
 #pragma clang loop unroll(disable)
     for (int ch = c_begin * 16; ch < c_end * 16; ++ch) {
@@ -184,7 +186,7 @@ __device__ __forceinline__ void x3_recompute(const LdsArgs& p, f16v (&acc)[2][2]
     *slot = s;
   }
 #pragma unroll
-  for (int i = 0; i < 4; ++i) acc[i >> 1][i & 1] = buf[i * 64 + lane];
+  for (int i = 0; i < 2 * NB; ++i) acc[i / NB][i % NB] = buf[i * 64 + lane];
 }
 
 // TWO: the input is two tensors (ctmr_conv3d_cat); the one-tensor kernel keeps
@@ -195,8 +197,9 @@ __device__ __forceinline__ void x3_recompute(const LdsArgs& p, f16v (&acc)[2][2]
 // with its own halo and weight slots) runs the chunks of range s of one brick,
 // and set 0 adds set 1's sums after the bias, the order of the split reduction
 // (bias, range 0, range 1, residual), with no partial planes in memory; both
-// sets run the same chunk count, so every barrier is the workgroup's.
-template <bool TWO, int XF, int WS>
+// sets run the same chunk count, so every barrier is the workgroup's.  NB: 32-
+// column blocks a workgroup computes, two, or one for 32 outputs.
+template <bool TWO, int XF, int WS, int NB = 2>
 __global__ __launch_bounds__(256 * WS, WS == 1 ? 2 : 1) void conv_lds_kernel(LdsArgs p) {
   static_assert(WS == 1 || WS == 2, "one or two wave sets");
   __shared__ __attribute__((aligned(256))) char lds_sets[WS * kX3Set];
@@ -278,7 +281,7 @@ __global__ __launch_bounds__(256 * WS, WS == 1 ? 2 : 1) void conv_lds_kernel(Lds
   const char* const av[2] = {lds + avox * kX3Row + 16 * (half ^ (r32 >> 4)),
                              lds + avox * kX3Row + 16 * (half ^ (r32 >> 4) ^ 1)};
   // B: this lane's column of column block 0 in slot 0.
-  const int n0 = n_tile * 64;
+  const int n0 = n_tile * 32 * NB;
   const char* const bv = lds + kX3Halo + r32 * kX3Row + 16 * (half ^ (r32 >> 4));
   // Weight split: thread t takes channels 4*(t&3)..+3 of column t>>2.
   char* const bw = lds + kX3Halo + (tid >> 2) * kX3Row + 16 * ((part >> 1) ^ ((tid >> 6) & 1)) + 8 * (part & 1);
@@ -287,11 +290,11 @@ __global__ __launch_bounds__(256 * WS, WS == 1 ? 2 : 1) void conv_lds_kernel(Lds
   const int boff = n0 * 64 + tid * 16;
   const int bchunk = p.np * 64;
 
-  f16v acc[2][2];
+  f16v acc[2][NB];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < NB; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
 
@@ -339,6 +342,7 @@ __global__ __launch_bounds__(256 * WS, WS == 1 ? 2 : 1) void conv_lds_kernel(Lds
     return __builtin_amdgcn_raw_buffer_load_b128(brsrc, boff, so, 0);
   };
   auto put_w = [&](u4 w, char* dst) {
+    if (NB == 1 && tid >= 128) return;  // the columns of a whole block only
     uint2 h, m, l;
     split_bf16x3(__builtin_bit_cast(f4, w), h, m, l);
     *reinterpret_cast<uint2*>(dst) = h;
@@ -352,15 +356,15 @@ __global__ __launch_bounds__(256 * WS, WS == 1 ? 2 : 1) void conv_lds_kernel(Lds
       A[mb] = *reinterpret_cast<const bf8*>(av[((mb + kh) >> 1) & 1] + ((kd * kHH + kh + mb) * kHW + kw) * kX3Row +
                                             pt * 32);
   };
-  auto read_b = [&](bf8 (&B)[2], const char* slot, int pt) {
+  auto read_b = [&](bf8 (&B)[NB], const char* slot, int pt) {
 #pragma unroll
-    for (int n = 0; n < 2; ++n) B[n] = *reinterpret_cast<const bf8*>(slot + n * 32 * kX3Row + pt * 32);
+    for (int n = 0; n < NB; ++n) B[n] = *reinterpret_cast<const bf8*>(slot + n * 32 * kX3Row + pt * 32);
   };
-  auto mma = [&](const bf8 (&A)[2], const bf8 (&B)[2]) {
+  auto mma = [&](const bf8 (&A)[2], const bf8 (&B)[NB]) {
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < NB; ++j)
         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(B[j], A[i], acc[i][j], 0, 0, 0);
   };
 
@@ -389,7 +393,7 @@ __global__ __launch_bounds__(256 * WS, WS == 1 ? 2 : 1) void conv_lds_kernel(Lds
   for (int i = 0; i < 3; ++i) raw[i] = load_w(i + 2, c_begin);
   for (int chunk = c_begin; chunk < c_end; ++chunk) {
     lds_barrier();  // the chunk's halo and the weights of its first two taps are in LDS
-    bf8 Ah[2], Am[2], Al[2], Bh[2], Bm[2], Bl[2];
+    bf8 Ah[2], Am[2], Al[2], Bh[NB], Bm[NB], Bl[NB];
     read_a(Al, 0, 2);
     read_b(Bh, bv + cur, 0);
     read_a(Am, 0, 1);
@@ -448,13 +452,13 @@ __global__ __launch_bounds__(256 * WS, WS == 1 ? 2 : 1) void conv_lds_kernel(Lds
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < NB; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) probe = fmaf(acc[i][j][e], 0.f, probe);
   lds_barrier();
   static_assert(4 * 64 * 256 <= kX3Set, "a set's results fit its staging buffers");
   if (__any(!(probe == 0.f)))
-    x3_recompute<XF>(p, acc, reinterpret_cast<f16v*>(lds) + wave * 256, b, z0 + wave, y0, x0, n0, lane, c_begin, c_end);
+    x3_recompute<XF>(p, acc, reinterpret_cast<f16v*>(lds) + wave * 128 * NB, b, z0 + wave, y0, x0, n0, lane, c_begin, c_end);
 
   // The statistics' reduction buffer and the hand-over below reuse the halos.
   double (*const red)[64][2] = reinterpret_cast<double (*)[64][2]>(lds_sets);
@@ -482,14 +486,14 @@ __global__ __launch_bounds__(256 * WS, WS == 1 ? 2 : 1) void conv_lds_kernel(Lds
 }
 
 // conv_lds_kernel for a staging transform xf (bit 0 affine, bit 1 SiLU).
-template <bool TWO, int WS>
+template <bool TWO, int WS, int NB = 2>
 static void launch_lds(int xf, dim3 grid, hipStream_t st, const LdsArgs& a) {
   const dim3 block(256 * WS);
   switch (xf) {
-    case 0: hipLaunchKernelGGL((conv_lds_kernel<TWO, 0, WS>), grid, block, 0, st, a); break;
-    case 1: hipLaunchKernelGGL((conv_lds_kernel<TWO, 1, WS>), grid, block, 0, st, a); break;
-    case 2: hipLaunchKernelGGL((conv_lds_kernel<TWO, 2, WS>), grid, block, 0, st, a); break;
-    default: hipLaunchKernelGGL((conv_lds_kernel<TWO, 3, WS>), grid, block, 0, st, a); break;
+    case 0: hipLaunchKernelGGL((conv_lds_kernel<TWO, 0, WS, NB>), grid, block, 0, st, a); break;
+    case 1: hipLaunchKernelGGL((conv_lds_kernel<TWO, 1, WS, NB>), grid, block, 0, st, a); break;
+    case 2: hipLaunchKernelGGL((conv_lds_kernel<TWO, 2, WS, NB>), grid, block, 0, st, a); break;
+    default: hipLaunchKernelGGL((conv_lds_kernel<TWO, 3, WS, NB>), grid, block, 0, st, a); break;
   }
 }
 
@@ -500,6 +504,7 @@ void launch_conv_lds(int xf, int wsets, dim3 grid, hipStream_t st, const LdsArgs
     else launch_lds<true, 1>(xf, grid, st, a);
   } else {
     if (wsets == 2) launch_lds<false, 2>(xf, grid, st, a);
+    else if (a.cout == 32) launch_lds<false, 1, 1>(xf, grid, st, a);
     else launch_lds<false, 1>(xf, grid, st, a);
   }
 }

@@ -44,6 +44,8 @@ CASES = [
     ("two sources", (1, 7, 8, 15, 64), 48, 64, 1),
     ("two wave sets", (1, 4, 16, 16, 128), 0, 64, 2),
     ("two sources, partial planes", (1, 4, 8, 8, 128), 112, 64, 3),
+    ("32 outputs", (1, 4, 8, 16, 32), 0, 32, 1),
+    ("32 outputs, ragged bricks, odd chunks", (2, 7, 15, 15, 48), 0, 32, 1),
 ]
 
 
@@ -104,6 +106,29 @@ def test_not_finite_through_the_norm_and_silu(ctmr, dev):
     taint = torch.zeros(1, 4, 8, 8, dtype=torch.bool)
     taint[0, 0:3, 2:5, 2:5] = True
     assert torch.equal(y.isnan().all(-1), taint) and torch.equal(y.isnan().any(-1), taint)
+
+
+@pytest.mark.parametrize("groups", [1, 4, 32])
+def test_statistics_of_32_outputs(ctmr, dev, groups):
+    """The epilogue's group-norm partials of the 32-column form, with bias, residual, affine and SiLU."""
+    f = ctmr.fast_fp32
+    g = torch.Generator().manual_seed(5)
+    x, w = torch.randn(2, 7, 15, 16, 32, generator=g), torch.randn(32, 32, 3, 3, 3, generator=g) * 0.05
+    bias, res = torch.randn(2, 32, generator=g), torch.randn(2, 7, 15, 16, 32, generator=g)
+    affine = torch.stack([torch.rand(2, 32, generator=g) + 0.5, torch.randn(2, 32, generator=g)], dim=-1)
+    a = affine[:, None, None, None]
+    src = torch.nn.functional.silu(x.double() * a[..., 0] + a[..., 1])
+    y = f.implicit_gemm_conv3d(x.to(dev), f.pack_weight(w.to(dev), dtype="fp32"), bias.to(dev), cout=32,
+                               affine=affine.to(dev), silu=True, residual=res.to(dev), split=1, gn_groups=groups)
+    ref = _conv64(src, w) + bias.double().reshape(2, 1, 1, 1, 32) + res.double()
+    # SiLU within 1e-6, bias and residual one rounding each
+    bar = _bar(src, w) + 1e-6 * _conv64(src.abs(), w.abs()) + 2.0 ** -23 * ref.abs()
+    assert bool(((y.cpu().double() - ref).abs() <= bar).all())
+    st = f.conv_output_stats(y, groups).cpu().sum(1)
+    yy = y.cpu().double().reshape(2, -1, groups, 32 // groups)
+    want = torch.stack([yy.sum((1, 3)), (yy * yy).sum((1, 3))], -1)
+    # float64 sums of under 2^16 values in another order
+    assert torch.allclose(st, want, rtol=1e-11, atol=1e-11 * float((yy * yy).sum()))
 
 
 # The register-streaming GEMM (whole pairs of 16-channel blocks; an odd block count stays on FP32 MFMA):
