@@ -31,9 +31,12 @@ namespace ctmr {
 // Bound by HBM and the matrix pipe about equally: 8 -> 8 channels at 256 x 256 x
 // 128 moves 0.54 GB (115 us at a large copy's rate) against 112 us of MFMAs.
 // Measured there with SiLU on the input, against the brick GEMM on FP32 MFMA and
-// a SiLU pass: 695 -> 200 us (the staging's VALU work is not hidden behind the
-// products); 8 -> 32 at stride 2, against im2col rows in memory, 907 -> 130 us.
-// A small volume is a chain of planes of about 3 us per workgroup.
+// a SiLU pass: 695 -> 200 us; 8 -> 32 at stride 2, against im2col rows in memory,
+// 907 -> 130 us.  What is left is latency: a workgroup alone takes about 3 us a
+// plane, 1.5 of them MFMAs, the next plane's loads in flight for one plane only
+// (registers allow no more).  Operands read one step ahead, or the next plane's
+// split set between the products' MFMAs, measured no faster (192 and 203 us
+// against 189 without SiLU).
 // Caller's pointers are 4-byte aligned.
 typedef float f4a4 __attribute__((ext_vector_type(4), aligned(4)));
 constexpr int kMarchVox = 48;
