@@ -1,6 +1,7 @@
 // Implicit-GEMM 3x3x3 / 1x1x1 convolution for MI355X (gfx950) on NDHWC fp32
-// activations, with FP32 MFMA (v_mfma_f32_16x16x4_f32; the brick GEMM of
-// conv_lds.hip multiplies fp32 operands in bf16 parts) or bf16-in /
+// activations: fp32 operands in three bf16 parts on bf16 MFMA (the streaming
+// GEMM here, the brick GEMM of conv_lds.hip, the plane-marching conv of
+// conv_march.hip) or on FP32 MFMA (v_mfma_f32_16x16x4_f32), or bf16-in /
 // fp32-accumulate MFMA (v_mfma_f32_16x16x32_bf16).
 //
 // Dataflow (reference: src/mlx_generate_ctmr/_nax_conv.py:1-35, 475-684):
