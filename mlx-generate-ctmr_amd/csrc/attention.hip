@@ -120,9 +120,9 @@ __device__ __forceinline__ void block_softmax(f4 (&s)[kKeyTiles][QT], float (&m)
 //  * kFp32: q, k, v and P as three bf16 parts h, m, l that together hold an
 //    fp32 value's 24 bits (split_bf16x3), the six part products at or above
 //    2^-17 of the full one on bf16 MFMA (FP32 MFMA runs at a sixteenth of its
-//    rate).  Rows of the output that are not finite are recomputed in plain
-//    fp32 (attention_recompute): the parts of an infinity would meet as
-//    inf - inf or 0 * inf.
+//    rate).  Rows of the output that are not finite are computed again on FP32
+//    MFMA (attention_rerun): the parts of an infinity would meet as inf - inf or
+//    0 * inf.
 //  * kF16x2: the reference's split-fp16 arithmetic (_flash_attention.py:
 //    140-290, 314-317): hi = fp16(x), lo = fp16((x - hi) * 2^11) of q (after
 //    scale * log2(e)), k, v and P, with
@@ -168,29 +168,73 @@ __device__ __forceinline__ f4 mfma_x3(const u4 (&a)[3], const u4 (&b)[3], f4 c) 
   return mfma32<kFp32>(a[0], b[0], c);
 }
 
-// One query's outputs at dims 4g .. 4g+3 and 16+4g .. 16+4g+3 in plain fp32
-// (two passes over the keys).
-__device__ __forceinline__ void attention_recompute(const float* q, const float* k, const float* v, int64_t ldk,
-                                                 int64_t ldv, int lk, int g, float qscale, float* out) {
-  auto score = [&](int key) {
-    float s = 0.f;
-#pragma clang loop unroll(disable)
-    for (int d = 0; d < kHeadDim; ++d) s = fmaf(k[(int64_t)key * ldk + d], q[d] * qscale, s);
-    return s;
+// A wave's 16 queries over all keys as fp32 products on FP32 MFMA
+// (v_mfma_f32_16x16x4_f32), keys and values straight from memory: for waves with
+// an output row that is not finite.  One NaN or infinity among the keys reaches
+// every query of its head, so the cost must stay a few times the finite one.
+// Two passes, the scores' maximum and then the probabilities, so that a score of
+// -inf is a key without weight wherever it stands.  S^T product j takes dims j
+// and 4 + j ... of each lane group g's dims 8g .. 8g + 7, P V product (u, r) the
+// keys 16u + 4g + r.  q: this lane's query row; out: dims 4g + r and 16 + 4g + r.
+template <typename Rows>
+__device__ __forceinline__ void attention_rerun(const AttnArgs& a, const float* q, const float* K, const float* V,
+                                                Rows rows_rsrc, int col, int g, f4 (&out)[2]) {
+  f4 qv[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) qv[i] = *reinterpret_cast<const f4*>(q + 8 * g + 4 * i) * a.qscale;
+  auto scores = [&](int k0, f4 (&s)[kKeyTiles]) {
+    const __amdgpu_buffer_rsrc_t rk = rows_rsrc(K, a.ldk, k0);
+#pragma unroll
+    for (int u = 0; u < kKeyTiles; ++u) {
+      const int row = min(u * 16 + col, a.lk - k0);  // rows past the end: zeros
+      const int off = (int)(((int64_t)row * a.ldk + 8 * g) * 4);
+      f4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const f4 kv = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(rk, off + 16 * i, 0, 0));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[e], qv[i][e], acc, 0, 0, 0);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) s[u][r] = k0 + u * 16 + 4 * g + r < a.lk ? acc[r] : -INFINITY;
+    }
   };
   float m = -INFINITY;
 #pragma clang loop unroll(disable)
-  for (int key = 0; key < lk; ++key) m = fmaxf(m, score(key));
-  float l = 0.f, o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma clang loop unroll(disable)
-  for (int key = 0; key < lk; ++key) {
-    const float p = __builtin_amdgcn_exp2f(score(key) - m);
-    l += p;
+  for (int k0 = 0; k0 < a.lk; k0 += kBlock) {
+    f4 s[kKeyTiles];
+    scores(k0, s);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] = fmaf(p, v[(int64_t)key * ldv + (e >> 2) * 16 + 4 * g + (e & 3)], o[e]);
+    for (int u = 0; u < kKeyTiles; ++u)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) m = fmaxf(m, s[u][r]);
   }
+  m = lane_group_max(m);
+  float l = 0.f;
+  out[0] = out[1] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma clang loop unroll(disable)
+  for (int k0 = 0; k0 < a.lk; k0 += kBlock) {
+    f4 s[kKeyTiles];
+    scores(k0, s);
+    const __amdgpu_buffer_rsrc_t rv = rows_rsrc(V, a.ldv, k0);
 #pragma unroll
-  for (int e = 0; e < 8; ++e) out[(e >> 2) * 16 + 4 * g + (e & 3)] = o[e] / l;
+    for (int u = 0; u < kKeyTiles; ++u)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int key = u * 16 + 4 * g + r;
+        const float pr = k0 + key < a.lk ? __builtin_amdgcn_exp2f(s[u][r] - m) : 0.f;
+        l += pr;
+        const int off = (int)(((int64_t)min(key, a.lk - k0) * a.ldv + col) * 4);
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          out[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+              __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rv, off + 64 * j, 0, 0)), pr, out[j], 0, 0, 0);
+      }
+  }
+  l += __shfl_xor(l, 16);
+  l += __shfl_xor(l, 32);
+#pragma unroll
+  for (int j = 0; j < 2; ++j) out[j] *= 1.0f / l;
 }
 
 // A workgroup of eight waves: KS key parts x (8 / KS) query groups of 16
@@ -209,7 +253,7 @@ __device__ __forceinline__ void attention_recompute(const float* q, const float*
 // block: 58 % of the cycles) and VALU (168 operations: 57 %) together; 32
 // queries a wave halve the reads but leave half the waves: 67, 70; 193, 177 us.
 template <int SCH, int KS>
-__global__ __launch_bounds__(kThreads, 4) void flash_attention_kernel(AttnArgs a) {
+__global__ __launch_bounds__(kThreads, SCH == kFp32 && KS == 1 ? 6 : 4) void flash_attention_kernel(AttnArgs a) {
   static_assert(KS == 1 || KS == 2, "one or two key parts");
   constexpr int QT = kQueryTiles;
   constexpr int kGroups = kWaves / KS, kPartThreads = kThreads / KS;
@@ -452,7 +496,6 @@ __global__ __launch_bounds__(kThreads, 4) void flash_attention_kernel(AttnArgs a
     lt += __shfl_xor(lt, 32);
     const float inv = 1.0f / lt;
     const int query = q0 + t * 16 + col;
-    if (query >= a.lq) continue;
     f4 o[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
@@ -463,16 +506,22 @@ __global__ __launch_bounds__(kThreads, 4) void flash_attention_kernel(AttnArgs a
       }
       o[j] *= inv;
     }
-    float* dst = O + (int64_t)query * a.ldo;
     if constexpr (SCH == kFp32) {
       float probe = 0.f;
 #pragma unroll
       for (int e = 0; e < 8; ++e) probe = fmaf(o[e >> 2][e & 3], 0.f, probe);
-      if (!(probe == 0.f)) {
-        attention_recompute(Q + (int64_t)query * a.ldq, K, V, a.ldk, a.ldv, a.lk, g, a.qscale, dst);
-        continue;
+      const bool bad = !(probe == 0.f);
+      if (__any(bad && query < a.lq)) {
+        f4 again[2];
+        attention_rerun(a, Q + (int64_t)min(query, a.lq - 1) * a.ldq, K, V, rows_rsrc, col, g, again);
+        if (bad) {
+          o[0] = again[0];
+          o[1] = again[1];
+        }
       }
     }
+    if (query >= a.lq) continue;
+    float* dst = O + (int64_t)query * a.ldo;
     *reinterpret_cast<f4*>(dst + 4 * g) = o[0];       // dims 4g .. 4g+3
     *reinterpret_cast<f4*>(dst + 16 + 4 * g) = o[1];  // dims 16 + 4g .. 16 + 4g+3
   }

@@ -1021,7 +1021,7 @@ __device__ __forceinline__ void store_tile(const ConvArgs& p, f4 (&acc)[4][NSUB]
 // channels 2431 / 1627; UNet pass 12.29 -> 11.82 ms.
 template <int DT, int NSUB, int WM, int WN, int KT, int STRIDE, bool UP, bool DIRECT = false, int KWS = 1,
           int SETS = 1, bool X3 = false>
-__global__ __launch_bounds__(256 * SETS, SETS == 1 ? 2 : 1) void conv_kernel(ConvArgs p) {
+__global__ __launch_bounds__(256 * SETS, SETS == 2 ? 1 : X3 && NSUB == 2 && !DIRECT ? 3 : 2) void conv_kernel(ConvArgs p) {
   static_assert(WM * WN * KWS == 4, "four waves per wave set");
   static_assert(SETS == 1 || (SETS == 2 && KWS == 4), "two wave sets only with the four-wave K split");
   static_assert(!DIRECT || (KT == 3 && !UP && DT == CTMR_F32), "direct reads: plain fp32 3x3x3 convs");
@@ -1127,7 +1127,7 @@ __global__ __launch_bounds__(256 * SETS, SETS == 1 ? 2 : 1) void conv_kernel(Con
   // advanced incrementally so a step costs a few scalar adds.
   const int rb = (int)p.row_bytes;
   int c_kb, c_tw, c_th, c_td, c_tapoff, c_bo;
-  {
+  auto seek_begin = [&]() {
     const int tap = s_begin * kStep / p.kb;
     c_kb = s_begin * kStep - tap * p.kb;
     c_tw = tap % KT;
@@ -1135,7 +1135,8 @@ __global__ __launch_bounds__(256 * SETS, SETS == 1 ? 2 : 1) void conv_kernel(Con
     c_td = tap / (KT * KT);
     c_tapoff = (c_td * p.P + c_th * p.Q + c_tw) * rb;
     c_bo = s_begin * bstep;
-  }
+  };
+  seek_begin();
   // DIRECT: the lane offsets of the cursor's tap (recomputed when the tap
   // changes): the real row, or 0x80000000 -- past any buffer range -- where the
   // tap leaves the volume.  A prefetch past the last step may test bits of a
@@ -1247,46 +1248,49 @@ __global__ __launch_bounds__(256 * SETS, SETS == 1 ? 2 : 1) void conv_kernel(Con
         __builtin_amdgcn_sched_barrier(0);
       }
     }
-    // Results that are not finite, again in plain fp32 (x3_recompute's reason),
-    // one per lane and pass; bit e of `bad` is row block e / (4 NSUB), column
-    // block (e / 4) % NSUB, column e % 4 of the lane's four.
-    static_assert(16 * NSUB <= 64, "one bit per result");
-    unsigned long long bad = 0;
+    // The wave's results that are not finite, again on FP32 MFMA (the reason and
+    // the bound on the cost as x3_rerun's in conv_lds.hip), a 16-column block at
+    // a time: product (q, j) takes channel 8g + 4q + j of each lane group g.
+    float probe = 0.f;
 #pragma unroll
-    for (int e = 0; e < 16 * NSUB; ++e)
-      if (!(fabsf(acc[e / (4 * NSUB)][(e / 4) % NSUB][e & 3]) < INFINITY)) bad |= 1ull << e;
-    while (__any(bad != 0)) {
-      if (bad == 0) continue;
-      const int e = __builtin_ctzll(bad);
-      bad &= bad - 1;
-      const int ms = e / (4 * NSUB), ns = (e / 4) % NSUB;
-      const int col = min(n0 + ns * 16 + 4 * lgrp + (e & 3), p.np - 1);
-      const int v = min(m0 + ms * 16 + lrow, S - 1);
-      const int d = v / ghw, r = v - d * ghw, h = r / p.gw, w = r - h * p.gw;
-      const int64_t row = window_row(v);
-      float sum = 0.f;
+    for (int ms = 0; ms < 4; ++ms)
+#pragma unroll
+      for (int ns = 0; ns < NSUB; ++ns)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) probe = fmaf(acc[ms][ns][e], 0.f, probe);
+    if (__any(!(probe == 0.f))) {
 #pragma clang loop unroll(disable)
-      for (int s = s_begin * kStep; s < s_end * kStep; ++s) {
-        const int tap = s / p.kb, kb = s - tap * p.kb;
-        const int td = tap / (KT * KT), th = (tap / KT) % KT, tw = tap % KT;
-        bool in = true;
-        int64_t off;
-        if constexpr (DIRECT) {
-          const int z = STRIDE * d - 1 + td, y = STRIDE * h - 1 + th, x = STRIDE * w - 1 + tw;
-          in = z >= 0 && z < p.in_d && y >= 0 && y < p.in_h && x >= 0 && x < p.in_w;
-          off = ((int64_t)z * p.in_h + y) * p.in_w + x;
-        } else {
-          off = row + (int64_t)td * p.P + (int64_t)th * p.Q + tw;
+      for (int nb = 0; nb < NSUB; ++nb) {
+        const int bo = min(n0 + nb * 16 + lrow, p.np - 1) * 64 + (lgrp >> 1) * p.np * 64 + (lgrp & 1) * 32;
+        f4 sum[4];
+#pragma unroll
+        for (int ms = 0; ms < 4; ++ms) sum[ms] = f4{0.f, 0.f, 0.f, 0.f};
+        seek_begin();
+        direct_offsets();
+#pragma clang loop unroll(disable)
+        for (int s = s_begin; s < s_end; ++s) {
+          u4 w[2];
+          load_a();
+#pragma unroll
+          for (int q = 0; q < 2; ++q) w[q] = __builtin_amdgcn_raw_buffer_load_b128(brsrc, bo + 16 * q, b_step(), 0);
+          advance();
+#pragma unroll
+          for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+              for (int ms = 0; ms < 4; ++ms)
+                sum[ms] = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(f4, w[q])[j],
+                                                               __builtin_bit_cast(f4, A[ms][q])[j], sum[ms], 0, 0, 0);
         }
-        const float* xa = reinterpret_cast<const float*>(
-            p.xp + ((int64_t)b * p.rows_per_batch + (in ? off : 0)) * p.row_bytes + kb * 64);
-        const float* wb = reinterpret_cast<const float*>(p.wp + bbase_off + ((int64_t)s * p.np + col) * 64);
-#pragma clang loop unroll(disable)
-        for (int c = 0; c < 16; ++c) sum = fmaf(in ? xa[c] : 0.f, wb[c], sum);
-      }
 #pragma unroll
-      for (int k = 0; k < 16 * NSUB; ++k)
-        if (k == e) acc[k / (4 * NSUB)][(k / 4) % NSUB][k & 3] = sum;
+        for (int ns = 0; ns < NSUB; ++ns)
+#pragma unroll
+          for (int ms = 0; ms < 4; ++ms)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (ns == nb && !(fabsf(acc[ms][ns][e]) < INFINITY)) acc[ms][ns][e] = sum[ms][e];
+      }
     }
   } else {
     u4 A0[4], B0[NSUB], A1[4], B1[NSUB];

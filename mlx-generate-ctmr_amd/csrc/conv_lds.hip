@@ -23,7 +23,7 @@ namespace ctmr {
 // exact in fp32), the dropped ml, lm, ll are below 2^-24 together, and fewer
 // fp32 roundings per sum (one per 16 channels and part product) leave the
 // results closer to 64 bits than FP32 MFMA's.  A result that is not finite
-// is recomputed in plain fp32 (x3_recompute): with an infinity among the
+// is summed again on FP32 MFMA (x3_rerun): with an infinity among the
 // operands the parts would meet as inf - inf or 0 * inf.
 //
 // Bound by the matrix pipe: 24 MFMAs of 32 cycles per wave, tap and chunk
@@ -141,52 +141,81 @@ __device__ __forceinline__ void store_brick32(const Args& p, f16v (&acc)[2][NB],
   }
 }
 
-// Plain fp32 sums of this lane's results that are not finite, over chunks
+// The wave's results that are not finite, again as fp32 products over chunks
 // [c_begin, c_end): a result of the part products is finite exactly when all
 // operands are and no sum overflows, so only these can differ from the fp32
 // convolution's.  Reached by volumes that hold an infinity, a NaN or values
-// near the fp32 limit.  `buf`: the wave's 16 KiB of LDS (no wave reads the
-// staged operands any more), so the results can be walked in a loop.
+// near the fp32 limit, and one of those can reach every output of the layers
+// after it (through a group norm), so the whole tile runs on FP32 MFMA
+// (v_mfma_f32_32x32x2_f32), operands straight from memory: the cost stays a
+// few times the finite one whatever the values.  Lane half h holds channels
+// 8h .. 8h + 7 of a chunk, product j the pair of channels j and 8 + j.
+// `buf`: the wave's 16 KiB of LDS (no wave reads the staged operands any more)
+// keeps the part products' results meanwhile.
 template <int XF, int NB>
-__device__ __forceinline__ void x3_recompute(const LdsArgs& p, f16v (&acc)[2][NB], f16v* buf, int b, int z, int y0,
-                                             int x0, int n0, int lane, int c_begin, int c_end) {
-  const int r32 = lane & 31, half = lane >> 5, x = x0 + (r32 & 7);
+__device__ __forceinline__ void x3_rerun(const LdsArgs& p, f16v (&acc)[2][NB], f16v* buf, int b, int z, int y0,
+                                         int x0, int n0, int lane, int c_begin, int c_end) {
+  const int r32 = lane & 31, half = lane >> 5, x = x0 + (r32 & 7), y = y0 + brick32_line(r32);
 #pragma unroll
-  for (int i = 0; i < 2 * NB; ++i) buf[i * 64 + lane] = acc[i / NB][i % NB];
+  for (int i = 0; i < 2 * NB; ++i) {
+    buf[i * 64 + lane] = acc[i / NB][i % NB];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[i / NB][i % NB][e] = 0.f;
+  }
 #pragma clang loop unroll(disable)
-  for (int e = 0; e < 32 * NB; ++e) {
-    float* const slot = reinterpret_cast<float*>(buf + (e >> 4) * 64 + lane) + (e & 15);
-    const int y = y0 + e / (16 * NB) + brick32_line(r32);
-    if (fabsf(*slot) < INFINITY || z >= p.d || y >= p.h || x >= p.w) continue;
-    const int col = n0 + (e >> 4) % NB * 32 + 8 * ((e >> 2) & 3) + 4 * half + (e & 3);
-    float s = 0.f;
-#pragma clang loop unroll(disable)
-    for (int ch = c_begin * 16; ch < c_end * 16; ++ch) {
-      const bool second = ch >= p.c1;
-      const float* src = second ? p.x2 + (ch - p.c1) : p.x + ch;
-      const int row = second ? p.cin - p.c1 : p.c1;
-      float sc = 1.f, of = 0.f;
-      if constexpr ((XF & 1) != 0) {
-        sc = p.affine[((int64_t)b * p.cin + ch) * 2];
-        of = p.affine[((int64_t)b * p.cin + ch) * 2 + 1];
-      }
-#pragma clang loop unroll(disable)
-      for (int tap = 0; tap < 27; ++tap) {
-        const int gz = z + tap / 9 - 1, gy = y + (tap / 3) % 3 - 1, gx = x + tap % 3 - 1;
-        float v = 0.f;
-        if (gz >= 0 && gz < p.d && gy >= 0 && gy < p.h && gx >= 0 && gx < p.w) {
-          v = src[((((int64_t)b * p.d + gz) * p.h + gy) * p.w + gx) * row];
-          if constexpr ((XF & 1) != 0) v = fmaf(v, sc, of);
-          if constexpr ((XF & 2) != 0) v = silu_f(v);
-        }
-        s = fmaf(v, reinterpret_cast<const float*>(p.wp)[(((int64_t)tap * p.kb + (ch >> 4)) * p.np + col) * 16 +
-                                                         (ch & 15)], s);
+  for (int chunk = c_begin; chunk < c_end; ++chunk) {
+    const bool second = chunk * 16 >= p.c1;
+    const int row = second ? p.cin - p.c1 : p.c1;
+    const float* src = (second ? p.x2 + (chunk * 16 - p.c1) : p.x + chunk * 16) + 8 * half;
+    float sc[8], of[8];
+    if constexpr ((XF & 1) != 0) {
+      const float* a = p.affine + ((int64_t)b * p.cin + chunk * 16 + 8 * half) * 2;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        sc[j] = a[2 * j];
+        of[j] = a[2 * j + 1];
       }
     }
-    *slot = s;
+#pragma clang loop unroll(disable)
+    for (int tap = 0; tap < 27; ++tap) {
+      const int gz = z + tap / 9 - 1, gx = x + tap % 3 - 1;
+      f4a4 A[2][2], B[NB][2];
+      bool in[2];
+#pragma unroll
+      for (int mb = 0; mb < 2; ++mb) {
+        const int gy = y + mb + (tap / 3) % 3 - 1;
+        in[mb] = gz >= 0 && gz < p.d && gy >= 0 && gy < p.h && gx >= 0 && gx < p.w;
+        const int64_t vox = in[mb] ? (((int64_t)b * p.d + gz) * p.h + gy) * p.w + gx : 0;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) A[mb][q] = *reinterpret_cast<const f4a4*>(src + vox * row + 4 * q);
+      }
+      const float* wb = reinterpret_cast<const float*>(p.wp) +
+                        (((int64_t)tap * p.kb + chunk) * p.np + n0 + r32) * 16 + 8 * half;
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) B[nb][q] = *reinterpret_cast<const f4a4*>(wb + nb * 32 * 16 + 4 * q);
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int mb = 0; mb < 2; ++mb) {
+          float v = A[mb][j >> 2][j & 3];
+          if constexpr ((XF & 1) != 0) v = fmaf(v, sc[j], of[j]);
+          if constexpr ((XF & 2) != 0) v = silu_f(v);
+          v = in[mb] ? v : 0.f;
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb)
+            acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(B[nb][j >> 2][j & 3], v, acc[mb][nb], 0, 0, 0);
+        }
+    }
   }
 #pragma unroll
-  for (int i = 0; i < 2 * NB; ++i) acc[i / NB][i % NB] = buf[i * 64 + lane];
+  for (int i = 0; i < 2 * NB; ++i) {
+    const f16v was = buf[i * 64 + lane];
+#pragma unroll
+    for (int e = 0; e < 16; ++e)
+      if (fabsf(was[e]) < INFINITY) acc[i / NB][i % NB][e] = was[e];
+  }
 }
 
 // TWO: the input is two tensors (ctmr_conv3d_cat); the one-tensor kernel keeps
@@ -458,7 +487,7 @@ __global__ __launch_bounds__(256 * WS, WS == 1 ? 2 : 1) void conv_lds_kernel(Lds
   lds_barrier();
   static_assert(4 * 64 * 256 <= kX3Set, "a set's results fit its staging buffers");
   if (__any(!(probe == 0.f)))
-    x3_recompute<XF>(p, acc, reinterpret_cast<f16v*>(lds) + wave * 128 * NB, b, z0 + wave, y0, x0, n0, lane, c_begin, c_end);
+    x3_rerun<XF>(p, acc, reinterpret_cast<f16v*>(lds) + wave * 128 * NB, b, z0 + wave, y0, x0, n0, lane, c_begin, c_end);
 
   // The statistics' reduction buffer and the hand-over below reuse the halos.
   double (*const red)[64][2] = reinterpret_cast<double (*)[64][2]>(lds_sets);

@@ -2,6 +2,8 @@
 // fp32 operands as three bf16 parts on bf16 MFMA.
 #include "conv_gemm.hpp"
 
+#include <type_traits>
+
 namespace ctmr {
 
 // ---------------------------------------------------------------------------
@@ -26,7 +28,7 @@ namespace ctmr {
 // depth tap: kd = 0, 1, 2 add to the sums of the next, this and the previous
 // output plane (stride 2: odd planes kd = 0 and 2, even planes kd = 1).
 // Six part products, summed smallest first in fp32 per (plane, column tap); a
-// result that is not finite is summed again in plain fp32 (march_recompute).
+// result that is not finite is summed again on FP32 MFMA (march_rerun).
 //
 // Bound by HBM and the matrix pipe about equally: 8 -> 8 channels at 256 x 256 x
 // 128 moves 0.54 GB (115 us at a large copy's rate) against 112 us of MFMAs.
@@ -38,7 +40,6 @@ namespace ctmr {
 // split set between the products' MFMAs, measured no faster (192 and 203 us
 // against 189 without SiLU).
 // Caller's pointers are 4-byte aligned.
-typedef float f4a4 __attribute__((ext_vector_type(4), aligned(4)));
 constexpr int kMarchVox = 48;
 constexpr int kMarchPitch = 1792;  // 7 * 256 >= 34 (stride 1) or 33 (stride 2) voxels
 
@@ -52,26 +53,56 @@ struct March {
   static constexpr int kAcc = STRIDE == 1 ? 3 : 2;  // output planes in flight
 };
 
-// Plain fp32 sum of one output: as the GEMM's im2col order, taps outer.
-__device__ __forceinline__ float march_recompute(const MarchArgs& p, int b, int oz, int oy, int ox, int col,
-                                                           int stride) {
-  float s = 0.f;
+// The sums of a wave's four row blocks (layout of `acc`) as fp32 products on
+// FP32 MFMA (v_mfma_f32_16x16x4_f32), operands straight from memory: for a plane
+// with a result that is not finite (x3_rerun's reason and bound on the cost,
+// conv_lds.hip).  Lane group g holds line g of one output row's window (lane
+// group 3 zeros on both sides: a zero weight must not meet an infinity), product
+// j its channel j; stride 1 computes its two output rows one after the other.
+// oy: the output row of block 0; ox: this lane's output column; wbase: the first
+// of the wave's output channels.
+template <int STRIDE>
+__device__ __forceinline__ void march_rerun(const MarchArgs& p, f4 (&sum)[4], int b, int oz, int oy, int ox, int wbase,
+                                            int lrow, int lgrp) {
+  const int wcol = min(STRIDE == 1 ? lrow & 7 : wbase + lrow, p.cout - 1);
 #pragma clang loop unroll(disable)
-  for (int tap = 0; tap < 27; ++tap) {
-    const int z = oz * stride + tap / 9 - 1, y = oy * stride + (tap / 3) % 3 - 1, x = ox * stride + tap % 3 - 1;
-    const bool in = z >= 0 && z < p.d && y >= 0 && y < p.h && x >= 0 && x < p.w;
+  for (int r = 0; r < (STRIDE == 1 ? 2 : 1); ++r) {
+    f4 part[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) part[t] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma clang loop unroll(disable)
-    for (int c = 0; c < 8; ++c) {
-      float v = 0.f;
-      if (in) {
-        v = p.x[((((int64_t)b * p.d + z) * p.h + y) * p.w + x) * 8 + c];
-        if (p.affine_on) v = fmaf(v, p.affine[(b * 8 + c) * 2], p.affine[(b * 8 + c) * 2 + 1]);
-        if (p.silu_on) v = silu_f(v);
+    for (int k = 0; k < 9; ++k) {
+      const int kd = k / 3, kw = k % 3, tap = (kd * 3 + min(lgrp, 2)) * 3 + kw;
+      const f4a4* wp = reinterpret_cast<const f4a4*>(p.wp + ((int64_t)(tap >> 1) * p.np + wcol) * 16 + (tap & 1) * 8);
+      f4 w[2] = {wp[0], wp[1]};
+      const int gz = oz * STRIDE + kd - 1, gx = ox * STRIDE + kw - 1;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int gy = (oy + (STRIDE == 1 ? 2 * t + r : t)) * STRIDE + lgrp - 1;
+        const bool in = lgrp < 3 && gz >= 0 && gz < p.d && gy >= 0 && gy < p.h && gx >= 0 && gx < p.w;
+        const int64_t vox = in ? (((int64_t)b * p.d + gz) * p.h + gy) * p.w + gx : 0;
+        const f4a4* xp = reinterpret_cast<const f4a4*>(p.x + vox * 8);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const f4 v = xp[e];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            float s = v[j];
+            if (p.affine_on) {
+              const float* a = p.affine + (b * 8 + e * 4 + j) * 2;
+              s = fmaf(s, a[0], a[1]);
+            }
+            if (p.silu_on) s = silu_f(s);
+            part[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(lgrp < 3 ? w[e][j] : 0.f, in ? s : 0.f, part[t], 0, 0, 0);
+          }
+        }
       }
-      s = fmaf(v, p.wp[((int64_t)(tap >> 1) * p.np + col) * 16 + (tap & 1) * 8 + c], s);
+    }
+    if (STRIDE == 2 || (lgrp >> 1) == r) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) sum[t] = part[t];
     }
   }
-  return s;
 }
 
 template <int STRIDE>
@@ -91,32 +122,48 @@ __global__ __launch_bounds__(256, 2) void conv_march_kernel(MarchArgs p) {
 
   // Weights: this lane's output column and halo line, all (kd, kw), split.
   // Stride 1: rows of 2 x 8 columns; stride 2: 16 of the outputs by wave parity.
-  const int wrow = STRIDE == 1 ? lrow >> 3 : 0;
-  const int wcol = STRIDE == 1 ? lrow & 7 : (wave & 1) * 16 + lrow;
-  const int kh = lgrp - wrow;
-  const bool w_on = kh >= 0 && kh < 3 && wcol < p.cout;
-  f4 raw[3][3][2];  // every load before the first split: one round of latency
-#pragma unroll
-  for (int t = 0; t < 9; ++t) {
-    const int tap = ((t / 3) * 3 + min(max(kh, 0), 2)) * 3 + t % 3;
-    const f4a4* src = reinterpret_cast<const f4a4*>(p.wp + ((tap >> 1) * p.np + min(wcol, p.cout - 1)) * 16 +
-                                                    (tap & 1) * 8);
-    raw[t / 3][t % 3][0] = src[0];
-    raw[t / 3][t % 3][1] = src[1];
-  }
+  // `first` on: every load before the first split, one round of latency; a kd at
+  // a time otherwise (the rerun's registers).
   u4 W[3][3][3];
+  auto load_weights = [&](int ln, auto first) {
+    const int wrow = STRIDE == 1 ? (ln & 15) >> 3 : 0;
+    const int wcol = STRIDE == 1 ? ln & 7 : (wave & 1) * 16 + (ln & 15);
+    const int kh = (ln >> 4) - wrow;
+    const bool w_on = kh >= 0 && kh < 3 && wcol < p.cout;
+    f4 raw[3][3][2];
+    auto load_kd = [&](int kd) {
 #pragma unroll
-  for (int kd = 0; kd < 3; ++kd)
+      for (int kw = 0; kw < 3; ++kw) {
+        const int tap = (kd * 3 + min(max(kh, 0), 2)) * 3 + kw;
+        const f4a4* src = reinterpret_cast<const f4a4*>(p.wp + ((tap >> 1) * p.np + min(wcol, p.cout - 1)) * 16 +
+                                                        (tap & 1) * 8);
+        raw[kd][kw][0] = src[0];
+        raw[kd][kw][1] = src[1];
+      }
+    };
+    if constexpr (decltype(first)::value) {
 #pragma unroll
-    for (int kw = 0; kw < 3; ++kw) {
-      const f4 zero = f4{0.f, 0.f, 0.f, 0.f};
-      uint2 h[2], m[2], l[2];
-#pragma unroll
-      for (int e = 0; e < 2; ++e) split_bf16x3(w_on ? raw[kd][kw][e] : zero, h[e], m[e], l[e]);
-      W[kd][kw][0] = u4{h[0].x, h[0].y, h[1].x, h[1].y};
-      W[kd][kw][1] = u4{m[0].x, m[0].y, m[1].x, m[1].y};
-      W[kd][kw][2] = u4{l[0].x, l[0].y, l[1].x, l[1].y};
+      for (int kd = 0; kd < 3; ++kd) load_kd(kd);
     }
+#pragma unroll
+    for (int kd = 0; kd < 3; ++kd) {
+      if constexpr (!decltype(first)::value) {
+        __builtin_amdgcn_sched_barrier(0);
+        load_kd(kd);
+      }
+#pragma unroll
+      for (int kw = 0; kw < 3; ++kw) {
+        const f4 zero = f4{0.f, 0.f, 0.f, 0.f};
+        uint2 h[2], m[2], l[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) split_bf16x3(w_on ? raw[kd][kw][e] : zero, h[e], m[e], l[e]);
+        W[kd][kw][0] = u4{h[0].x, h[0].y, h[1].x, h[1].y};
+        W[kd][kw][1] = u4{m[0].x, m[0].y, m[1].x, m[1].y};
+        W[kd][kw][2] = u4{l[0].x, l[0].y, l[1].x, l[1].y};
+      }
+    }
+  };
+  load_weights(lane, std::true_type{});
 
   // Staging: thread t holds halo voxels t + 256 i; offsets within a plane (the
   // host checks a plane spans under 2 GiB), -1 outside the volume.
@@ -224,21 +271,34 @@ __global__ __launch_bounds__(256, 2) void conv_march_kernel(MarchArgs p) {
   }
   double s1[4] = {0.0, 0.0, 0.0, 0.0}, s2[4] = {0.0, 0.0, 0.0, 0.0};
   auto store = [&](f4 (&sum)[4], int oz) {
+    float probe = 0.f;  // not finite: a NaN or an infinity among the results to be stored
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int oy = y0 + orow + (STRIDE == 1 ? 2 * t : t);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (oy < p.oh && ox < p.ow && ocol < p.cout) probe = fmaf(sum[t][j], 0.f, probe);
+    }
+    if (__any(!(probe == 0.f))) {
+      // The weights are loaded again afterwards, and the lane's indices are
+      // opaque copies: neither then holds registers in the loop or in here.
+      int ln = threadIdx.x & 63;
+      asm volatile("" : "+v"(ln));
+      f4 again[4];
+      march_rerun<STRIDE>(p, again, b, oz, y0 + (STRIDE == 1 ? 8 : 4) * (wave >> 1),
+                          x0 + (STRIDE == 1 ? (wave & 1) * 16 : 0) + (ln & 15), (wave & 1) * 16, ln & 15, ln >> 4);
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (!(fabsf(sum[t][j]) < INFINITY)) sum[t][j] = again[t][j];
+      load_weights(ln, std::false_type{});
+    }
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const int oy = y0 + orow + (STRIDE == 1 ? 2 * t : t);
       if (oy >= p.oh || ox >= p.ow || ocol >= p.cout) continue;
       f4 v = sum[t];
-      if (!(fabsf(v[0]) < INFINITY && fabsf(v[1]) < INFINITY && fabsf(v[2]) < INFINITY && fabsf(v[3]) < INFINITY)) {
-#pragma clang loop unroll(disable)
-        for (int j = 0; j < 4; ++j) {
-          const float r = march_recompute(p, b, oz, oy, ox, ocol + j, STRIDE);
-          v[0] = j == 0 ? r : v[0];
-          v[1] = j == 1 ? r : v[1];
-          v[2] = j == 2 ? r : v[2];
-          v[3] = j == 3 ? r : v[3];
-        }
-      }
       v += bias;
       const int64_t at = ((((int64_t)b * p.od + oz) * p.oh + oy) * p.ow + ox) * p.cout + ocol;
       if (p.res) v += *reinterpret_cast<const f4a4*>(p.res + at);

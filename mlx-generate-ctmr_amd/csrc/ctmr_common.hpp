@@ -14,6 +14,7 @@
 namespace ctmr {
 
 typedef float f4 __attribute__((ext_vector_type(4)));
+typedef float f4a4 __attribute__((ext_vector_type(4), aligned(4)));  // in memory at any 4-byte address
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
