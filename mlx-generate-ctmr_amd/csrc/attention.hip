@@ -291,31 +291,37 @@ __global__ __launch_bounds__(kThreads, SCH == kFp32 && KS == 1 ? 6 : 4) void fla
   // (u = i / 128, g' = (i / 32) % 4: P^T's k slot 8 g + 4 u + r is key 16 u +
   // 4 g + r).
   const int st = threadIdx.x % kPartThreads;
-  int goff[KS], loff[KS];
+  // Rows past lk take row lk's offset, out of range: where lk < 32 a row of the
+  // block can lie past 2^32 bytes, and its offset must not wrap into the range.
+  unsigned goff[KS];
+  int loff[KS];
 #pragma unroll
   for (int j = 0; j < KS; ++j) {
     const int id = st + j * kPartThreads;
     if (id < 256) {
-      goff[j] = (int)(((int64_t)(id >> 3) * a.ldk + 4 * (id & 7)) * 4);
+      goff[j] = (unsigned)(((int64_t)min(id >> 3, a.lk) * a.ldk + 4 * (id & 7)) * 4);
       loff[j] = (id >> 3) * kRow + 8 * (id & 7);
     } else {
       const int i = id - 256, kq = i >> 5;
-      goff[j] = (int)(((int64_t)(4 * kq) * a.ldv + (i & 31)) * 4);
+      goff[j] = (unsigned)(((int64_t)min(4 * kq, a.lk) * a.ldv + (i & 31)) * 4);
       loff[j] = SCH * kPlane + (i & 31) * kRow + 16 * (kq & 3) + 8 * (kq >> 2);
     }
   }
-  const int vrow = (int)(a.ldv * 4);
+  const unsigned vrow = (unsigned)(a.ldv * 4);
   f4 raw[KS];
   auto fetch = [&](int k0) {
     const __amdgpu_buffer_rsrc_t rk = rows_rsrc(K, a.ldk, k0), rv = rows_rsrc(V, a.ldv, k0);
 #pragma unroll
     for (int j = 0; j < KS; ++j) {
       if (wave_piece_is_k<KS>(wave, j)) {  // wave-uniform
-        raw[j] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(rk, goff[j], 0, 0));
+        raw[j] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(rk, (int)goff[j], 0, 0));
       } else {
+        unsigned off = goff[j];
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          raw[j][r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rv, goff[j] + r * vrow, 0, 0));
+        for (int r = 0; r < 4; ++r) {
+          raw[j][r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rv, (int)off, 0, 0));
+          off = __builtin_elementwise_add_sat(off, vrow);
+        }
       }
     }
   };

@@ -60,3 +60,20 @@ def test_operands_that_are_not_finite(ctmr, dev, lq, lk):
     assert torch.equal(y.isneginf(), ref.isneginf())
     ok = ref.isfinite()
     assert bool(((y.double() - ref).abs()[ok] <= 1e-5).all()) and 64 < int((~ok).sum()) < ok.numel() // 2
+
+
+@pytest.mark.parametrize("precision", ["fp32", "f16x2"])
+def test_rows_a_gigabyte_apart(ctmr, dev, precision):
+    """Rows of a key block past the last key whose byte offset exceeds 2^32: two keys, rows 2^30 - 256 bytes
+    apart, so that row 5's offset wraps to the gap behind row 0.  The gap holds NaN, which no output may show."""
+    f = ctmr.fast_fp32
+    ld = (1 << 28) - 64
+    buf = torch.full((2 * ld,), float("nan"), device=dev)
+    rows = buf.as_strided((1, 2, 64), (2 * ld, ld, 1))
+    g = torch.Generator().manual_seed(3)
+    kv, q = torch.randn(1, 2, 64, generator=g), torch.randn(1, 20, 32, generator=g)
+    rows.copy_(kv)
+    with f.precision(precision):
+        y = f.flash_attention(q.to(dev), rows[..., :32], rows[..., 32:], heads=1, scale=32 ** -0.5)
+    err = (y.cpu().double() - _reference(q, kv[..., :32], kv[..., 32:], 1, 32 ** -0.5)).abs().max().item()
+    assert err <= 2e-6 * kv.abs().max().item(), err
