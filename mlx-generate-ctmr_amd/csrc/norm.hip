@@ -489,13 +489,16 @@ __global__ __launch_bounds__(256) void resample_kernel(int op, int n, int d, int
 //    two transposed copies, statistics, finalize and apply (same bits).
 //  * Longer runs are cut into chunks: one launch writes each chunk's (sum, sum
 //    of squares), the next sums its run's chunk partials -- every workgroup
-//    the same sums in the same order -- and applies its chunk.
+//    the same sums in the same order -- and applies its chunk.  Every workgroup
+//    reads all of its run's partials, so their number is bounded (32 KiB, and
+//    from there on the chunks grow with the run).
 // VEC 4 reads 16 bytes: s % 4 == 0 and 16-byte pointers, so that four values
 // share a channel; otherwise one value at a time.
 constexpr int kPlanarThreads = 1024;
 constexpr int kPlanarVecs = 8;                                     // vectors a thread of the one-launch form holds
 constexpr int kPlanarRun = kPlanarThreads * kPlanarVecs;           // x VEC values: the one-launch form's longest run
-constexpr int kPlanarChunk = 256 * 16;                             // vectors per chunk of the two-launch form
+constexpr int kPlanarChunk = 256 * 16;                             // a chunk of the two-launch form: this many vectors, or a
+constexpr int kPlanarChunks = 2048;                                // multiple of them that leaves at most so many chunks
 constexpr int kPlanarMaxCpg = 1024;
 
 struct PlanarArgs {
@@ -505,6 +508,7 @@ struct PlanarArgs {
   float* y;
   double* part;     // (n * groups, chunks, 2)
   int s, c, groups, cpg, chunks, silu;
+  unsigned chunk;   // vectors per chunk
   float eps;
 };
 
@@ -615,17 +619,16 @@ __global__ __launch_bounds__(256) void gn_planar_partial_kernel(PlanarArgs p) {
   const int run = blockIdx.z * p.groups + blockIdx.y;
   const unsigned vecs = (unsigned)((int64_t)p.s * p.cpg / VEC);
   const float* xr = p.x + (int64_t)run * p.s * p.cpg;
-  const unsigned i0 = blockIdx.x * (unsigned)kPlanarChunk + threadIdx.x;
+  const unsigned c0 = blockIdx.x * p.chunk, c1 = min(c0 + p.chunk, vecs);
   double a = 0.0, b = 0.0;
-#pragma unroll
-  for (int u0 = 0; u0 < kPlanarChunk / 256; u0 += 8) {
+  for (unsigned i0 = c0 + threadIdx.x; i0 < c1; i0 += 8 * 256) {
     PlanarVec<VEC> q[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u)
-      if (i0 + (u0 + u) * 256 < vecs) q[u] = planar_load<VEC>(xr + (int64_t)(i0 + (u0 + u) * 256) * VEC);
+      if (i0 + u * 256 < c1) q[u] = planar_load<VEC>(xr + (int64_t)(i0 + u * 256) * VEC);
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      if (i0 + (u0 + u) * 256 >= vecs) continue;
+      if (i0 + u * 256 >= c1) continue;
 #pragma unroll
       for (int k = 0; k < VEC; ++k) {
         const double d = (double)q[u].v[k];
@@ -657,16 +660,15 @@ __global__ __launch_bounds__(256) void gn_planar_apply_kernel(PlanarArgs p) {
   }
   planar_block_sum<256>(a, b);
   planar_affine<256>(p, blockIdx.y, a, b, aff);
-  const unsigned i0 = blockIdx.x * (unsigned)kPlanarChunk + threadIdx.x;
-#pragma unroll
-  for (int u0 = 0; u0 < kPlanarChunk / 256; u0 += 8) {
+  const unsigned c0 = blockIdx.x * p.chunk, c1 = min(c0 + p.chunk, vecs);
+  for (unsigned i0 = c0 + threadIdx.x; i0 < c1; i0 += 8 * 256) {
     PlanarVec<VEC> q[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u)
-      if (i0 + (u0 + u) * 256 < vecs) q[u] = planar_load<VEC>(p.x + base + (int64_t)(i0 + (u0 + u) * 256) * VEC);
+      if (i0 + u * 256 < c1) q[u] = planar_load<VEC>(p.x + base + (int64_t)(i0 + u * 256) * VEC);
 #pragma unroll
     for (int u = 0; u < 8; ++u)
-      if (i0 + (u0 + u) * 256 < vecs) planar_store<VEC>(p, p.y + base, i0 + (u0 + u) * 256, q[u], aff);
+      if (i0 + u * 256 < c1) planar_store<VEC>(p, p.y + base, i0 + u * 256, q[u], aff);
   }
 }
 
@@ -854,13 +856,18 @@ int ctmr_resample(int32_t op, int32_t n, int32_t d, int32_t h, int32_t w, int32_
   return check_launch("resample");
 }
 
+// Vectors per chunk of a run.
+static int64_t planar_chunk(int64_t vecs) {
+  return kPlanarChunk * ceil_div(vecs, (int64_t)kPlanarChunk * kPlanarChunks);
+}
+
 // Chunks a run is cut into, 1 when one workgroup holds it (workspace-free).
 // The size rule leaves out the alignment, so the workspace depends on the
 // shape only; a run read one value at a time may take more chunks than `vec`
 // ones would, never fewer.
 static int64_t planar_chunks(int64_t s, int32_t cpg, int vec) {
   const int64_t vecs = s * cpg / vec;
-  return vecs <= kPlanarRun ? 1 : ceil_div(vecs, kPlanarChunk);
+  return vecs <= kPlanarRun ? 1 : ceil_div(vecs, planar_chunk(vecs));
 }
 
 static int planar_check(int32_t n, int64_t s, int32_t c, int32_t groups) {
@@ -900,6 +907,7 @@ int ctmr_gn_planar(int32_t n, int64_t s, int32_t c, int32_t groups, float eps, c
   p.groups = groups;
   p.cpg = c / groups;
   p.chunks = (int)planar_chunks(s, p.cpg, vec ? 4 : 1);
+  p.chunk = (unsigned)planar_chunk(s * p.cpg / (vec ? 4 : 1));
   p.silu = silu;
   p.eps = eps;
   hipStream_t st = (hipStream_t)stream;

@@ -164,6 +164,17 @@ def test_invalid_descriptors(ctmr, native_loaded, kw, status, message):
     assert message in L.last_error()
 
 
+def test_planar_group_norm_chunks_are_bounded(native_loaded):
+    """Every workgroup of ``ctmr_gn_planar``'s second launch reads all chunk sums of its run (16 bytes each, sized
+    for single values): at most 2048 of them, however long the run."""
+    size = native_loaded.ctmr_gn_planar_workspace_bytes
+    assert size(1, 2048, 4, 1) == 0  # 8192 values stay in one workgroup
+    assert size(1, 2049, 4, 1) == 3 * 16  # chunks of 4096 values
+    for s, c in ((256**3, 64), (8192, 1024), (8193, 1024)):
+        assert 0 < size(1, s, c, 1) <= 2048 * 16, (s, c)
+    assert size(1, 8192, 1024, 1) == 2048 * 16
+
+
 def test_conv_rejects_null_and_small_workspace_before_launch(ctmr, native_loaded):
     L = ctmr._lib
     d = L.conv_desc(1, 4, 4, 4, 16, 16)

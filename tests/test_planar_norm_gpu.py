@@ -26,6 +26,8 @@ CASES = [
     ("chunked vector run, remainder chunk", 2, 64, 32, (20, 22, 42), True, 0),
     ("one group of every channel, misaligned storage", 1, 48, 1, (12, 12, 12), True, 3),
     ("many channels a group", 1, 1024, 1, (2, 3, 2), True, 0),
+    # past 2048 chunks of 4096 vectors: two of them a chunk, the last chunk in its first
+    ("scalar run of more than 2^23 values", 1, 64, 1, (51, 51, 51), True, 0),
 ]
 
 
