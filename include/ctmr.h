@@ -144,18 +144,17 @@ int ctmr_conv3d_split(const ctmr_conv_desc* desc);
  * (fast_fp32.py:93-99, _nax_conv.py:578-581); tests and tools use it to
  * assert which kernel a shape takes (the choice depends on the desc only). */
 enum ctmr_conv_kernel {
-  CTMR_K_STREAM = 0,        /* register-streaming GEMM over the packed copy (cin 8 at stride 2,
-                               large: x streamed plane by plane) */
+  CTMR_K_STREAM = 0,        /* register-streaming GEMM over the packed copy */
   CTMR_K_STREAM_DIRECT = 1, /* register-streaming GEMM reading x itself */
   CTMR_K_LDS = 2,           /* fp32 LDS-staged GEMM (halo bricks of x, three bf16 parts) */
   CTMR_K_LDS_BF16 = 3,      /* bf16 LDS-staged GEMM over the packed copy */
   CTMR_K_POINTWISE = 4,     /* persistent one-tap GEMM (1x1x1, im2col rows) */
   CTMR_K_SPLIT_WAVES = 5,   /* 64 x 64 tiles, each split range over the four waves */
   CTMR_K_TAP_EXPAND = 6,    /* cout <= 4: 27*cout-column GEMM + tap sum */
-  CTMR_K_LDS_SMALL = 7,     /* cin 4 / 8: im2col rows read from an LDS halo brick (8 -> 8, large:
-                               LDS halo planes) */
+  CTMR_K_LDS_SMALL = 7,     /* cin 4 / 8: im2col rows read from an LDS halo brick */
   CTMR_K_SMALL_COUT = 8,    /* cout <= 4: direct FMA conv from an LDS halo brick */
-  CTMR_K_LDS_F16X2 = 9      /* split-fp16 LDS-staged GEMM over the packed hi/lo copy */
+  CTMR_K_LDS_F16X2 = 9,     /* split-fp16 LDS-staged GEMM over the packed hi/lo copy */
+  CTMR_K_MARCH = 10         /* cin 8, large volumes: x walked plane by plane (three bf16 parts) */
 };
 int ctmr_conv3d_kernel(const ctmr_conv_desc* desc);
 

@@ -21,9 +21,9 @@ MODE_PLAIN, MODE_NEAREST2X, MODE_TRILINEAR2X = 0, 1, 2
 F_AFFINE, F_SILU, F_BATCH_BIAS, F_RESIDUAL, F_STREAM, F_SPLIT_WAVES = 1, 2, 4, 8, 16, 32
 DT_F32, DT_BF16, DT_F16X2 = 0, 1, 2
 (K_STREAM, K_STREAM_DIRECT, K_LDS, K_LDS_BF16, K_POINTWISE, K_SPLIT_WAVES, K_TAP_EXPAND, K_LDS_SMALL,
- K_SMALL_COUT, K_LDS_F16X2) = range(10)
+ K_SMALL_COUT, K_LDS_F16X2, K_MARCH) = range(11)
 KERNEL_NAMES = ("stream", "stream_direct", "lds", "lds_bf16", "pointwise", "split_waves", "tap_expand", "lds_small",
-                "small_cout", "lds_f16x2")
+                "small_cout", "lds_f16x2", "march")
 AVGPOOL2, NEAREST2X, TRILINEAR2X = 0, 1, 2
 ABI_VERSION = 5
 NOALLOC_SCRATCH_BYTES = 256 << 20  # CTMR_NOALLOC_SCRATCH_BYTES

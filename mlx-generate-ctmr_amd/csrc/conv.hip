@@ -3376,7 +3376,8 @@ int ctmr_conv3d_kernel(const ctmr_conv_desc* desc) {
   int rc = geometry(desc, g);
   if (rc) return rc;
   if (g.lds) return CTMR_K_LDS;
-  if (g.lds_small || (g.march && desc->stride == 1)) return CTMR_K_LDS_SMALL;
+  if (g.march) return CTMR_K_MARCH;
+  if (g.lds_small) return CTMR_K_LDS_SMALL;
   if (g.lds16) return desc->dtype == CTMR_F16X2 ? CTMR_K_LDS_F16X2 : CTMR_K_LDS_BF16;
   if (g.small_out) return CTMR_K_SMALL_COUT;
   if (g.layout == WL_EXPAND) return CTMR_K_TAP_EXPAND;

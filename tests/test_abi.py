@@ -332,8 +332,13 @@ def test_conv_group_norm_partial_tiles(ctmr, native_loaded):
     ((2, 64, 64, 32, 64), 4, {"flags": 3 | 8}, "tap_expand"),             # with a residual
     ((1, 20, 64, 64, 64), 1, {"flags": 16}, "tap_expand"),                # CTMR_F_STREAM
     ((2, 64, 64, 32, 4), 64, {}, "lds_small"),                            # conv_in: im2col rows from LDS
-    ((1, 256, 256, 256, 8), 8, {}, "lds_small"),                          # condition encoder 8 -> 8
-    ((1, 256, 256, 256, 8), 32, {"stride": 2}, "stream"),                 # stride 2: im2col rows in HBM
+    ((1, 256, 256, 256, 8), 8, {}, "march"),                              # condition encoder 8 -> 8
+    ((1, 256, 256, 256, 8), 32, {"stride": 2}, "march"),                  # stride 2: 8 -> 32
+    ((1, 80, 64, 64, 8), 8, {}, "march"),                                 # 5 * 2^16 outputs, and one row fewer
+    ((1, 80, 64, 63, 8), 8, {}, "lds_small"),
+    ((1, 64, 64, 64, 8), 32, {"stride": 2}, "march"),                     # 2^15 outputs, and one row fewer
+    ((1, 64, 64, 62, 8), 32, {"stride": 2}, "stream"),                    # im2col rows in HBM
+    ((1, 80, 64, 64, 8), 8, {"flags": 16}, "stream"),                     # CTMR_F_STREAM: the im2col GEMM
     ((2, 64, 64, 32, 4), 64, {"flags": 16}, "stream"),                    # CTMR_F_STREAM: the im2col GEMM
     # brick epilogues store at 32-bit offsets from the brick's first output plane: the brick's output
     # planes (4, or 8 for nearest-2x) must span under 2 GiB; at 2 GiB the route moves off the brick GEMMs

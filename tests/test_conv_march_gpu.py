@@ -65,8 +65,9 @@ def test_against_float64_and_the_im2col_gemm(ctmr, dev, shape, cout, stride, opt
     f, L = ctmr.fast_fp32, ctmr._lib
     x, w, bias, affine, res = _inputs(shape, cout, stride, opts, dev)
     silu, groups = bool(opts.get("silu")), opts.get("gn", 0)
-    # this kernel reads x itself (stride 2: no im2col rows in the workspace)
-    assert L.workspace_bytes(ctmr.ops.make_desc(shape, cout, 3, stride, L.MODE_PLAIN, 0, L.DT_F32, 0)) == 0
+    desc = ctmr.ops.make_desc(shape, cout, 3, stride, L.MODE_PLAIN, 0, L.DT_F32, 0)
+    assert L.conv_kernel(desc) == "march"
+    assert L.workspace_bytes(desc) == 0  # x itself is read: no im2col rows
     run = lambda stream: f.implicit_gemm_conv3d(x, f.pack_weight(w), bias, cout=cout, affine=affine, silu=silu,
                                                 stride=stride, residual=res, stream_gemm=stream, gn_groups=groups)
     y, y1 = run(False), run(True)
@@ -92,7 +93,8 @@ def test_against_float64_and_the_im2col_gemm(ctmr, dev, shape, cout, stride, opt
 def test_non_finite_values_reach_their_windows_only(ctmr, dev, shape, cout, stride):
     """An infinity or a NaN makes the outputs of its 3x3x3 windows what fp32 sums make them and no others (the
     zero weights beside a row's window must not spread it)."""
-    f = ctmr.fast_fp32
+    f, L = ctmr.fast_fp32, ctmr._lib
+    assert L.conv_kernel(ctmr.ops.make_desc(shape, cout, 3, stride, L.MODE_PLAIN, 0, L.DT_F32, 0)) == "march"
     x, w, bias, _, _ = _inputs(shape, cout, stride, {}, dev)
     x[0, 7, 11, 13, 2] = float("inf")
     x[0, 20, 0, 31, 5] = float("-inf")

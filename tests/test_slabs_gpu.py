@@ -29,6 +29,8 @@ CASES = [
     ("split fp16 LDS GEMM", (1, 16, 32, 32, 64), 0, 64, {"fused": True}, "f16x2", True),
     ("two-source input", (2, 16, 32, 32, 64), 32, 64, {"fused": True}, "fp32", True),
     ("1x1x1 over a GN + SiLU pack", (1, 16, 32, 32, 128), 0, 64, {"fused": True, "ksize": 1}, "fp32", True),
+    # its slabs would fall below the plane-marching conv's size: another kernel, so the volume runs whole
+    ("8 -> 8 plane by plane", (1, 160, 64, 64, 8), 0, 8, {"fused": True}, "fp32", False),
 ]
 
 
@@ -81,7 +83,7 @@ def test_depth_slabs_match_whole_volume(ctmr, dev, monkeypatch, name, shape, cin
     slabs = f.implicit_gemm_conv3d(xin, packed, bias, **call)
     print(f"{name}: route {ctmr._lib.conv_kernel(desc)}, split {ctmr._lib.conv_split(desc)}, "
           f"{calls['n']} slab launches", flush=True)
-    if slabbed:
-        assert calls["n"] > 1, "the budget should have split this conv into slabs"
+    if slabbed is not None:
+        assert (calls["n"] > 1) == slabbed, "slabs" if slabbed else "no slab depth keeps this conv's kernel"
     assert tuple(slabs.shape) == tuple(whole.shape)
     assert torch.equal(slabs, whole), "a slabbed conv must return the whole volume's bits"
