@@ -2696,6 +2696,7 @@ struct Geometry {
   bool lds_small;        // LDS-staged im2col GEMM for cin 4 / 8 (conv_lds_small_kernel)
   bool cat;              // input given as two tensors, channels [0, c1) and [c1, cin)
   int c1;
+  bool x16;              // x read in place must be 16-byte aligned (4 bytes otherwise)
   bool pointwise;        // one-tap GEMM on the persistent pointwise_kernel
   bool direct;           // streaming GEMM reading the unpadded input (no pack)
   bool kws;              // 64 x 64 tiles, the K range of each split over the four waves
@@ -2756,6 +2757,7 @@ static int geometry(const ctmr_conv_desc* d, Geometry& g) {
     return fail(CTMR_E_UNSUPPORTED, "1x1x1 conv supports only stride 1, no resampling");
   g.cat = d->cin1 != 0;
   g.c1 = g.cat ? d->cin1 : d->cin;
+  g.x16 = true;
   if (g.cat && (d->cin1 < 0 || d->cin1 >= d->cin || d->cin1 % 16 != 0 || d->cin % 16 != 0))
     return fail(CTMR_E_INVALID, "two-source input needs 0 < cin1 < cin, both multiples of 16");
   if (g.cat && d->mode != CTMR_MODE_PLAIN)
@@ -2849,6 +2851,11 @@ static int geometry(const ctmr_conv_desc* d, Geometry& g) {
   // taken (outputs past that span would be dropped by the buffer range).
   const bool brick_out_fits =
       (int64_t)kBD * (g.phases == 8 ? 2 : 1) * g.oh * g.ow * d->cout * 4 < (1ll << 31);
+  // 4x8x8 bricks of a stride-1 conv of 4 or 8 channels at least 3/4 full and 6
+  // staged planes within 32-bit buffer offsets: the brick GEMM's shapes below.
+  const int64_t small_slots = ceil_div(d->d, kBD) * ceil_div(d->h, kBH) * ceil_div(d->w, kBW) * (kBD * kBH * kBW);
+  const bool small_bricks = 4 * S >= 3 * small_slots && (int64_t)kHD * d->h * d->w * d->cin * 4 < (1ll << 31) &&
+                            brick_out_fits;
   // Plane-marching conv: 8 input channels, fp32, stride 1 to 8 outputs or
   // stride 2 to 17 .. 32.  Reads x itself.  From about 2^18 outputs at
   // stride 1 and 2^15 at stride 2, tiles at least half full; a plane of x within
@@ -2865,6 +2872,7 @@ static int geometry(const ctmr_conv_desc* d, Geometry& g) {
     const int64_t slots = ty * march_rows(d->stride) * tx * march_cols(d->stride);
     if (2 * (int64_t)g.oh * g.ow >= slots) {
       g.march = true;
+      g.x16 = d->stride == 1 && small_bricks;  // shapes the brick GEMM takes too; im2col rows take any x
       g.pack = false;
       g.ty = (int)ty; g.tx = (int)tx;
       g.run = march_run(ty * tx * d->n, g.od, d->stride);
@@ -2892,9 +2900,7 @@ static int geometry(const ctmr_conv_desc* d, Geometry& g) {
       (d->cin == 4 || d->cin == 8) && d->cout % 4 == 0 && (d->cout % 64 == 0 || d->cout <= 32) &&
       !(d->flags & CTMR_F_STREAM)) {
     const int tz = (int)ceil_div(d->d, kBD), ty = (int)ceil_div(d->h, kBH), tx = (int)ceil_div(d->w, kBW);
-    const int64_t slots = (int64_t)tz * ty * tx * kBD * kBH * kBW;
-    const int64_t planes = (int64_t)kHD * d->h * d->w * d->cin * 4;
-    if (4 * S >= 3 * slots && planes < (1ll << 31) && brick_out_fits) {
+    if (small_bricks) {
       g.lds_small = true;
       g.pack = false;
       g.tz = tz; g.ty = ty; g.tx = tx;
@@ -3147,9 +3153,9 @@ static int split_gn_rows(const ctmr_conv_desc* d, const Geometry& g) {
 static int gn_stats_tiles(const ctmr_conv_desc* d, const Geometry& g, int groups) {
   if (groups <= 0 || d->cout % groups != 0) return 0;
   if (g.layout == WL_EXPAND) return 0;
-  if (g.march) {  // the stride-2 form's 32-column tiles
+  if (g.march) {  // 8 or up to 32 columns
     const int cpg = d->cout / groups;
-    return d->stride == 2 && 32 % cpg == 0 ? g.m_tiles : 0;
+    return (d->stride == 1 || 32 % cpg == 0) ? g.m_tiles : 0;
   }
   if (g.lds_small) {  // 64-column bricks only (the narrow epilogue writes no statistics)
     const int cpg = d->cout / groups;
@@ -3613,7 +3619,7 @@ static int conv3d_gemm_impl(const ctmr_conv_desc* desc, const float* x, const fl
   if ((desc->flags & CTMR_F_BATCH_BIAS) && !bias) return fail(CTMR_E_INVALID, "batch bias flag without bias");
   if ((rc = check_workspace(g, workspace, workspace_bytes))) return rc;
   const char* xp = g.pack ? (const char*)workspace : (const char*)x;
-  if (!g.pack && !(g.march && desc->stride == 2) && ((uintptr_t)x & 15) != 0) return fail(CTMR_E_INVALID, "x must be 16-byte aligned");
+  if (!g.pack && g.x16 && ((uintptr_t)x & 15) != 0) return fail(CTMR_E_INVALID, "x must be 16-byte aligned");
   // The bf16 LDS GEMM and the pointwise GEMM store (and read the residual) 16 bytes at a time.
   const uintptr_t wide = (uintptr_t)y | ((desc->flags & CTMR_F_RESIDUAL) ? (uintptr_t)residual : 0) |
                          (g.split > 1 ? (uintptr_t)workspace : 0);

@@ -109,6 +109,7 @@ template <int STRIDE>
 __global__ __launch_bounds__(256, 2) void conv_march_kernel(MarchArgs p) {
   using M = March<STRIDE>;
   __shared__ __attribute__((aligned(256))) char lds[2 * M::kBuf];
+  __shared__ double red[4][16][2];  // group-norm sums: each wave's 16 output columns
   const int tid = threadIdx.x, lane = tid & 63, lrow = lane & 15, lgrp = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // XCD-aware order: tiles that share halo lines run on one XCD
@@ -269,7 +270,6 @@ __global__ __launch_bounds__(256, 2) void conv_march_kernel(MarchArgs p) {
     const float* bq = p.bias + (p.batch_bias ? b * p.cout : 0) + ocol;
     bias = f4{bq[0], bq[1], bq[2], bq[3]};
   }
-  double s1[4] = {0.0, 0.0, 0.0, 0.0}, s2[4] = {0.0, 0.0, 0.0, 0.0};
   auto store = [&](f4 (&sum)[4], int oz) {
     float probe = 0.f;  // not finite: a NaN or an infinity among the results to be stored
 #pragma unroll
@@ -298,23 +298,39 @@ __global__ __launch_bounds__(256, 2) void conv_march_kernel(MarchArgs p) {
     for (int t = 0; t < 4; ++t) {
       const int oy = y0 + orow + (STRIDE == 1 ? 2 * t : t);
       if (oy >= p.oh || ox >= p.ow || ocol >= p.cout) continue;
-      f4 v = sum[t];
+      f4& v = sum[t];
       v += bias;
       const int64_t at = ((((int64_t)b * p.od + oz) * p.oh + oy) * p.ow + ox) * p.cout + ocol;
       if (p.res) v += *reinterpret_cast<const f4a4*>(p.res + at);
       *reinterpret_cast<f4a4*>(p.y + at) = v;
-      if constexpr (STRIDE == 2) {
-        if (p.stats) {
+    }
+    if (p.stats) {  // one column at a time: its lane sums over the row blocks, then the 16 columns of a line
+#pragma clang loop unroll(disable)
+      for (int j = 0; j < 4; ++j) {
+        double a = 0.0, q = 0.0;
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            s1[j] += (double)v[j];
-            s2[j] = fma((double)v[j], (double)v[j], s2[j]);
+        for (int t = 0; t < 4; ++t) {
+          const int oy = y0 + orow + (STRIDE == 1 ? 2 * t : t);
+          const double v = j == 0 ? sum[t][0] : j == 1 ? sum[t][1] : j == 2 ? sum[t][2] : sum[t][3];
+          if (oy < p.oh && ox < p.ow && ocol < p.cout) {
+            a += v;
+            q = fma(v, v, q);
           }
+        }
+        a = row16_sum(a);
+        q = row16_sum(q);
+        if (lrow == 0) {
+          red[wave][lgrp * 4 + j][0] += a;
+          red[wave][lgrp * 4 + j][1] += q;
         }
       }
     }
   };
 
+  if (p.stats && lrow == 0) {  // read and added to by this lane only, until the last barrier
+#pragma unroll
+    for (int j = 0; j < 4; ++j) red[wave][lgrp * 4 + j][0] = red[wave][lgrp * 4 + j][1] = 0.0;
+  }
   // Planes oz0 * STRIDE - 1 .. (oz1 - 1) * STRIDE + 1, those outside the volume
   // skipped: zeros add nothing.  One barrier per plane: a wave writes a buffer
   // after the barrier of the plane between, which every wave reaches only when
@@ -369,30 +385,21 @@ __global__ __launch_bounds__(256, 2) void conv_march_kernel(MarchArgs p) {
         acc[1][t] = f4{0.f, 0.f, 0.f, 0.f};
       }
     }
-    if (p.stats) {  // a kernel argument: every thread reaches the barriers
-      double (*red)[16][2] = reinterpret_cast<double (*)[16][2]>(lds);
-      __syncthreads();
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const double q1 = row16_sum(s1[j]), q2 = row16_sum(s2[j]);
-        if (lrow == 0) {
-          red[wave][lgrp * 4 + j][0] = q1;
-          red[wave][lgrp * 4 + j][1] = q2;
+  }
+  if (p.stats) {  // a kernel argument: every thread reaches the barrier
+    __syncthreads();
+    const int cpg = p.cout / p.gn_groups;
+    if (tid < p.gn_groups) {  // columns, then the waves that hold them (both rows of stride 1), ascending
+      double a = 0.0, q = 0.0;
+      for (int c = tid * cpg; c < (tid + 1) * cpg; ++c)
+        for (int half = 0; half < (STRIDE == 1 ? 8 : 2); ++half) {
+          const double* r = STRIDE == 1 ? red[half >> 1][(half & 1) * 8 + c] : red[half * 2 + (c >> 4)][c & 15];
+          a += r[0];
+          q += r[1];
         }
-      }
-      __syncthreads();
-      const int cpg = p.cout / p.gn_groups;
-      if (tid < p.gn_groups) {  // columns, then row halves, ascending
-        double a = 0.0, q = 0.0;
-        for (int c = tid * cpg; c < (tid + 1) * cpg; ++c)
-          for (int half = 0; half < 2; ++half) {
-            a += red[half * 2 + (c >> 4)][c & 15][0];
-            q += red[half * 2 + (c >> 4)][c & 15][1];
-          }
-        double* out = p.stats + ((int64_t)tile * p.gn_groups + tid) * 2;
-        out[0] = a;
-        out[1] = q;
-      }
+      double* out = p.stats + ((int64_t)tile * p.gn_groups + tid) * 2;
+      out[0] = a;
+      out[1] = q;
     }
   }
 }

@@ -19,7 +19,9 @@ CASES = [
     ((1, 64, 64, 96, 8), 8, 1, {}),
     ((1, 65, 71, 75, 8), 8, 1, {"silu": True}),
     ((2, 97, 47, 77, 8), 8, 1, {"affine": True, "silu": True, "residual": True, "batch_bias": True}),
-    ((1, 5, 270, 250, 8), 8, 1, {"affine": True}),
+    ((1, 5, 270, 250, 8), 8, 1, {"affine": True, "gn": 4}),
+    ((2, 97, 47, 77, 8), 8, 1, {"residual": True, "gn": 8}),
+    ((1, 65, 71, 75, 8), 8, 1, {"silu": True, "gn": 1}),
     ((1, 64, 64, 64, 8), 32, 2, {"silu": True}),
     ((1, 75, 83, 101, 8), 32, 2, {}),
     ((2, 66, 57, 79, 8), 20, 2, {"affine": True, "silu": True, "residual": True, "batch_bias": True}),
@@ -107,3 +109,23 @@ def test_non_finite_values_reach_their_windows_only(ctmr, dev, shape, cout, stri
     assert torch.equal(torch.isinf(y), inf) and torch.equal(y[inf], y1[inf])
     ok = torch.isfinite(y1)
     assert bool(((y[ok].double() - y1[ok].double()).abs() <= 1e-5 * (1 + y1[ok].double().abs())).all())
+
+
+@pytest.mark.parametrize(("shape", "cout", "stride"), [((1, 5, 270, 250, 8), 8, 1), ((1, 64, 64, 64, 8), 32, 2)])
+def test_input_at_any_four_byte_address(ctmr, dev, shape, cout, stride):
+    """Volumes whose im2col rows would be packed (4x8x8 bricks under 3/4 full, or stride 2) take x at any 4-byte
+    address, as the pack does: the aligned call's bits."""
+    import ctypes
+
+    f, L = ctmr.fast_fp32, ctmr._lib
+    x, w, bias, _, _ = _inputs(shape, cout, stride, {}, dev)
+    packed = f.pack_weight(w)
+    desc = ctmr.ops.make_desc(shape, cout, 3, stride, L.MODE_PLAIN, 0, L.DT_F32, 0)
+    assert L.conv_kernel(desc) == "march" and L.workspace_bytes(desc) == 0
+    y = f.implicit_gemm_conv3d(x, packed, bias, cout=cout, stride=stride)
+    odd = torch.empty(x.numel() + 1, device=dev)[1:].view(shape)
+    odd.copy_(x)
+    again = torch.zeros_like(y)
+    L.check(L.lib().ctmr_conv3d(ctypes.byref(desc), odd.data_ptr(), packed.data_ptr(), bias.data_ptr(), None, None,
+                                again.data_ptr(), None, 0, torch.cuda.current_stream().cuda_stream), "ctmr_conv3d")
+    assert torch.equal(again, y)
