@@ -394,8 +394,8 @@ int ctmr_resample(int32_t op, int32_t n, int32_t d, int32_t h, int32_t w, int32_
  * (0, 1 or 2) is a hint: every wave takes 16 queries, the fastest form
  * throughout, and results do not depend on it.  Keys are visited in a fixed
  * order: ascending 32-key blocks, or -- for small grids, decided from n, lq, lk
- * and heads only -- two such runs over the key halves, combined first half
- * first.  The fp32 operands are multiplied as three bf16 parts that together
+ * and heads only -- two or four such runs over equal key parts, combined in
+ * ascending order.  The fp32 operands are multiplied as three bf16 parts that together
  * hold their 24 significant bits (as CTMR_K_LDS convolutions); output rows that
  * are not finite are recomputed with plain fp32 products. */
 typedef struct ctmr_attn_desc {

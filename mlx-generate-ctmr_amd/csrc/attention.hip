@@ -55,14 +55,18 @@ __device__ __forceinline__ float lane_group_max(float v) {
   return fmaxf(__uint_as_float(q[0]), __uint_as_float(q[1]));
 }
 
-// Keys of the first part of a two-part key split: half the keys, rounded up
-// to a multiple of 64 (whole key blocks, so only the last block is ragged).
-__device__ __forceinline__ int attention_part_keys(int lk) { return (((lk + 1) / 2 + 63) / 64) * 64; }
+// Keys of every part but the last of a split in KS: an equal share, rounded up
+// to whole key blocks, so only the last block is ragged (halves to 64 keys).
+template <int KS>
+__device__ __forceinline__ int attention_part_keys(int lk) {
+  constexpr int kUnit = KS == 2 ? 64 : kBlock;
+  return ((lk + KS - 1) / KS + kUnit - 1) / kUnit * kUnit;
+}
 
-// Whether a wave's staging piece j (flash_attention_kernel) is of K.
+// Whether a wave's staging piece j of KS (flash_attention_kernel) is of K.
 template <int KS>
 __device__ __forceinline__ bool wave_piece_is_k(int wave, int j) {
-  return KS == 1 ? wave < kWaves / 2 : j == 0;
+  return KS == 1 ? wave < kWaves / 2 : j < KS / 2;
 }
 
 // Online softmax of one 32-key block, shared by both kernels: scores -> P^T in
@@ -238,29 +242,34 @@ __device__ __forceinline__ void attention_rerun(const AttnArgs& a, const float* 
 }
 
 // A workgroup of eight waves: KS key parts x (8 / KS) query groups of 16
-// queries (KS = 2 for small grids: part p takes the keys from
-// p * attention_part_keys on).  Each step the threads of a part load its next
-// 32-key block of K and V as fp32, split it once for all the part's waves and
-// publish it in LDS in MFMA operand order (K rows of 32 dims; V transposed,
-// 32 dims x 32 keys in P^T's k order), one block ahead, one barrier a step.
-// The fp32 loads of the block after the next are in flight during a step.
+// queries (KS = 2 or 4 for small grids: part p takes the keys from
+// p * attention_part_keys on).  Each step the threads of a part load a 32-key
+// block of K and V as fp32, split it once for all the part's waves and publish
+// it in LDS in MFMA operand order (K rows of 32 dims; V transposed, 32 dims x
+// 32 keys in P^T's k order), one block ahead, one barrier a step.  The fp32
+// loads of the next block, or of the next two with key parts, are in flight
+// during a step.
 // Sharing the blocks is what the time followed: with every wave loading its
 // own operands the kernel took as long on fp16 MFMA as on FP32 MFMA, and 16
 // queries a wave 1.6 times 32 queries a wave at any occupancy.  Measured, that
-// form / this one us: 2048 tokens x 16 heads fp32 84 / 69, split fp16 82 / 51
-// (its separate split pass included); 4158 x 8 245 / 178, 225 / 144; 4800 x 16
-// 553 / 334, 503 / 256.  Now bound by LDS reads (8 or 12 of 1 KiB a wave and
+// form (its separate split pass included) / this one us: 2048 tokens x 8 heads
+// x 2 fp32 87 / 70, split fp16 86 / 53; 4158 x 8 244 / 173, 237 / 143; 4800 x
+// 16 553 / 334, 500 / 263.  Now bound by LDS reads (8 or 12 of 1 KiB a wave and
 // block: 58 % of the cycles) and VALU (168 operations: 57 %) together; 32
 // queries a wave halve the reads but leave half the waves: 67, 70; 193, 177 us.
+// A small grid is bound by the latency of its steps: 1024 tokens x 8 heads 16.2
+// / 15.2, 33.4 / 13.8; 256 x 16 x 2 7.2 / 7.8, 13.4 / 6.8 (with two parts and
+// one block in flight 21.6, 18.8; 8.8, 7.6).
 template <int SCH, int KS>
 __global__ __launch_bounds__(kThreads, SCH == kFp32 && KS == 1 ? 6 : 4) void flash_attention_kernel(AttnArgs a) {
-  static_assert(KS == 1 || KS == 2, "one or two key parts");
+  static_assert(KS == 1 || KS == 2 || KS == 4, "one, two or four key parts");
   constexpr int QT = kQueryTiles;
   constexpr int kGroups = kWaves / KS, kPartThreads = kThreads / KS;
+  constexpr int kAhead = KS == 1 ? 1 : 2;  // blocks in registers beyond the one in LDS
   constexpr int kBuf = 2 * SCH * kPlane;  // K planes, then V planes
   constexpr int NO = SCH == kF16x2 ? 4 : 2;  // output accumulators per query tile
   __shared__ __attribute__((aligned(16))) char lds[2][KS][kBuf];
-  static_assert((kWaves / KS) * (KS - 1) * QT * (2 + 4 * NO) * 64 * 4 <= 2 * KS * kBuf, "the hand-over fits");
+  static_assert(kGroups * (KS - 1) * QT * (2 + 4 * NO) * 64 * 4 <= 2 * KS * kBuf, "the hand-over fits");
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, g = lane >> 4;
@@ -269,7 +278,7 @@ __global__ __launch_bounds__(kThreads, SCH == kFp32 && KS == 1 ? 6 : 4) void fla
   const int q0 = (blockIdx.x * kGroups + group) * (QT * 16);
   // Wave-uniform.  Every wave reaches every barrier: a query group past the
   // end runs on clamped rows and stores nothing.
-  const int part_keys = KS == 1 ? a.lk : attention_part_keys(a.lk);
+  const int part_keys = KS == 1 ? a.lk : attention_part_keys<KS>(a.lk);
   const int k_begin = min(a.lk, part * part_keys), k_end = min(a.lk, k_begin + part_keys);
   const int steps = (min(part_keys, a.lk) + kBlock - 1) / kBlock;  // part 0's, the most of any part
 
@@ -308,8 +317,7 @@ __global__ __launch_bounds__(kThreads, SCH == kFp32 && KS == 1 ? 6 : 4) void fla
     }
   }
   const unsigned vrow = (unsigned)(a.ldv * 4);
-  f4 raw[KS];
-  auto fetch = [&](int k0) {
+  auto fetch = [&](int k0, f4 (&raw)[KS]) {
     const __amdgpu_buffer_rsrc_t rk = rows_rsrc(K, a.ldk, k0), rv = rows_rsrc(V, a.ldv, k0);
 #pragma unroll
     for (int j = 0; j < KS; ++j) {
@@ -325,7 +333,7 @@ __global__ __launch_bounds__(kThreads, SCH == kFp32 && KS == 1 ? 6 : 4) void fla
       }
     }
   };
-  auto publish = [&](char* buf) {
+  auto publish = [&](char* buf, const f4 (&raw)[KS]) {
 #pragma unroll
     for (int j = 0; j < KS; ++j) {
       uint2 p[SCH];
@@ -334,6 +342,12 @@ __global__ __launch_bounds__(kThreads, SCH == kFp32 && KS == 1 ? 6 : 4) void fla
       for (int i = 0; i < SCH; ++i) *reinterpret_cast<uint2*>(buf + loff[j] + i * kPlane) = p[i];
     }
   };
+
+  // The first blocks and Q in one round of latency.
+  f4 raw0[KS], raw[kAhead][KS];
+  fetch(k_begin, raw0);
+#pragma unroll
+  for (int i = 0; i < kAhead; ++i) fetch(k_begin + (1 + i) * kBlock, raw[i]);
 
   // Q^T as the B operand of S^T = K Q^T: query q0 + 16t + col, dims 8g .. 8g+7.
   u4 qf[QT][SCH];
@@ -444,30 +458,35 @@ __global__ __launch_bounds__(kThreads, SCH == kFp32 && KS == 1 ? 6 : 4) void fla
     }
   };
 
-  fetch(k_begin);
-  publish(lds[0][part]);
-  fetch(k_begin + kBlock);
-  for (int i = 0; i < steps; ++i) {
+  publish(lds[0][part], raw0);
+  auto step = [&](int i, f4 (&ahead)[KS]) {
     // Block i is published, and every wave is done with block i - 1, whose
     // buffer takes block i + 1 (past the part's keys: other keys or zeros,
     // never used).
     lds_barrier();
-    publish(lds[(i + 1) & 1][part]);
+    publish(lds[(i + 1) & 1][part], ahead);
     const int k0 = k_begin + i * kBlock;
-    fetch(k0 + 2 * kBlock);
+    fetch(k0 + (1 + kAhead) * kBlock, ahead);
     if (k0 + kBlock <= k_end) block(lds[i & 1][part], k0, std::false_type{});
     else if (k0 < k_end) block(lds[i & 1][part], k0, std::true_type{});
+  };
+  for (int i = 0; i < steps; i += kAhead) {
+    step(i, raw[0]);
+    if constexpr (kAhead == 2) {
+      if (i + 1 < steps) step(i + 1, raw[1]);
+    }
   }
 
-  if constexpr (KS == 2) {
-    // The second part's waves hand their running max, sum and accumulators to
-    // the first's, which rescale both and add them in that fixed order.
-    float* const xch = reinterpret_cast<float*>(&lds[0][0][0]) + group * (QT * (2 + 4 * NO) * 64) + lane;
+  if constexpr (KS > 1) {
+    // The later parts' waves hand their running max, sum and accumulators to
+    // the first's, which rescales and adds them part by part, ascending.
+    constexpr int kSlot = QT * (2 + 4 * NO) * 64;  // one wave's
+    float* const xch = reinterpret_cast<float*>(&lds[0][0][0]) + group * (KS - 1) * kSlot + lane;
     lds_barrier();
-    if (part == 1) {
+    if (part > 0) {
 #pragma unroll
       for (int t = 0; t < QT; ++t) {
-        float* o = xch + t * (2 + 4 * NO) * 64;
+        float* o = xch + (part - 1) * kSlot + t * (2 + 4 * NO) * 64;
         o[0] = m[t];
         o[64] = l[t];
 #pragma unroll
@@ -477,19 +496,22 @@ __global__ __launch_bounds__(kThreads, SCH == kFp32 && KS == 1 ? 6 : 4) void fla
       }
     }
     lds_barrier();
-    if (part == 1) return;
+    if (part > 0) return;
 #pragma unroll
-    for (int t = 0; t < QT; ++t) {
-      const float* o = xch + t * (2 + 4 * NO) * 64;
-      const float m1 = o[0];
-      const float mm = fmaxf(m[t], m1);  // the first part always holds keys: finite
-      const float a0 = exp2f(m[t] - mm), a1 = exp2f(m1 - mm);  // a1 = 0 for an empty second part
-      l[t] = l[t] * a0 + o[64] * a1;
+    for (int k = 0; k < KS - 1; ++k)
 #pragma unroll
-      for (int j = 0; j < NO; ++j)
+      for (int t = 0; t < QT; ++t) {
+        const float* o = xch + k * kSlot + t * (2 + 4 * NO) * 64;
+        const float m1 = o[0];
+        const float mm = fmaxf(m[t], m1);  // the first part always holds keys: finite
+        const float a0 = exp2f(m[t] - mm), a1 = exp2f(m1 - mm);  // a1 = 0 for an empty part
+        m[t] = mm;
+        l[t] = l[t] * a0 + o[64] * a1;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[t][j][e] = acc[t][j][e] * a0 + o[(2 + 4 * j + e) * 64] * a1;
-    }
+        for (int j = 0; j < NO; ++j)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[t][j][e] = acc[t][j][e] * a0 + o[(2 + 4 * j + e) * 64] * a1;
+      }
   }
 
   float* O = a.out + (int64_t)b * a.lq * a.ldo + h * kHeadDim;
@@ -546,12 +568,15 @@ bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 }  // namespace
 
 // Key parts, from the shape only: two when there are at least 128 keys and the
-// grid of two parts stays under two rounds of 512 workgroups.  Measured, one /
-// two parts us: 4158 tokens x 8 heads 210 / 178 (fp32), 160 / 144 (split
-// fp16); 3000 x 16 154 / 137, 118 / 110.
+// grid of two parts stays under two rounds of 512 workgroups; four when their
+// grid, 32 queries a workgroup, leaves every workgroup a CU of its own.
+// Measured, one / two parts us: 4158 tokens x 8 heads 210 / 178 (fp32), 160 /
+// 144 (split fp16); 3000 x 16 154 / 137, 118 / 110.  Two / four: 512 x 8 12.8 /
+// 9.6, 11.2 / 8.8; 648 x 8 16.6 / 12.3, 14.7 / 11.2.
 int attention_key_parts(int n, int lq, int lk, int heads) {
-  const int64_t blocks = ceil_div(ceil_div(lq, 16), kWaves / 2) * n * heads;
-  return (lk >= 128 && blocks < 1024) ? 2 : 1;
+  if (lk < 128) return 1;
+  if (ceil_div(lq, 32) * n * heads <= 256) return 4;
+  return ceil_div(lq, 64) * n * heads < 1024 ? 2 : 1;
 }
 
 }  // namespace ctmr
@@ -601,8 +626,11 @@ int run_attention(const ctmr_attn_desc* d, const float* q, const float* k, const
   const AttnArgs a{q, k, v, out, d->ldq, d->ldk, d->ldv, d->ldo, d->lq, d->lk, d->heads,
                    (float)((double)d->scale * 1.4426950408889634)};
   hipStream_t st = (hipStream_t)stream;
-  return attention_key_parts(d->n, d->lq, d->lk, d->heads) == 2 ? launch_attention<SCH, 2>(a, d->n, st)
-                                                                : launch_attention<SCH, 1>(a, d->n, st);
+  switch (attention_key_parts(d->n, d->lq, d->lk, d->heads)) {
+    case 1: return launch_attention<SCH, 1>(a, d->n, st);
+    case 2: return launch_attention<SCH, 2>(a, d->n, st);
+    default: return launch_attention<SCH, 4>(a, d->n, st);
+  }
 }
 
 // Split-fp16 workspace: six fp16 planes (Q hi/lo, K hi/lo, V^T hi/lo), each

@@ -19,10 +19,13 @@ def _reference(q, k, v, heads, scale):
     return (p @ split(v)).transpose(1, 2).reshape(n, lq, c)
 
 
-# one key; a block less one / whole / plus one; the two-part split's edges (an empty, one-key and full second part);
+# one key; a block less one / whole / plus one; the four-part split's edges (empty, one-key and full last parts);
 # query tiles and groups less one / plus one
 SHAPES = [(1, 1, 1, 1), (2, 15, 31, 2), (1, 16, 32, 1), (1, 17, 33, 3), (1, 65, 127, 2), (2, 64, 128, 1), (1, 63, 129, 2),
-          (1, 129, 192, 1), (1, 128, 193, 2), (1, 40, 255, 1), (1, 300, 257, 2), (1, 128, 2049, 1), (3, 2048, 64, 16)]
+          (1, 129, 192, 1), (1, 128, 193, 2), (1, 40, 255, 1), (1, 300, 257, 2), (1, 128, 2049, 1), (3, 2048, 64, 16),
+          # four parts to 256 workgroups of 32 queries, two to 1023 of 64, then one; the two-part split's edges
+          (2, 256, 128, 16), (2, 257, 128, 16), (2, 288, 129, 16), (2, 300, 192, 16), (2, 300, 193, 16),
+          (2, 270, 255, 16), (3, 1300, 300, 16), (1, 1023 * 64, 161, 1), (1, 1023 * 64 + 1, 161, 1)]
 
 
 @pytest.mark.parametrize("precision", ["fp32", "f16x2"])
