@@ -415,10 +415,11 @@ int ctmr_flash_attention(const ctmr_attn_desc* desc, const float* q, const float
  * P = 2^(S - m) is split the same way and the cross terms of P V are summed
  * apart and added at the end.  About 2^-22 relative per product;
  * |q * scale * log2(e)|, |k| and |v| must stay below 65504.  Same descriptor,
- * checks and key order as ctmr_flash_attention.  workspace: at least
- * ctmr_flash_attention_f16x2_workspace_bytes(desc) bytes, 256-byte aligned
- * (-1 from that call for an invalid shape); checked, but not written: the
- * kernel splits each key block into LDS. */
+ * checks and key order as ctmr_flash_attention.  The kernel splits each key
+ * block into LDS and needs no workspace: null with 0 bytes.  One that is given
+ * is checked and not written: at least
+ * ctmr_flash_attention_f16x2_workspace_bytes(desc) bytes (-1 from that call for
+ * an invalid shape), 256-byte aligned. */
 int64_t ctmr_flash_attention_f16x2_workspace_bytes(const ctmr_attn_desc* desc);
 int ctmr_flash_attention_f16x2(const ctmr_attn_desc* desc, const float* q, const float* k, const float* v,
                                float* out, void* workspace, int64_t workspace_bytes, void* stream);

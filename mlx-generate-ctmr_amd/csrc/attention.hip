@@ -79,45 +79,40 @@ __device__ __forceinline__ bool wave_piece_is_k(int wave, int j) {
 // skipped (output / sum is the same quotient for any reference).  The decision
 // is per query, so every tiling computes the same bits.  RAGGED masks keys at
 // or past k_end (the last block only).
-template <int QT, bool RAGGED>
-__device__ __forceinline__ void block_softmax(f4 (&s)[kKeyTiles][QT], float (&m)[QT], float (&l)[QT],
-                                              float (&alpha)[QT], int k0, int k_end, int g) {
+template <bool RAGGED>
+__device__ __forceinline__ void block_softmax(f4 (&s)[kKeyTiles], float& m, float& l, float& alpha, int k0, int k_end,
+                                              int g) {
   if constexpr (RAGGED) {
 #pragma unroll
     for (int u = 0; u < kKeyTiles; ++u)
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        if (k0 + u * 16 + 4 * g + r >= k_end)
-#pragma unroll
-          for (int t = 0; t < QT; ++t) s[u][t][r] = -INFINITY;
+        if (k0 + u * 16 + 4 * g + r >= k_end) s[u][r] = -INFINITY;
   }
+  float bm = s[0][0];
 #pragma unroll
-  for (int t = 0; t < QT; ++t) {
-    float bm = s[0][t][0];
+  for (int u = 0; u < kKeyTiles; ++u)
 #pragma unroll
-    for (int u = 0; u < kKeyTiles; ++u)
+    for (int r = 0; r < 4; ++r) bm = fmaxf(bm, s[u][r]);
+  bm = lane_group_max(bm);
+  // Every block holds at least one real key, so bm is finite and the first
+  // block moves the reference (alpha = 2^-inf = 0).  Arguments are <= 8:
+  // the hardware exp2 (v_exp_f32) differs from exp2f only below 2^-126,
+  // far under the resolution of the running sum (>= 1).
+  const bool move = bm > m + kLazyMax;
+  const float mn = move ? bm : m;
+  alpha = move ? __builtin_amdgcn_exp2f(m - mn) : 1.0f;
+  m = mn;
+  float ps = 0.f;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) bm = fmaxf(bm, s[u][t][r]);
-    bm = lane_group_max(bm);
-    // Every block holds at least one real key, so bm is finite and the first
-    // block moves the reference (alpha = 2^-inf = 0).  Arguments are <= 8:
-    // the hardware exp2 (v_exp_f32) differs from exp2f only below 2^-126,
-    // far under the resolution of the running sum (>= 1).
-    const bool move = bm > m[t] + kLazyMax;
-    const float mn = move ? bm : m[t];
-    alpha[t] = move ? __builtin_amdgcn_exp2f(m[t] - mn) : 1.0f;
-    m[t] = mn;
-    float ps = 0.f;
+  for (int u = 0; u < kKeyTiles; ++u)
 #pragma unroll
-    for (int u = 0; u < kKeyTiles; ++u)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float p = __builtin_amdgcn_exp2f(s[u][t][r] - mn);
-        s[u][t][r] = p;
-        ps += p;
-      }
-    l[t] = l[t] * alpha[t] + ps;
-  }
+    for (int r = 0; r < 4; ++r) {
+      const float p = __builtin_amdgcn_exp2f(s[u][r] - mn);
+      s[u][r] = p;
+      ps += p;
+    }
+  l = l * alpha + ps;
 }
 
 // Operand schemes of flash_attention_kernel.
@@ -137,7 +132,6 @@ __device__ __forceinline__ void block_softmax(f4 (&s)[kKeyTiles][QT], float (&m)
 constexpr int kFp32 = 3, kF16x2 = 2;  // the value is the number of parts
 
 constexpr int kThreads = 64 * kWaves;
-constexpr int kQueryTiles = 1;             // 16-query tiles a wave owns
 constexpr int kRow = 96;                   // LDS bytes of a 32-value row (64 used): conflict-free b128 reads of 16 rows
 constexpr int kPlane = kBlock * kRow;      // one part of one operand of a key block
 
@@ -263,19 +257,18 @@ __device__ __forceinline__ void attention_rerun(const AttnArgs& a, const float* 
 template <int SCH, int KS>
 __global__ __launch_bounds__(kThreads, SCH == kFp32 && KS == 1 ? 6 : 4) void flash_attention_kernel(AttnArgs a) {
   static_assert(KS == 1 || KS == 2 || KS == 4, "one, two or four key parts");
-  constexpr int QT = kQueryTiles;
   constexpr int kGroups = kWaves / KS, kPartThreads = kThreads / KS;
   constexpr int kAhead = KS == 1 ? 1 : 2;  // blocks in registers beyond the one in LDS
   constexpr int kBuf = 2 * SCH * kPlane;  // K planes, then V planes
   constexpr int NO = SCH == kF16x2 ? 4 : 2;  // output accumulators per query tile
   __shared__ __attribute__((aligned(16))) char lds[2][KS][kBuf];
-  static_assert(kGroups * (KS - 1) * QT * (2 + 4 * NO) * 64 * 4 <= 2 * KS * kBuf, "the hand-over fits");
+  static_assert(kGroups * (KS - 1) * (2 + 4 * NO) * 64 * 4 <= 2 * KS * kBuf, "the hand-over fits");
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, g = lane >> 4;
   const int b = blockIdx.y / a.heads, h = blockIdx.y % a.heads;
   const int part = wave / kGroups, group = wave % kGroups;
-  const int q0 = (blockIdx.x * kGroups + group) * (QT * 16);
+  const int q0 = (blockIdx.x * kGroups + group) * 16;
   // Wave-uniform.  Every wave reaches every barrier: a query group past the
   // end runs on clamped rows and stores nothing.
   const int part_keys = KS == 1 ? a.lk : attention_part_keys<KS>(a.lk);
@@ -349,12 +342,10 @@ __global__ __launch_bounds__(kThreads, SCH == kFp32 && KS == 1 ? 6 : 4) void fla
 #pragma unroll
   for (int i = 0; i < kAhead; ++i) fetch(k_begin + (1 + i) * kBlock, raw[i]);
 
-  // Q^T as the B operand of S^T = K Q^T: query q0 + 16t + col, dims 8g .. 8g+7.
-  u4 qf[QT][SCH];
-#pragma unroll
-  for (int t = 0; t < QT; ++t) {
-    const int row = min(q0 + t * 16 + col, a.lq - 1);
-    const f4* p = reinterpret_cast<const f4*>(Q + (int64_t)row * a.ldq + 8 * g);
+  // Q^T as the B operand of S^T = K Q^T: query q0 + col, dims 8g .. 8g+7.
+  u4 qf[SCH];
+  {
+    const f4* p = reinterpret_cast<const f4*>(Q + (int64_t)min(q0 + col, a.lq - 1) * a.ldq + 8 * g);
     f4 v0 = p[0] * a.qscale, v1 = p[1] * a.qscale;
     // opaque: the scaled values are rounded to fp32 before they are split
     asm volatile("" : "+v"(v0), "+v"(v1));
@@ -362,82 +353,69 @@ __global__ __launch_bounds__(kThreads, SCH == kFp32 && KS == 1 ? 6 : 4) void fla
     split_parts<SCH>(v0, p0);
     split_parts<SCH>(v1, p1);
 #pragma unroll
-    for (int i = 0; i < SCH; ++i) qf[t][i] = u4{p0[i].x, p0[i].y, p1[i].x, p1[i].y};
+    for (int i = 0; i < SCH; ++i) qf[i] = u4{p0[i].x, p0[i].y, p1[i].x, p1[i].y};
   }
 
-  // acc[t][0..1]: dims 16j + 4g + r; split fp16: acc[t][2..3] the 2^11-scaled
-  // cross terms.
-  f4 acc[QT][NO];
-  float m[QT], l[QT], alpha[QT];
+  // acc[0..1]: dims 16j + 4g + r; split fp16: acc[2..3] the 2^11-scaled cross
+  // terms.
+  f4 acc[NO];
 #pragma unroll
-  for (int t = 0; t < QT; ++t) {
-#pragma unroll
-    for (int j = 0; j < NO; ++j) acc[t][j] = f4{0.f, 0.f, 0.f, 0.f};
-    m[t] = -INFINITY;
-    l[t] = 0.f;
-  }
+  for (int j = 0; j < NO; ++j) acc[j] = f4{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f, alpha;
 
   const int rd = col * kRow + 16 * g;  // this lane's 16 bytes of row `col`
   // One key block from `buf`: S^T, the softmax, the split of P, P V.
   auto block = [&](const char* buf, int k0, auto ragged) {
-    f4 s[kKeyTiles][QT];
+    f4 s[kKeyTiles];
 #pragma unroll
     for (int u = 0; u < kKeyTiles; ++u) {
       u4 kf[SCH];
 #pragma unroll
       for (int i = 0; i < SCH; ++i) kf[i] = *reinterpret_cast<const u4*>(buf + i * kPlane + u * 16 * kRow + rd);
+      const f4 z = {0.f, 0.f, 0.f, 0.f};
+      if constexpr (SCH == kFp32) {
+        s[u] = mfma_x3(kf, qf, z);
+      } else {
+        const f4 hh = mfma32<SCH>(kf[0], qf[0], z);
+        f4 cr = mfma32<SCH>(kf[0], qf[1], z);
+        cr = mfma32<SCH>(kf[1], qf[0], cr);
 #pragma unroll
-      for (int t = 0; t < QT; ++t) {
-        const f4 z = {0.f, 0.f, 0.f, 0.f};
-        if constexpr (SCH == kFp32) {
-          s[u][t] = mfma_x3(kf, qf[t], z);
-        } else {
-          const f4 hh = mfma32<SCH>(kf[0], qf[t][0], z);
-          f4 cr = mfma32<SCH>(kf[0], qf[t][1], z);
-          cr = mfma32<SCH>(kf[1], qf[t][0], cr);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) s[u][t][r] = fmaf(cr[r], 1.0f / 2048.0f, hh[r]);
-        }
+        for (int r = 0; r < 4; ++r) s[u][r] = fmaf(cr[r], 1.0f / 2048.0f, hh[r]);
       }
     }
-    block_softmax<QT, decltype(ragged)::value>(s, m, l, alpha, k0, k_end, g);
+    block_softmax<decltype(ragged)::value>(s, m, l, alpha, k0, k_end, g);
     // acc *= alpha, skipped (same bits: every factor is exactly 1) unless a
     // lane of the wave moved its reference.
+    if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {
 #pragma unroll
-    for (int t = 0; t < QT; ++t)
-      if (__builtin_amdgcn_ballot_w64(alpha[t] != 1.0f)) {
+      for (int j = 0; j < NO; ++j) acc[j] *= alpha;
+    }
+    u4 pf[SCH];
+    if constexpr (SCH == kFp32) {
+      uint2 p0[SCH], p1[SCH];
+      split_parts<SCH>(s[0], p0);
+      split_parts<SCH>(s[1], p1);
 #pragma unroll
-        for (int j = 0; j < NO; ++j) acc[t][j] *= alpha[t];
-      }
-    u4 pf[QT][SCH];
+      for (int i = 0; i < SCH; ++i) pf[i] = u4{p0[i].x, p0[i].y, p1[i].x, p1[i].y};
+    } else {
+      h8 ph, pl;
 #pragma unroll
-    for (int t = 0; t < QT; ++t) {
-      if constexpr (SCH == kFp32) {
-        uint2 p0[SCH], p1[SCH];
-        split_parts<SCH>(s[0][t], p0);
-        split_parts<SCH>(s[1][t], p1);
+      for (int u = 0; u < kKeyTiles; ++u)
 #pragma unroll
-        for (int i = 0; i < SCH; ++i) pf[t][i] = u4{p0[i].x, p0[i].y, p1[i].x, p1[i].y};
-      } else {
-        h8 ph, pl;
+        for (int r = 0; r < 4; ++r) ph[4 * u + r] = (_Float16)s[u][r];
+      // The low halves below read hi from these packed registers (an opaque
+      // copy: otherwise the compiler converts each p to fp16 a second time).
+      asm volatile("" : "+v"(ph));
+      // lo = fp16((p - hi) * 2^11) = fp16(2^11 p - 2^11 hi): both products and
+      // their difference are exact in fp32, so one rounding of the fused form
+      // (v_fma_mix) gives the same half.
 #pragma unroll
-        for (int u = 0; u < kKeyTiles; ++u)
+      for (int u = 0; u < kKeyTiles; ++u)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) ph[4 * u + r] = (_Float16)s[u][t][r];
-        // The low halves below read hi from these packed registers (an opaque
-        // copy: otherwise the compiler converts each p to fp16 a second time).
-        asm volatile("" : "+v"(ph));
-        // lo = fp16((p - hi) * 2^11) = fp16(2^11 p - 2^11 hi): both products and
-        // their difference are exact in fp32, so one rounding of the fused form
-        // (v_fma_mix) gives the same half.
-#pragma unroll
-        for (int u = 0; u < kKeyTiles; ++u)
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            pl[4 * u + r] = (_Float16)__builtin_fmaf((float)ph[4 * u + r], -2048.0f, s[u][t][r] * 2048.0f);
-        pf[t][0] = __builtin_bit_cast(u4, ph);
-        pf[t][1] = __builtin_bit_cast(u4, pl);
-      }
+        for (int r = 0; r < 4; ++r)
+          pl[4 * u + r] = (_Float16)__builtin_fmaf((float)ph[4 * u + r], -2048.0f, s[u][r] * 2048.0f);
+      pf[0] = __builtin_bit_cast(u4, ph);
+      pf[1] = __builtin_bit_cast(u4, pl);
     }
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
@@ -445,15 +423,12 @@ __global__ __launch_bounds__(kThreads, SCH == kFp32 && KS == 1 ? 6 : 4) void fla
 #pragma unroll
       for (int i = 0; i < SCH; ++i)
         vf[i] = *reinterpret_cast<const u4*>(buf + (SCH + i) * kPlane + j * 16 * kRow + rd);
-#pragma unroll
-      for (int t = 0; t < QT; ++t) {
-        if constexpr (SCH == kFp32) {
-          acc[t][j] = mfma_x3(vf, pf[t], acc[t][j]);
-        } else {
-          acc[t][j] = mfma32<SCH>(vf[0], pf[t][0], acc[t][j]);
-          acc[t][2 + j] = mfma32<SCH>(vf[0], pf[t][1], acc[t][2 + j]);
-          acc[t][2 + j] = mfma32<SCH>(vf[1], pf[t][0], acc[t][2 + j]);
-        }
+      if constexpr (SCH == kFp32) {
+        acc[j] = mfma_x3(vf, pf, acc[j]);
+      } else {
+        acc[j] = mfma32<SCH>(vf[0], pf[0], acc[j]);
+        acc[2 + j] = mfma32<SCH>(vf[0], pf[1], acc[2 + j]);
+        acc[2 + j] = mfma32<SCH>(vf[1], pf[0], acc[2 + j]);
       }
     }
   };
@@ -480,79 +455,69 @@ __global__ __launch_bounds__(kThreads, SCH == kFp32 && KS == 1 ? 6 : 4) void fla
   if constexpr (KS > 1) {
     // The later parts' waves hand their running max, sum and accumulators to
     // the first's, which rescales and adds them part by part, ascending.
-    constexpr int kSlot = QT * (2 + 4 * NO) * 64;  // one wave's
+    constexpr int kSlot = (2 + 4 * NO) * 64;  // one wave's
     float* const xch = reinterpret_cast<float*>(&lds[0][0][0]) + group * (KS - 1) * kSlot + lane;
     lds_barrier();
     if (part > 0) {
+      float* o = xch + (part - 1) * kSlot;
+      o[0] = m;
+      o[64] = l;
 #pragma unroll
-      for (int t = 0; t < QT; ++t) {
-        float* o = xch + (part - 1) * kSlot + t * (2 + 4 * NO) * 64;
-        o[0] = m[t];
-        o[64] = l[t];
+      for (int j = 0; j < NO; ++j)
 #pragma unroll
-        for (int j = 0; j < NO; ++j)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) o[(2 + 4 * j + e) * 64] = acc[t][j][e];
-      }
+        for (int e = 0; e < 4; ++e) o[(2 + 4 * j + e) * 64] = acc[j][e];
     }
     lds_barrier();
     if (part > 0) return;
 #pragma unroll
-    for (int k = 0; k < KS - 1; ++k)
+    for (int k = 0; k < KS - 1; ++k) {
+      const float* o = xch + k * kSlot;
+      const float m1 = o[0];
+      const float mm = fmaxf(m, m1);  // the first part always holds keys: finite
+      const float a0 = exp2f(m - mm), a1 = exp2f(m1 - mm);  // a1 = 0 for an empty part
+      m = mm;
+      l = l * a0 + o[64] * a1;
 #pragma unroll
-      for (int t = 0; t < QT; ++t) {
-        const float* o = xch + k * kSlot + t * (2 + 4 * NO) * 64;
-        const float m1 = o[0];
-        const float mm = fmaxf(m[t], m1);  // the first part always holds keys: finite
-        const float a0 = exp2f(m[t] - mm), a1 = exp2f(m1 - mm);  // a1 = 0 for an empty part
-        m[t] = mm;
-        l[t] = l[t] * a0 + o[64] * a1;
+      for (int j = 0; j < NO; ++j)
 #pragma unroll
-        for (int j = 0; j < NO; ++j)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) acc[t][j][e] = acc[t][j][e] * a0 + o[(2 + 4 * j + e) * 64] * a1;
-      }
+        for (int e = 0; e < 4; ++e) acc[j][e] = acc[j][e] * a0 + o[(2 + 4 * j + e) * 64] * a1;
+    }
   }
 
-  float* O = a.out + (int64_t)b * a.lq * a.ldo + h * kHeadDim;
+  // The four lane groups hold partial sums of the same query; xor pairs add
+  // commutatively, so every lane ends with the same bits.
+  l += __shfl_xor(l, 16);
+  l += __shfl_xor(l, 32);
+  const float inv = 1.0f / l;
+  const int query = q0 + col;
+  f4 o[2];
 #pragma unroll
-  for (int t = 0; t < QT; ++t) {
-    // The four lane groups hold partial sums of the same query; xor pairs add
-    // commutatively, so every lane ends with the same bits.
-    float lt = l[t];
-    lt += __shfl_xor(lt, 16);
-    lt += __shfl_xor(lt, 32);
-    const float inv = 1.0f / lt;
-    const int query = q0 + t * 16 + col;
-    f4 o[2];
+  for (int j = 0; j < 2; ++j) {
+    o[j] = acc[j];
+    if constexpr (SCH == kF16x2) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      o[j] = acc[t][j];
-      if constexpr (SCH == kF16x2) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) o[j][r] = acc[t][j][r] + acc[t][2 + j][r] * (1.0f / 2048.0f);
-      }
-      o[j] *= inv;
+      for (int r = 0; r < 4; ++r) o[j][r] = acc[j][r] + acc[2 + j][r] * (1.0f / 2048.0f);
     }
-    if constexpr (SCH == kFp32) {
-      float probe = 0.f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) probe = fmaf(o[e >> 2][e & 3], 0.f, probe);
-      const bool bad = !(probe == 0.f);
-      if (__any(bad && query < a.lq)) {
-        f4 again[2];
-        attention_rerun(a, Q + (int64_t)min(query, a.lq - 1) * a.ldq, K, V, rows_rsrc, col, g, again);
-        if (bad) {
-          o[0] = again[0];
-          o[1] = again[1];
-        }
-      }
-    }
-    if (query >= a.lq) continue;
-    float* dst = O + (int64_t)query * a.ldo;
-    *reinterpret_cast<f4*>(dst + 4 * g) = o[0];       // dims 4g .. 4g+3
-    *reinterpret_cast<f4*>(dst + 16 + 4 * g) = o[1];  // dims 16 + 4g .. 16 + 4g+3
+    o[j] *= inv;
   }
+  if constexpr (SCH == kFp32) {
+    float probe = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) probe = fmaf(o[e >> 2][e & 3], 0.f, probe);
+    const bool bad = !(probe == 0.f);
+    if (__any(bad && query < a.lq)) {
+      f4 again[2];
+      attention_rerun(a, Q + (int64_t)min(query, a.lq - 1) * a.ldq, K, V, rows_rsrc, col, g, again);
+      if (bad) {
+        o[0] = again[0];
+        o[1] = again[1];
+      }
+    }
+  }
+  if (query >= a.lq) return;
+  float* const dst = a.out + ((int64_t)b * a.lq + query) * a.ldo + h * kHeadDim;
+  *reinterpret_cast<f4*>(dst + 4 * g) = o[0];       // dims 4g .. 4g+3
+  *reinterpret_cast<f4*>(dst + 16 + 4 * g) = o[1];  // dims 16 + 4g .. 16 + 4g+3
 }
 
 template <int SCH, int KS>
@@ -633,25 +598,12 @@ int run_attention(const ctmr_attn_desc* d, const float* q, const float* k, const
   }
 }
 
-// Split-fp16 workspace: six fp16 planes (Q hi/lo, K hi/lo, V^T hi/lo), each
-// starting on a 256-byte boundary.
-struct SplitPlan {
-  int64_t lkp, plane_bytes[3], offset[6], bytes;
-};
-
-SplitPlan split_plan(const ctmr_attn_desc* d) {
-  SplitPlan s{};
-  s.lkp = round_up(d->lk, kBlock);
+// What ctmr_flash_attention_f16x2_workspace_bytes answers, and the least a
+// caller's workspace must hold: six fp16 planes (Q, K and V, hi and lo), each in
+// whole 256 bytes.  Nothing is written to it.
+int64_t split_workspace_bytes(const ctmr_attn_desc* d) {
   const int64_t items = (int64_t)d->n * d->heads * kHeadDim * 2;
-  s.plane_bytes[0] = round_up(items * d->lq, 256);
-  s.plane_bytes[1] = s.plane_bytes[2] = round_up(items * s.lkp, 256);
-  int64_t at = 0;
-  for (int i = 0; i < 6; ++i) {
-    s.offset[i] = at;
-    at += s.plane_bytes[i / 2];
-  }
-  s.bytes = at;
-  return s;
+  return 2 * round_up(items * d->lq, 256) + 4 * round_up(items * round_up(d->lk, kBlock), 256);
 }
 
 }  // namespace
@@ -667,16 +619,17 @@ extern "C" int ctmr_flash_attention(const ctmr_attn_desc* d, const float* q, con
 extern "C" int64_t ctmr_flash_attention_f16x2_workspace_bytes(const ctmr_attn_desc* d) {
   using namespace ctmr;
   if (!d || d->n < 1 || d->lq < 1 || d->lk < 1 || d->heads < 1) return -1;
-  return split_plan(d).bytes;
+  return split_workspace_bytes(d);
 }
 
 extern "C" int ctmr_flash_attention_f16x2(const ctmr_attn_desc* d, const float* q, const float* k, const float* v,
                                           float* out, void* workspace, int64_t workspace_bytes, void* stream) {
   using namespace ctmr;
   if (const int rc = check_attn(d, q, k, v, out, "ctmr_flash_attention_f16x2")) return rc;
-  const SplitPlan plan = split_plan(d);
-  if (!workspace || workspace_bytes < plan.bytes) {
-    set_error("ctmr_flash_attention_f16x2: workspace of %lld bytes needed, %lld given", (long long)plan.bytes,
+  const int64_t need = split_workspace_bytes(d);
+  const bool none = !workspace && workspace_bytes == 0;
+  if (!none && (!workspace || workspace_bytes < need)) {
+    set_error("ctmr_flash_attention_f16x2: workspace of %lld bytes needed, %lld given", (long long)need,
               (long long)(workspace ? workspace_bytes : 0));
     return CTMR_E_INVALID;
   }

@@ -543,14 +543,11 @@ def flash_attention_f16x2(q: Tensor, k: Tensor, v: Tensor, heads: int, scale: fl
     out = torch.empty((n, lq, c), device=q.device, dtype=torch.float32)
     desc = _lib.AttnDesc(n, lq, lk, int(heads), c // int(heads), int(query_tiles),
                          q.stride(1), k.stride(1), v.stride(1), c, float(scale))
-    lib = _lib.lib()
-    nbytes = int(lib.ctmr_flash_attention_f16x2_workspace_bytes(ctypes.byref(desc)))
-    if nbytes < 0:
+    if min(n, lq, lk, int(heads)) < 1:
         raise ValueError(f"flash_attention_f16x2: invalid shape {(n, lq, lk, heads)}")
-    ws = torch.empty((nbytes,), device=q.device, dtype=torch.uint8)
     _lib.check(
-        lib.ctmr_flash_attention_f16x2(ctypes.byref(desc), q.data_ptr(), k.data_ptr(), v.data_ptr(),
-                                       out.data_ptr(), ws.data_ptr(), nbytes, _stream(q.device)),
+        _lib.lib().ctmr_flash_attention_f16x2(ctypes.byref(desc), q.data_ptr(), k.data_ptr(), v.data_ptr(),
+                                              out.data_ptr(), None, 0, _stream(q.device)),
         "ctmr_flash_attention_f16x2",
     )
     return out

@@ -7,7 +7,7 @@ the oracle's restatement of the reference's split arithmetic
 (``oracle.reference_math.flash_attention_split_f16``: the same fp16 halves and the same three
 products per multiply-add, summed in float64; bar 1e-6, which a dropped cross term or an
 unsplit operand misses by two orders of magnitude), and the float64 CPU oracle of the
-production attention blocks.  Different query tilings are bit-identical.
+production attention blocks.  ``query_tiles`` is a hint that changes no bit.
 """
 
 from __future__ import annotations
@@ -69,8 +69,8 @@ def test_split_attention_matches_float64_and_reference_arithmetic(ctmr, dev, see
 @pytest.mark.parametrize(("seed", "n", "lq", "lk", "heads", "q_gain"), _sweep_cases(24, 23),
                          ids=[f"sweep{i:02d}" for i in range(24)])
 def test_split_attention_random_shapes(ctmr, dev, seed, n, lq, lk, heads, q_gain):
-    """Seeded sweep around the block boundaries (full or ragged last key block, one or two key parts,
-    both query tilings, cross lengths, large score ranges)."""
+    """Seeded sweep around the block boundaries (full or ragged last key block, one or four key
+    parts, cross lengths, large score ranges)."""
     test_split_attention_matches_float64_and_reference_arithmetic(ctmr, dev, seed, n, lq, lk, heads, q_gain)
 
 
@@ -97,6 +97,16 @@ def test_split_attention_through_c_abi(ctmr, dev, native_loaded):
     assert native_loaded.ctmr_flash_attention_f16x2(*args, nbytes, stream) == 0
     torch.cuda.synchronize()
     assert torch.equal(out, expected)
+    out.zero_()  # no workspace at all: the kernel writes none
+    assert native_loaded.ctmr_flash_attention_f16x2(*args[:-1], None, 0, stream) == 0
+    assert torch.equal(out, expected)
+    torch.cuda.reset_peak_memory_stats(dev)
+    before = torch.cuda.memory_allocated(dev)
+    with ctmr.fast_fp32.precision("f16x2"):
+        again = ctmr.fast_fp32.flash_attention(q, k, v, heads=heads, scale=0.2)
+    # the output alone, in the allocator's 512-byte units
+    assert torch.cuda.max_memory_allocated(dev) - before <= (out.numel() * 4 + 511) // 512 * 512
+    assert torch.equal(again, expected)
     ref = _ref_attention(*(np.ascontiguousarray(t.cpu().numpy()) for t in (q, k, v)), heads, 0.2)
     assert rm.max_rel_error(out.cpu().numpy(), ref) <= FP32_REL
 

@@ -5,7 +5,7 @@ recorded MONAI attention block (tests/golden/maisi/attention.*) for the
 residual spatial-attention composition, and the float64 CPU oracle
 (oracle/maisi_torch.attention) at the production UNet's attention shapes.
 Bar: max relative error (max |a - b| / max |b|) within 1e-5, the FP32
-per-layer tolerance; different query tilings are bit-identical.
+per-layer tolerance; ``query_tiles`` is a hint that changes no bit.
 """
 
 from __future__ import annotations
@@ -75,8 +75,8 @@ def test_flash_attention_matches_float64(ctmr, dev, seed, n, lq, lk, heads, q_ga
 
 def _sweep_cases(count, seed):
     """Random shapes around the kernel's block boundaries: key counts that leave the last 32-key block
-    full or ragged, an odd or even number of blocks per key part, one or two key parts (at least 128
-    keys and a small grid), both query tilings, cross lengths and large score ranges."""
+    full or ragged, an odd or even number of blocks per key part, one or four key parts (at
+    least 128 keys), cross lengths and large score ranges."""
     rng = np.random.default_rng(seed)
     cases = []
     for i in range(count):
@@ -92,7 +92,7 @@ def _sweep_cases(count, seed):
 @pytest.mark.parametrize(("seed", "n", "lq", "lk", "heads", "q_gain"), _sweep_cases(40, 11),
                          ids=[f"sweep{i:02d}" for i in range(40)])
 def test_flash_attention_random_shapes(ctmr, dev, seed, n, lq, lk, heads, q_gain):
-    """Seeded sweep: every shape within the FP32 bar of float64 and both query tilings bit-identical."""
+    """Seeded sweep: every shape within the FP32 bar of float64, repeats bit-identical."""
     test_flash_attention_matches_float64(ctmr, dev, seed, n, lq, lk, heads, q_gain)
 
 
