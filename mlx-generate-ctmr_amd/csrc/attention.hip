@@ -119,9 +119,8 @@ __device__ __forceinline__ void block_softmax(f4 (&s)[kKeyTiles], float& m, floa
 //  * kFp32: q, k, v and P as three bf16 parts h, m, l that together hold an
 //    fp32 value's 24 bits (split_bf16x3), the six part products at or above
 //    2^-17 of the full one on bf16 MFMA (FP32 MFMA runs at a sixteenth of its
-//    rate).  Rows of the output that are not finite are computed again on FP32
-//    MFMA (attention_rerun): the parts of an infinity would meet as inf - inf or
-//    0 * inf.
+//    rate).  Rows with an output outside what the parts hold (part_sum_keep) are
+//    computed again on FP32 MFMA (attention_rerun).
 //  * kF16x2: the reference's split-fp16 arithmetic (_flash_attention.py:
 //    140-290, 314-317): hi = fp16(x), lo = fp16((x - hi) * 2^11) of q (after
 //    scale * log2(e)), k, v and P, with
@@ -168,7 +167,7 @@ __device__ __forceinline__ f4 mfma_x3(const u4 (&a)[3], const u4 (&b)[3], f4 c) 
 
 // A wave's 16 queries over all keys as fp32 products on FP32 MFMA
 // (v_mfma_f32_16x16x4_f32), keys and values straight from memory: for waves with
-// an output row that is not finite.  One NaN or infinity among the keys reaches
+// an output that the part products do not hold (part_sum_keep).  One NaN or infinity among the keys reaches
 // every query of its head, so the cost must stay a few times the finite one.
 // Two passes, the scores' maximum and then the probabilities, so that a score of
 // -inf is a key without weight wherever it stands.  S^T product j takes dims j
@@ -501,10 +500,10 @@ __global__ __launch_bounds__(kThreads, SCH == kFp32 && KS == 1 ? 6 : 4) void fla
     o[j] *= inv;
   }
   if constexpr (SCH == kFp32) {
-    float probe = 0.f;
+    PartSumTest test;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) probe = fmaf(o[e >> 2][e & 3], 0.f, probe);
-    const bool bad = !(probe == 0.f);
+    for (int e = 0; e < 8; ++e) test.add(o[e >> 2][e & 3]);
+    const bool bad = test.any();
     if (__any(bad && query < a.lq)) {
       f4 again[2];
       attention_rerun(a, Q + (int64_t)min(query, a.lq - 1) * a.ldq, K, V, rows_rsrc, col, g, again);

@@ -1248,17 +1248,27 @@ __global__ __launch_bounds__(256 * SETS, SETS == 2 ? 1 : X3 && NSUB == 2 && !DIR
         __builtin_amdgcn_sched_barrier(0);
       }
     }
-    // The wave's results that are not finite, again on FP32 MFMA (the reason and
-    // the bound on the cost as x3_rerun's in conv_lds.hip), a 16-column block at
-    // a time: product (q, j) takes channel 8g + 4q + j of each lane group g.
-    float probe = 0.f;
+    // The wave's results that the part products do not hold (part_sum_keep), on
+    // FP32 MFMA (the bound on the cost as x3_rerun's in conv_lds.hip), a
+    // 16-column block at a time: product (q, j) takes channel 8g + 4q + j of each
+    // lane group g.
+    PartSumProbe probe;
 #pragma unroll
     for (int ms = 0; ms < 4; ++ms)
 #pragma unroll
       for (int ns = 0; ns < NSUB; ++ns)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) probe = fmaf(acc[ms][ns][e], 0.f, probe);
-    if (__any(!(probe == 0.f))) {
+        for (int e = 0; e < 4; e += 2) probe.add(acc[ms][ns][e], acc[ms][ns][e + 1]);
+    PartSumTest test;
+    if (__any(probe.maybe())) {
+#pragma unroll
+      for (int ms = 0; ms < 4; ++ms)
+#pragma unroll
+        for (int ns = 0; ns < NSUB; ++ns)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) test.add(acc[ms][ns][e]);
+    }
+    if (__any(test.any())) {
 #pragma clang loop unroll(disable)
       for (int nb = 0; nb < NSUB; ++nb) {
         const int bo = min(n0 + nb * 16 + lrow, p.np - 1) * 64 + (lgrp >> 1) * p.np * 64 + (lgrp & 1) * 32;
@@ -1289,7 +1299,7 @@ __global__ __launch_bounds__(256 * SETS, SETS == 2 ? 1 : X3 && NSUB == 2 && !DIR
           for (int ms = 0; ms < 4; ++ms)
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-              if (ns == nb && !(fabsf(acc[ms][ns][e]) < INFINITY)) acc[ms][ns][e] = sum[ms][e];
+              if (ns == nb) acc[ms][ns][e] = part_sum_keep(acc[ms][ns][e], sum[ms][e]);
       }
     }
   } else {

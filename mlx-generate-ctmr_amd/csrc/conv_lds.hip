@@ -17,14 +17,14 @@ namespace ctmr {
 // Products.  FP32 MFMA runs at a sixteenth of the bf16 rate, so each fp32
 // operand v is staged as three bf16 parts h = bf16(v), m = bf16(v - h), l =
 // bf16(v - h - m), round to nearest: both differences are exact and h + m + l
-// holds all 24 significant bits at v's own exponent (no scaling, the full
-// fp32 range).  Of the nine part products the six at or above 2^-17 of the
-// full product run on v_mfma_f32_32x32x16_bf16 (hh, hm, mh, mm, hl, lh; each
-// exact in fp32), the dropped ml, lm, ll are below 2^-24 together, and fewer
-// fp32 roundings per sum (one per 16 channels and part product) leave the
-// results closer to 64 bits than FP32 MFMA's.  A result that is not finite
-// is summed again on FP32 MFMA (x3_rerun): with an infinity among the
-// operands the parts would meet as inf - inf or 0 * inf.
+// holds all 24 significant bits at v's own exponent, for v from 2^-110 (l's
+// last bit is then bf16's smallest, 2^-133) to bf16's largest.  Of the nine
+// part products the six at or above 2^-17 of the full product run on
+// v_mfma_f32_32x32x16_bf16 (hh, hm, mh, mm, hl, lh; each exact in fp32), the
+// dropped ml, lm, ll are below 2^-24 together, and fewer fp32 roundings per sum
+// (one per 16 channels and part product) leave the results closer to 64 bits
+// than FP32 MFMA's.  Results outside what the parts hold (part_sum_keep: not
+// finite, or below 2^-60) are summed again on FP32 MFMA (x3_rerun).
 //
 // Bound by the matrix pipe: 24 MFMAs of 32 cycles per wave, tap and chunk
 // against 12 ds_read_b128, 1 KiB each.  A and B both come from LDS: a staged
@@ -141,12 +141,11 @@ __device__ __forceinline__ void store_brick32(const Args& p, f16v (&acc)[2][NB],
   }
 }
 
-// The wave's results that are not finite, again as fp32 products over chunks
-// [c_begin, c_end): a result of the part products is finite exactly when all
-// operands are and no sum overflows, so only these can differ from the fp32
-// convolution's.  Reached by volumes that hold an infinity, a NaN or values
-// near the fp32 limit, and one of those can reach every output of the layers
-// after it (through a group norm), so the whole tile runs on FP32 MFMA
+// The wave's results that the part products do not hold (part_sum_keep), as
+// fp32 products over chunks [c_begin, c_end).  Reached by volumes that hold an
+// infinity, a NaN or values near either end of fp32's range, and one of those
+// can reach every output of the layers after it (through a group norm), so the
+// whole tile runs on FP32 MFMA
 // (v_mfma_f32_32x32x2_f32), operands straight from memory: the cost stays a
 // few times the finite one whatever the values.  Lane half h holds channels
 // 8h .. 8h + 7 of a chunk, product j the pair of channels j and 8 + j.
@@ -214,7 +213,7 @@ __device__ __forceinline__ void x3_rerun(const LdsArgs& p, f16v (&acc)[2][NB], f
     const f16v was = buf[i * 64 + lane];
 #pragma unroll
     for (int e = 0; e < 16; ++e)
-      if (fabsf(was[e]) < INFINITY) acc[i / NB][i % NB][e] = was[e];
+      acc[i / NB][i % NB][e] = part_sum_keep(was[e], acc[i / NB][i % NB][e]);
   }
 }
 
@@ -476,17 +475,25 @@ __global__ __launch_bounds__(256 * WS, WS == 1 ? 2 : 1) void conv_lds_kernel(Lds
     }(std::make_integer_sequence<int, 27>{});
   }
 
-  // Any result that is not finite sums to NaN or infinity here.
-  float probe = 0.f;
+  PartSumProbe probe;
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < NB; ++j)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) probe = fmaf(acc[i][j][e], 0.f, probe);
+      for (int e = 0; e < 16; e += 2) probe.add(acc[i][j][e], acc[i][j][e + 1]);
   lds_barrier();
   static_assert(4 * 64 * 256 <= kX3Set, "a set's results fit its staging buffers");
-  if (__any(!(probe == 0.f)))
+  PartSumTest test;
+  if (__any(probe.maybe())) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) test.add(acc[i][j][e]);
+  }
+  if (__any(test.any()))
     x3_rerun<XF>(p, acc, reinterpret_cast<f16v*>(lds) + wave * 128 * NB, b, z0 + wave, y0, x0, n0, lane, c_begin, c_end);
 
   // The statistics' reduction buffer and the hand-over below reuse the halos.

@@ -28,7 +28,7 @@ namespace ctmr {
 // depth tap: kd = 0, 1, 2 add to the sums of the next, this and the previous
 // output plane (stride 2: odd planes kd = 0 and 2, even planes kd = 1).
 // Six part products, summed smallest first in fp32 per (plane, column tap); a
-// result that is not finite is summed again on FP32 MFMA (march_rerun).
+// result that they do not hold is summed again on FP32 MFMA (march_rerun).
 //
 // Bound by HBM and the matrix pipe about equally: 8 -> 8 channels at 256 x 256 x
 // 128 moves 0.54 GB (115 us at a large copy's rate) against 112 us of MFMAs.
@@ -55,8 +55,8 @@ struct March {
 
 // The sums of a wave's four row blocks (layout of `acc`) as fp32 products on
 // FP32 MFMA (v_mfma_f32_16x16x4_f32), operands straight from memory: for a plane
-// with a result that is not finite (x3_rerun's reason and bound on the cost,
-// conv_lds.hip).  Lane group g holds line g of one output row's window (lane
+// with a result that the part products do not hold (part_sum_keep; the bound on
+// the cost as x3_rerun's, conv_lds.hip).  Lane group g holds line g of one output row's window (lane
 // group 3 zeros on both sides: a zero weight must not meet an infinity), product
 // j its channel j; stride 1 computes its two output rows one after the other.
 // oy: the output row of block 0; ox: this lane's output column; wbase: the first
@@ -271,15 +271,22 @@ __global__ __launch_bounds__(256, 2) void conv_march_kernel(MarchArgs p) {
     bias = f4{bq[0], bq[1], bq[2], bq[3]};
   }
   auto store = [&](f4 (&sum)[4], int oz) {
-    float probe = 0.f;  // not finite: a NaN or an infinity among the results to be stored
+    PartSumProbe probe;
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      const int oy = y0 + orow + (STRIDE == 1 ? 2 * t : t);
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (oy < p.oh && ox < p.ow && ocol < p.cout) probe = fmaf(sum[t][j], 0.f, probe);
+      probe.add(sum[t][0], sum[t][1]);
+      probe.add(sum[t][2], sum[t][3]);
     }
-    if (__any(!(probe == 0.f))) {
+    PartSumTest test;  // of the results to be stored
+    if (__any(probe.maybe())) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int oy = y0 + orow + (STRIDE == 1 ? 2 * t : t);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) test.add(oy < p.oh && ox < p.ow && ocol < p.cout ? sum[t][j] : 0.f);
+      }
+    }
+    if (__any(test.any())) {
       // The weights are loaded again afterwards, and the lane's indices are
       // opaque copies: neither then holds registers in the loop or in here.
       int ln = threadIdx.x & 63;
@@ -291,7 +298,7 @@ __global__ __launch_bounds__(256, 2) void conv_march_kernel(MarchArgs p) {
       for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          if (!(fabsf(sum[t][j]) < INFINITY)) sum[t][j] = again[t][j];
+          sum[t][j] = part_sum_keep(sum[t][j], again[t][j]);
       load_weights(ln, std::false_type{});
     }
 #pragma unroll

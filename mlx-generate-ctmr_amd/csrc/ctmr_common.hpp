@@ -92,6 +92,47 @@ __device__ __forceinline__ void split_bf16x3(f4 v, uint2& h, uint2& m, uint2& l)
   l = uint2{pl[0], pl[1]};
 }
 
+// Results of part products (split_bf16x3) that are computed again on FP32 MFMA.
+//  * Not finite: the parts of an infinity, of a NaN or of a value that rounds
+//    to infinity in bf16 meet as inf - inf or 0 * inf.  A result is finite
+//    exactly when all its operands are and no sum overflows.
+//  * Below 2^-60, not zero: bf16 parts reach down to 2^-133, so an operand
+//    below 2^-110 loses bits of its 24.  The error of a product is then at most
+//    2^-134 of the other operand: under 2^-24 of a result of 2^-60 and more that
+//    sums up to 2^16 products with operands up to 2^30.
+// part_sum_keep: the result `was`, or `now` for one of these (and for a zero: it
+// is no reason, but taken again where another result of the wave is one).  By a
+// bit mask: with a comparison each, the results of a tile hold enough scalar
+// registers to make the kernels around spill theirs.
+constexpr int kPartSumLeast = 0x21800000, kPartSumInfinity = 0x7f800000;  // 2^-60
+__device__ __forceinline__ float part_sum_keep(float was, float now) {
+  const int u = __float_as_int(was) & 0x7fffffff;
+  const int again = ((u - kPartSumLeast) | (kPartSumInfinity - 1 - u)) >> 31;
+  return __int_as_float((__float_as_int(was) & ~again) | (__float_as_int(now) & again));
+}
+
+// Whether a set holds a reason: PartSumProbe from a fused multiply-add and half a
+// minimum a value, true for a zero too; PartSumTest exactly.
+struct PartSumProbe {
+  float finite = 0.f, least = INFINITY;
+  __device__ __forceinline__ void add(float a, float b) {
+    finite = fmaf(b, 0.f, fmaf(a, 0.f, finite));
+    asm("v_min3_f32 %0, |%1|, |%2|, %0" : "+v"(least) : "v"(a), "v"(b));
+  }
+  __device__ __forceinline__ bool maybe() const { return !(finite == 0.f) || least < 0x1p-60f; }
+};
+struct PartSumTest {
+  unsigned most = 0u, least = ~0u;  // zero is the largest of the second kind
+  __device__ __forceinline__ void add(float v) {
+    const unsigned u = __float_as_uint(v) << 1;
+    most = max(most, u);
+    least = min(least, u - 1);
+  }
+  __device__ __forceinline__ bool any() const {
+    return most >= 2u * kPartSumInfinity || least < 2u * kPartSumLeast - 1;
+  }
+};
+
 // Workgroup barrier that orders LDS only: global loads stay in flight across it.
 __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");

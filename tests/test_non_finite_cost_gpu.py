@@ -59,8 +59,11 @@ def test_conv_of_nan(ctmr, dev, name, shape, cout, options, kernel):
     run = lambda v: f.implicit_gemm_conv3d(v, packed, None, cout=cout, **opts)
     nan = torch.full_like(x, float("nan"))
     finite, taken = _time(lambda: run(x)), _time(lambda: run(nan))
-    print(f"{name}: finite {finite * 1e3:.1f} us, NaN {taken * 1e3:.1f} us, {taken / finite:.1f}x", flush=True)
+    zero = _time(lambda: run(torch.zeros_like(x)))  # exact zeros are no reason to compute again
+    print(f"{name}: finite {finite * 1e3:.1f} us, NaN {taken * 1e3:.1f} us, {taken / finite:.1f}x, zeros "
+          f"{zero * 1e3:.1f} us", flush=True)
     assert bool(run(nan).isnan().all()) and bool(run(x).isfinite().all())
+    assert zero <= 1.6 * finite + 0.02  # the fill and the exact test
     assert taken <= 16 * finite
 
 
