@@ -126,13 +126,13 @@ __global__ __launch_bounds__(256, 2) void conv_march_kernel(MarchArgs p) {
   // `first` on: every load before the first split, one round of latency; a kd at
   // a time otherwise (the rerun's registers).
   u4 W[3][3][3];
-  auto load_weights = [&](int ln, auto first) {
+  auto load_weights = [&](int ln, auto first) __attribute__((always_inline)) {
     const int wrow = STRIDE == 1 ? (ln & 15) >> 3 : 0;
     const int wcol = STRIDE == 1 ? ln & 7 : (wave & 1) * 16 + (ln & 15);
     const int kh = (ln >> 4) - wrow;
     const bool w_on = kh >= 0 && kh < 3 && wcol < p.cout;
     f4 raw[3][3][2];
-    auto load_kd = [&](int kd) {
+    auto load_kd = [&](int kd) __attribute__((always_inline)) {
 #pragma unroll
       for (int kw = 0; kw < 3; ++kw) {
         const int tap = (kd * 3 + min(max(kh, 0), 2)) * 3 + kw;
@@ -278,7 +278,7 @@ __global__ __launch_bounds__(256, 2) void conv_march_kernel(MarchArgs p) {
       probe.add(sum[t][2], sum[t][3]);
     }
     PartSumTest test;  // of the results to be stored
-    if (__any(probe.maybe())) {
+    if (__builtin_expect(__any(probe.maybe()), 0)) {
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         const int oy = y0 + orow + (STRIDE == 1 ? 2 * t : t);
@@ -286,7 +286,7 @@ __global__ __launch_bounds__(256, 2) void conv_march_kernel(MarchArgs p) {
         for (int j = 0; j < 4; ++j) test.add(oy < p.oh && ox < p.ow && ocol < p.cout ? sum[t][j] : 0.f);
       }
     }
-    if (__any(test.any())) {
+    if (__builtin_expect(__any(test.any()), 0)) {
       // The weights are loaded again afterwards, and the lane's indices are
       // opaque copies: neither then holds registers in the loop or in here.
       int ln = threadIdx.x & 63;
