@@ -78,12 +78,18 @@ enum ctmr_conv_flags {
 };
 
 enum ctmr_dtype {
-  CTMR_F32 = 0,   /* fp32 operands, fp32 accumulate: the LDS-staged GEMM (CTMR_K_LDS) splits
-                     each operand into three bf16 parts that together hold its 24
-                     significant bits and sums the six part products at or above 2^-17 of
-                     the full one on bf16 MFMA (v_mfma_f32_32x32x16_bf16); results that
-                     are not finite are recomputed with plain fp32 products.  The other
-                     formulations run FP32 MFMA (v_mfma_f32_16x16x4_f32). */
+  CTMR_F32 = 0,   /* fp32 operands, fp32 accumulate.  The LDS-staged GEMM (CTMR_K_LDS), the
+                     plane-marching conv (CTMR_K_MARCH) and the streaming GEMM over taps
+                     (CTMR_K_STREAM, _STREAM_DIRECT and _SPLIT_WAVES, with an even number of
+                     16-channel blocks and more than 16 outputs) split each operand into
+                     three bf16 parts that together hold its 24 significant bits and sum the
+                     six part products at or above 2^-17 of the full one on bf16 MFMA.
+                     Results that are not finite, or not zero and below 2^-60, are computed
+                     again on FP32 MFMA: operands below 2^-110 keep fewer bits in bf16 parts
+                     (below 2^-134 none: products of such alone are zero), which only shows
+                     in a larger result where the other operand exceeds 2^30.  The other formulations (one-tap GEMMs, im2col rows, tap
+                     expansion, an odd block count) run FP32 MFMA throughout, and
+                     CTMR_K_SMALL_COUT fp32 FMAs. */
   CTMR_BF16 = 1,  /* bf16 operands, fp32 accumulate (v_mfma_f32_16x16x32_bf16);
                      activations and outputs stay fp32 in memory */
   CTMR_F16X2 = 2  /* split fp16, the reference's "exact" mode for fp32 tensors
@@ -395,9 +401,10 @@ int ctmr_resample(int32_t op, int32_t n, int32_t d, int32_t h, int32_t w, int32_
  * throughout, and results do not depend on it.  Keys are visited in a fixed
  * order: ascending 32-key blocks, or -- for small grids, decided from n, lq, lk
  * and heads only -- two or four such runs over equal key parts, combined in
- * ascending order.  The fp32 operands are multiplied as three bf16 parts that together
- * hold their 24 significant bits (as CTMR_K_LDS convolutions); output rows that
- * are not finite are recomputed with plain fp32 products. */
+ * ascending order.  The fp32 operands are multiplied as three bf16 parts that
+ * together hold their 24 significant bits; rows with an output that is not
+ * finite, or not zero and below 2^-60, are computed again on FP32 MFMA (see
+ * CTMR_F32). */
 typedef struct ctmr_attn_desc {
   int32_t n, lq, lk, heads, head_dim, query_tiles;
   int64_t ldq, ldk, ldv, ldo;

@@ -17,8 +17,9 @@
 //   * the S^T registers, split, are already P^T's B operand for the next product
 //     (k slot 8g + 4u + r is key 16u + 4g + r), and
 //   * the running-output rescale is one scalar per lane.
-// Everything accumulates in FP32; keys are visited in ascending blocks, so the
-// result does not depend on the launch shape or on other work on the device.
+// Everything accumulates in FP32; keys are visited in ascending blocks within one,
+// two or four parts chosen from the shape, so a shape's results are always the
+// same bits, whatever else runs on the device.
 #include "ctmr_common.hpp"
 
 #include <algorithm>
@@ -247,9 +248,11 @@ __device__ __forceinline__ void attention_rerun(const AttnArgs& a, const float* 
 // queries a wave 1.6 times 32 queries a wave at any occupancy.  Measured, that
 // form (its separate split pass included) / this one us: 2048 tokens x 8 heads
 // x 2 fp32 87 / 70, split fp16 86 / 53; 4158 x 8 244 / 173, 237 / 143; 4800 x
-// 16 553 / 334, 500 / 263.  Now bound by LDS reads (8 or 12 of 1 KiB a wave and
-// block: 58 % of the cycles) and VALU (168 operations: 57 %) together; 32
-// queries a wave halve the reads but leave half the waves: 67, 70; 193, 177 us.
+// 16 553 / 334, 500 / 263.  Now bound by a step's chain (barrier, LDS reads,
+// S^T, softmax, split, P V), which four waves a SIMD cover in part: VALU issues
+// in 54 % of the cycles (168 operations a wave and block), the MFMAs take 30 %
+// (fp32) or 19 %, LDS bank conflicts 16 %.  32 queries a wave halve the LDS
+// reads but leave half the waves: 67, 70; 193, 177 us.
 // A small grid is bound by the latency of its steps: 1024 tokens x 8 heads 16.2
 // / 15.2, 33.4 / 13.8; 256 x 16 x 2 7.2 / 7.8, 13.4 / 6.8 (with two parts and
 // one block in flight 21.6, 18.8; 8.8, 7.6).

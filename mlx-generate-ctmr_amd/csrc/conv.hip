@@ -1017,8 +1017,10 @@ __device__ __forceinline__ void store_tile(const ConvArgs& p, f4 (&acc)[4][NSUB]
 // next step as soon as it is split, so one set of raw registers suffices.
 // Bound by those VALU operations as much as by the MFMAs.  Measured, FP32 MFMA
 // / part products us: 16x16x8 x 2, 256 channels (split waves) 120 / 98, 8x8x4
-// x 2, 512 channels 70 / 62, 25^3, 256 channels 549 / 336, 49x49x33, 256
-// channels 2431 / 1627; UNet pass 12.29 -> 11.82 ms.
+// x 2, 512 channels 60 / 49, 25^3, 256 channels 549 / 336, 49x49x33, 256
+// channels 2431 / 1627; UNet pass 12.29 -> 11.82 ms.  Small grids too, so the
+// rule has no size: 4x4x4, 512 channels 16.0 / 15.0, 8x8x8, 128 channels 16.5 /
+// 15.6.
 template <int DT, int NSUB, int WM, int WN, int KT, int STRIDE, bool UP, bool DIRECT = false, int KWS = 1,
           int SETS = 1, bool X3 = false>
 __global__ __launch_bounds__(256 * SETS, SETS == 2 ? 1 : X3 && NSUB == 2 && !DIRECT ? 3 : 2) void conv_kernel(ConvArgs p) {
@@ -1385,7 +1387,8 @@ __global__ __launch_bounds__(256 * SETS, SETS == 2 ? 1 : X3 && NSUB == 2 && !DIR
 // ---------------------------------------------------------------------------
 // 3b. Brick GEMMs (the fp32 LDS-staged one is conv_lds_kernel, conv_lds.hip)
 // ---------------------------------------------------------------------------
-// Epilogue of the brick GEMMs (conv_lds_kernel, conv_lds_bf16_kernel) from
+// Epilogue of the brick GEMMs here (conv_lds_bf16_kernel, conv_lds_small_kernel;
+// conv_lds_kernel's is store_brick32) from
 // transposed accumulators: lane l of block (ms, ns) holds voxel (z0 + wave,
 // y0 + ms + 4*((l/8)%2), x0 + l%8) of the 4x8x8 brick and output columns
 // n0 + ns*16 + 4*(l/16) .. +3 (cout % 64 == 0), stored -- bias first, then the

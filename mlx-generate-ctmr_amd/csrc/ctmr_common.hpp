@@ -97,7 +97,8 @@ __device__ __forceinline__ void split_bf16x3(f4 v, uint2& h, uint2& m, uint2& l)
 //    to infinity in bf16 meet as inf - inf or 0 * inf.  A result is finite
 //    exactly when all its operands are and no sum overflows.
 //  * Below 2^-60, not zero: bf16 parts reach down to 2^-133, so an operand
-//    below 2^-110 loses bits of its 24.  The error of a product is then at most
+//    below 2^-110 loses bits of its 24 (below 2^-134 all: exact zeros stay, as
+//    the zeros of an empty volume must cost nothing).  The error of a product is then at most
 //    2^-134 of the other operand: under 2^-24 of a result of 2^-60 and more that
 //    sums up to 2^16 products with operands up to 2^30.
 // part_sum_keep: the result `was`, or `now` for one of these (and for a zero: it
