@@ -338,15 +338,11 @@ __global__ __launch_bounds__(kThreads, SCH == kFp32 && KS == 1 ? 6 : 4) void fla
     }
   };
 
-  // The first blocks and Q: of a small grid in one round of latency; a full one
-  // hides it, and does without the second block's registers until the first is
-  // published (4096 tokens x 8 heads x 2, fp32: 225 us, 229 in one round).
+  // The first blocks and Q in one round of latency.
   f4 raw0[KS], raw[kAhead][KS];
   fetch(k_begin, raw0);
-  if constexpr (KS > 1) {
 #pragma unroll
-    for (int i = 0; i < kAhead; ++i) fetch(k_begin + (1 + i) * kBlock, raw[i]);
-  }
+  for (int i = 0; i < kAhead; ++i) fetch(k_begin + (1 + i) * kBlock, raw[i]);
 
   // Q^T as the B operand of S^T = K Q^T: query q0 + col, dims 8g .. 8g+7.
   u4 qf[SCH];
@@ -440,7 +436,6 @@ __global__ __launch_bounds__(kThreads, SCH == kFp32 && KS == 1 ? 6 : 4) void fla
   };
 
   publish(lds[0][part], raw0);
-  if constexpr (KS == 1) fetch(k_begin + kBlock, raw[0]);
   auto step = [&](int i, f4 (&ahead)[KS]) {
     // Block i is published, and every wave is done with block i - 1, whose
     // buffer takes block i + 1 (past the part's keys: other keys or zeros,
