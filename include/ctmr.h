@@ -87,9 +87,9 @@ enum ctmr_dtype {
                      Results that are not finite, or not zero and below 2^-60, are computed
                      again on FP32 MFMA: operands below 2^-110 keep fewer bits in bf16 parts
                      (below 2^-134 none: products of such alone are zero), which only shows
-                     in a larger result where the other operand exceeds 2^30.  The other formulations (one-tap GEMMs, im2col rows, tap
-                     expansion, an odd block count) run FP32 MFMA throughout, and
-                     CTMR_K_SMALL_COUT fp32 FMAs. */
+                     in a larger result where the other operand exceeds 2^30.  The other
+                     formulations (one-tap GEMMs, im2col rows, tap expansion, an odd block
+                     count) run FP32 MFMA throughout, and CTMR_K_SMALL_COUT fp32 FMAs. */
   CTMR_BF16 = 1,  /* bf16 operands, fp32 accumulate (v_mfma_f32_16x16x32_bf16);
                      activations and outputs stay fp32 in memory */
   CTMR_F16X2 = 2  /* split fp16, the reference's "exact" mode for fp32 tensors

@@ -1023,7 +1023,8 @@ __device__ __forceinline__ void store_tile(const ConvArgs& p, f4 (&acc)[4][NSUB]
 // 15.6.
 template <int DT, int NSUB, int WM, int WN, int KT, int STRIDE, bool UP, bool DIRECT = false, int KWS = 1,
           int SETS = 1, bool X3 = false>
-__global__ __launch_bounds__(256 * SETS, SETS == 2 ? 1 : X3 && NSUB == 2 && !DIRECT ? 3 : 2) void conv_kernel(ConvArgs p) {
+__global__ __launch_bounds__(256 * SETS, SETS == 2 ? 1 : X3 && NSUB == 2 && !DIRECT ? 3 : 2)  // waves per SIMD
+void conv_kernel(ConvArgs p) {
   static_assert(WM * WN * KWS == 4, "four waves per wave set");
   static_assert(SETS == 1 || (SETS == 2 && KWS == 4), "two wave sets only with the four-wave K split");
   static_assert(!DIRECT || (KT == 3 && !UP && DT == CTMR_F32), "direct reads: plain fp32 3x3x3 convs");

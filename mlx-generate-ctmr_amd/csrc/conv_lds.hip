@@ -494,7 +494,8 @@ __global__ __launch_bounds__(256 * WS, WS == 1 ? 2 : 1) void conv_lds_kernel(Lds
         for (int e = 0; e < 16; ++e) test.add(acc[i][j][e]);
   }
   if (__any(test.any()))
-    x3_rerun<XF>(p, acc, reinterpret_cast<f16v*>(lds) + wave * 128 * NB, b, z0 + wave, y0, x0, n0, lane, c_begin, c_end);
+    x3_rerun<XF>(p, acc, reinterpret_cast<f16v*>(lds) + wave * 128 * NB, b, z0 + wave, y0, x0, n0, lane, c_begin,
+                 c_end);
 
   // The statistics' reduction buffer and the hand-over below reuse the halos.
   double (*const red)[64][2] = reinterpret_cast<double (*)[64][2]>(lds_sets);

@@ -56,11 +56,11 @@ struct March {
 // The sums of a wave's four row blocks (layout of `acc`) as fp32 products on
 // FP32 MFMA (v_mfma_f32_16x16x4_f32), operands straight from memory: for a plane
 // with a result that the part products do not hold (part_sum_keep; the bound on
-// the cost as x3_rerun's, conv_lds.hip).  Lane group g holds line g of one output row's window (lane
-// group 3 zeros on both sides: a zero weight must not meet an infinity), product
-// j its channel j; stride 1 computes its two output rows one after the other.
-// oy: the output row of block 0; ox: this lane's output column; wbase: the first
-// of the wave's output channels.
+// the cost as x3_rerun's, conv_lds.hip).  Lane group g holds line g of one output
+// row's window (lane group 3 zeros on both sides: a zero weight must not meet an
+// infinity), product j its channel j; stride 1 computes its two output rows one
+// after the other.  oy: the output row of block 0; ox: this lane's output column;
+// wbase: the first of the wave's output channels.
 template <int STRIDE>
 __device__ __forceinline__ void march_rerun(const MarchArgs& p, f4 (&sum)[4], int b, int oz, int oy, int ox, int wbase,
                                             int lrow, int lgrp) {

@@ -497,8 +497,10 @@ __global__ __launch_bounds__(256) void resample_kernel(int op, int n, int d, int
 constexpr int kPlanarThreads = 1024;
 constexpr int kPlanarVecs = 8;                                     // vectors a thread of the one-launch form holds
 constexpr int kPlanarRun = kPlanarThreads * kPlanarVecs;           // x VEC values: the one-launch form's longest run
-constexpr int kPlanarChunk = 256 * 16;                             // a chunk of the two-launch form: this many vectors, or a
-constexpr int kPlanarChunks = 2048;                                // multiple of them that leaves at most so many chunks
+// A chunk of the two-launch form: kPlanarChunk vectors, or the multiple of them
+// that leaves at most kPlanarChunks chunks.
+constexpr int kPlanarChunk = 256 * 16;
+constexpr int kPlanarChunks = 2048;
 constexpr int kPlanarMaxCpg = 1024;
 
 struct PlanarArgs {
